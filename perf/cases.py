@@ -113,6 +113,7 @@ class _State:
         self.eng = dnnl.engine(dnnl.engine.kind.gpu, 0)
         self.stream = dnnl.stream(self.eng, hip_stream=torch.cuda.current_stream().cuda_stream)
         self.args, self.keep, self.out = {}, [], None
+        self.plain = None  # exact() sets a dict here, which then gets every operand as it was before any prepacking
 
     def normal(self, shape, std=1.0):
         return torch.randn(shape, generator=self.gen, device="cuda") * std
@@ -133,6 +134,8 @@ class _State:
         return memory(md, self.eng, tensor.data_ptr())
 
     def bind(self, arg, md, tensor):
+        if self.plain is not None:
+            self.plain.setdefault(arg, tensor)
         self.args[arg] = self.memory(md, tensor)
 
     def vector(self, arg, code, tensor):
@@ -140,6 +143,8 @@ class _State:
 
     def packed(self, pd, plain_md, tensor):
         """Weights in the layout the primitive asked for, written by the reorder primitive."""
+        if self.plain is not None:
+            self.plain[dnnl.DNNL_ARG_WEIGHTS] = tensor
         md = pd.weights_desc()
         self.bind(dnnl.DNNL_ARG_WEIGHTS, md, torch.empty(md.get_size(), dtype=torch.uint8, device="cuda"))
         plain = memory(plain_md, self.eng, tensor.data_ptr())
@@ -274,10 +279,13 @@ def _sdpa(s, c):
     s.primitive = dnnl.sdpa(pd)
 
 
-def prepare(case, seed):
-    s = _State(seed)
+def _fill(s, case):
     {"scores": _scores, "sdpa": _sdpa}.get(case["kind"], _linear)(s, case)
     return s
+
+
+def prepare(case, seed):
+    return _fill(_State(seed), case)
 
 
 def run(state):
@@ -318,3 +326,62 @@ def tolerance(case):
         # (few rows of 8-bit weights: the offset of the byte -> float trick leaves through the sum of the activations)
         return {"rel": 1e-6, "max": 1e-5} if kind == "w8a8" else {"rel": 1e-4, "max": 6e-4}
     return {"rel": 6e-3, "max": 0.02} if dst == "bf16" else {"rel": 1e-3, "max": 3e-3}
+
+
+def _nibbles(x, n, signed=False):
+    """[rows, n] doubles out of bytes that hold two values each, the first in the low half."""
+    v = torch.stack((x & 15, x >> 4), -1).reshape(-1, n).double()
+    return torch.where(v > 7, v - 16, v) if signed else v
+
+
+def exact(case, seed):
+    """The outputs of run() for these inputs in float64, from the plain operands."""
+    s = _State(seed)
+    s.plain = {}
+    _fill(s, case)
+    c, kind, x = case, case["kind"], s.plain
+    if kind == "scores":
+        q, k = x[dnnl.DNNL_ARG_SRC].double(), x[dnnl.DNNL_ARG_WEIGHTS].double()
+        scale = x[SCALE_SRC].double() * x[SCALE_WEI].double()
+        mask = x[dnnl.DNNL_ARG_ATTR_MULTIPLE_POST_OP(0) | dnnl.DNNL_ARG_SRC_1].double()
+        return torch.stack([q[b] @ k[b] * scale + mask for b in range(c["heads"])])
+    if kind == "sdpa":
+        q, scale = x[dnnl.DNNL_ARG_QUERIES].double(), x[dnnl.DNNL_ARG_SCALE].double()
+        kv = []
+        for arg in (dnnl.DNNL_ARG_KEYS, dnnl.DNNL_ARG_VALUES):
+            t = x[arg].double()
+            if c["cache"] == "s8":
+                t = (t - x[dnnl.DNNL_ARG_ATTR_ZERO_POINTS | arg].double()[:, :, None]) * x[dnnl.DNNL_ARG_ATTR_SCALES | arg].double()[:, :, None]
+            kv.append(t)
+        hidden = torch.ones((c["queries"], c["keys"]), dtype=torch.bool, device="cuda").triu(1) if c["causal"] else None
+        out = []
+        for h in range(c["heads"]):
+            g = h // (c["heads"] // c["kv_heads"])
+            w = q[h] @ kv[0][g].t().contiguous() * scale
+            if hidden is not None:
+                w.masked_fill_(hidden, -math.inf)
+            out.append(torch.softmax(w, -1) @ kv[1][g])
+        return torch.stack(out)[None]
+    k, n = c["k"], c["n"]
+    src, wei = x[dnnl.DNNL_ARG_SRC].double(), x[dnnl.DNNL_ARG_WEIGHTS]
+    if kind == "w8a8":
+        if c["src"] == "u8":
+            src = (src - x[ZERO_SRC].double()) * x[SCALE_SRC].double()
+        else:
+            src = src * x[SCALE_SRC].double()[:, None]
+        wei = wei.double() * x[SCALE_WEI].double()
+    elif kind == "fp8":
+        wei = wei.double() * (x[SCALE_SRC].double() * x[SCALE_WEI].double())
+    elif kind == "w8":
+        wei = (wei.double() - x[ZERO_WEI].double()) * x[SCALE_WEI].double()
+    else:
+        wei = _nibbles(wei, n, signed=kind == "w4a8").view(-1, GROUP, n)
+        if kind == "w4":
+            wei = wei - _nibbles(x[ZERO_WEI], n)[:, None]
+        else:
+            src = (src.view(-1, k // GROUP, GROUP) * x[SCALE_SRC].double()[:, :, None]).view(-1, k)
+        wei = (wei * x[SCALE_WEI].double()[:, None]).view(k, n)
+    r = src @ wei
+    if kind == "fp8":
+        r += x[dnnl.DNNL_ARG_DST].double()  # this run() has not been called: still the residual
+    return r * torch.sigmoid(r) if c.get("swish") else r
