@@ -23,6 +23,8 @@
 //     staged once per block in LDS in MFMA operand order.
 #include <type_traits>
 
+#include <cstring>
+
 #include "qmm_device.hpp"
 #include "qmm_plan.hpp"
 
@@ -872,6 +874,9 @@ gemv_w4_fast_cb_kernel(const uint8_t *__restrict__ pB,
 void launch_gemm_w4f(const gemv_params_t &p, int shifts, int flags_m,
         hipStream_t stream);
 bool gemm_w4f_wins(const gemv_params_t &p);
+void launch_gemm_g128_f16(const g128_params_t &p, int rows, hipStream_t stream);
+void launch_gemm_g128_bf16(const g128_params_t &p, int rows, hipStream_t stream);
+int gemm_g128_rows(int M, int N, bool s8);
 
 // Returns false when no kernel takes the problem (nothing is launched then).
 bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
@@ -934,6 +939,36 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
         // an absent zero-point buffer is never dereferenced past its first
         // byte: the weights stand in for it
         const uint8_t *zp = p.zps ? (const uint8_t *)p.zps : p.B;
+        // 4-bit weights at many rows: the kernel whose wave tile is up to 96 rows
+        // tall (direct 16-byte loads: rows on 16-byte boundaries, whole groups of
+        // 128 k, 32-bit offsets inside a tile of rows)
+        const int g128_rows = gemm_g128_rows(p.M, p.N, false);
+        if (g128_rows && !p.w8 && p.K == Kpad && p.lda % 8 == 0 && p.lda < (1 << 23)
+                && ((uintptr_t)p.A & 15) == 0) {
+            g128_params_t t;
+            std::memset(&t, 0, sizeof(t));
+            t.A = (const uint8_t *)p.A;
+            t.lda = p.lda * 2;
+            t.B = p.B;
+            t.scales = p.scales;
+            t.sw_f16 = p.scale_dt == dt_f16;
+            t.gs_shift = q.gs_shift;
+            t.gz_shift = q.gz_shift;
+            t.scale_per_n = p.scale_per_n;
+            t.zp_per_n = p.zp_per_n;
+            t.zps = p.zps;
+            t.zp4 = p.zp_dt == dt_s4 || p.zp_dt == dt_u4;
+            t.zp_signed = p.zp_dt == dt_s4 || p.zp_dt == dt_s8;
+            t.wei_signed = p.wei_signed;
+            t.M = p.M;
+            t.N = p.N;
+            t.ng = p.kg128;
+            t.nb = p.nb16;
+            t.ep = p.ep;
+            if (p.act_f16) launch_gemm_g128_f16(t, g128_rows, stream);
+            else launch_gemm_g128_bf16(t, g128_rows, stream);
+            return true;
+        }
         // More than 16 rows: the tiled kernel (a weights tile unpacked once
         // for 32 or 64 rows) where it beats this one once per block of 16 rows.
         if (gemm_w4f_wins(p)) {

@@ -266,6 +266,27 @@ struct w4a8_prep_t {
     int32_t *zsT, *c2T; // nullptr unless the source has zero points or is u8
 };
 
+// ---- 4-bit weights with groups of 128 k, many rows (qmm_gemm_g128.hip) --------
+struct g128_params_t {
+    const uint8_t *A; // s8, f16 or bf16 rows, K-contiguous
+    int64_t lda; // bytes
+    const uint8_t *B; // QMM_LAYOUT_MFMA_W4K64 (s8) or QMM_LAYOUT_MFMA_W4
+    const void *ss; // s8: f16 / bf16 source scales, strides over (row, group)
+    int64_t ss_sm, ss_sk;
+    const void *scales; // f16 / bf16 weights scales
+    int64_t sw_sk, sw_sn; // s8: strides over (group, column)
+    // f16 / bf16 activations: rows of N (scale_per_n) or single values, one per
+    // 128 << shift k (-1: one for all of K); zero points likewise
+    int32_t gs_shift, gz_shift, scale_per_n, zp_per_n;
+    const void *zps; // nullptr: none
+    int32_t zp4, zp_signed, wei_signed;
+    int32_t ss_f16, sw_f16; // f16 (else bf16) scales
+    int32_t M, N, ng; // ng groups of 128 k
+    int32_t nb; // column blocks of the packed weights (16 columns; s8: 32)
+    int32_t tiles_m, tiles_n; // set by the launcher
+    epilogue_t ep;
+};
+
 // Rows <= 64 (decode): the K range is cut into `splits` slices of `gps` groups,
 // one workgroup per (64 columns, slice); slice results are summed in slice
 // order by w4a8_reduce_kernel, which also runs the epilogue. No pre-pass: the

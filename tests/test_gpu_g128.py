@@ -1,0 +1,99 @@
+"""GPU parity of the tiled kernel for 4-bit weights with groups of 128 k at many rows (qmm_gemm_g128.hip): s8
+activations (hip:gfx950:mfma_w4a8) and f16 / bf16 activations (hip:gfx950:decode_w4), at the edges of its tiles.
+
+Sizes are chosen by its rule (gemm_g128_rows): more than 192 (s8) or 256 blocks of 64 rows x 256 columns, and the
+taller tile where that needs fewer rounds. Bars as in the tests of the kernels beside it: bit for bit where every
+order of operations gives the same bits, else a share of the summed magnitudes (f32 sums of a few hundred terms).
+"""
+import numpy as np
+import pytest
+
+import onednn_amd as dnnl
+import oracle as O
+import test_gpu_parity as parity
+from qmm_harness import assert_bf16_within_1ulp, assert_bit_exact, assert_f32_close, dt
+from test_gpu_w4a8 import W4A8, dynamic_quant
+
+pytestmark = pytest.mark.gpu
+A = dnnl.algorithm
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    eng = dnnl.engine(dnnl.engine.kind.gpu, 0)
+    return eng, dnnl.stream(eng)
+
+
+S8_CASES = {
+    # 64-row tiles: row and column tails, one group, an odd number of groups
+    "rows64_one_group_tails": dict(M=129, K=128, N=16650),
+    "rows64_three_groups_bf16_scales": dict(M=193, K=384, N=16642, scale_dt=dt.bf16),
+    # 128-row tiles
+    "rows128_tails": dict(M=700, K=256, N=14330),
+    "rows128_whole_tiles": dict(M=640, K=512, N=14336, dst_dt=dt.f16),
+}
+
+
+@pytest.mark.parametrize("name", sorted(S8_CASES))
+def test_s8_exact(ctx, name):
+    eng, strm = ctx
+    print("[case] g128 s8 %s" % name, flush=True)
+    p = dynamic_quant(seed=500 + len(name), exact=True, **S8_CASES[name])
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == W4A8
+    assert_bit_exact(got, p.run_oracle(), name)
+
+
+def test_s8_extreme_sums(ctx):
+    """The largest sums a group can reach, both signs: 128 * (-128) * (-8) and 128 * (-128) * 7, times 16."""
+    eng, strm = ctx
+    print("[case] g128 s8 extremes", flush=True)
+    p = dynamic_quant(129, 256, 16640, 7, exact=True)
+    p.src.set(np.full((129, 256), -128.0))
+    p.wei.set(np.where(np.arange(16640) % 2 == 0, -8.0, 7.0)[None].repeat(256, 0))
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == W4A8
+    assert_bit_exact(got, p.run_oracle(), "extremes")
+
+
+def test_s8_arbitrary_scales_and_post_ops(ctx):
+    eng, strm = ctx
+    print("[case] g128 s8 arbitrary scales", flush=True)
+    p = dynamic_quant(257, 256, 14350, 19, dst_dt=dt.f32,
+                      post_ops=[{"kind": "eltwise", "alg": A.eltwise_relu, "alpha": 0.5}])
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == W4A8
+    assert_f32_close(got, p.run_oracle(), rel=1e-5, scale=p.term_scale, what="f32")
+
+
+W4_CASES = {
+    # 64-row tiles
+    "f16_u4_rows64_tails": dict(M=100, K=128, N=32900, act_dt=dt.f16, zp_dt=dt.u4),
+    "bf16_s4_zp_s8_rows64": dict(M=100, K=384, N=32770, wei_dt=dt.s4, zp_dt=dt.s8, scale_dt=dt.bf16),
+    "f16_u4_zp_u8_groups256_f32_dst": dict(M=97, K=512, N=32766, act_dt=dt.f16, zp_dt=dt.u8, G=256, zp_group=128,
+                                           dst_dt=dt.f32),
+    # 96-row tiles
+    "f16_s4_no_zp_rows96_tails": dict(M=190, K=256, N=32700, act_dt=dt.f16, wei_dt=dt.s4, with_zp=False),
+    "bf16_u4_rows96_relu": dict(M=129, K=256, N=22200, post_ops=[{"kind": "eltwise", "alg": A.eltwise_relu, "alpha": 0.0}]),
+    "f16_u4_per_column_rows96": dict(M=65, K=256, N=33000, act_dt=dt.f16, zp_dt=dt.u4, per_column=True),
+}
+
+
+@pytest.mark.parametrize("name", sorted(W4_CASES))
+def test_16bit_activations(ctx, name):
+    eng, strm = ctx
+    print("[case] g128 %s" % name, flush=True)
+    kw = W4_CASES[name]
+    p = parity.decode_w4(seed=600 + len(name), **kw)
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == parity.DECODE
+    want = p.run_oracle()
+    code, M, N = p.dst.dt, kw["M"], kw["N"]
+    terms = parity.decode_term_scale(p).reshape(M, N)
+    if code == dt.bf16:
+        assert_bf16_within_1ulp(got, want, name, abs_slack=2e-5 * terms.reshape(-1))
+        return
+    g, w = O.to_f32(code, got).reshape(M, N), O.to_f32(code, want).reshape(M, N)
+    # f32 sums in another order: 2e-5 of the summed magnitudes; an f16 result one step (2^-10) more
+    bar = 2e-5 * terms + (np.abs(w) * 2.0 ** -10 if code == dt.f16 else 0)
+    assert np.all(np.abs(g.astype(np.float64) - w) <= bar), name
