@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "qmm_device.hpp"
 #include "qmm_hip.h"
@@ -94,7 +95,8 @@ struct sdpa_params_t {
     // few queries (decode): the keys are cut into nsplit ranges of tps tiles
     int32_t nsplit, tps;
     int32_t fastq, bf; // f16 scales and 8-bit zero points: f16 dequantisation
-    float *part; // [head][split][16 queries][D + 2]: O (unnormalised), m, l
+    int32_t pack; // few queries: heads of one K / V head that share a workgroup
+    float *part; // [head][split][query][D + 2]: O (unnormalised), m, l
 };
 
 // Lanes that differ only in their 16-lane row hold parts of one query. The two
@@ -143,11 +145,13 @@ QMM_D float ld_zp(int dt, const void *p, int64_t i) {
 // significant bits, so rounding the f16 product is the same single rounding as
 // f16(f32 product): the values of the reference's dequantizing reorder, at 1.5
 // instructions per element. `raw`: bytes with the sign bit already flipped for
-// s8; zb: zero point (+ 128 for s8), within [0, 1023].
+// s8; sc: the scale twice; off: 1024 + zero point (+ 128 for s8), an integer within
+// [1024, 2047], twice.
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-QMM_D uint4 dequant8_f16(uint32_t w0, uint32_t w1, float s1, float zb) {
-    const h2 off = h2 {(_Float16)(1024.f + zb), (_Float16)(1024.f + zb)};
-    const h2 sc = h2 {(_Float16)s1, (_Float16)s1};
+QMM_D h2 twice(float v) {
+    return h2 {(_Float16)v, (_Float16)v};
+}
+QMM_D uint4 dequant8_f16(uint32_t w0, uint32_t w1, const h2 &sc, const h2 &off) {
     const uint32_t w[2] = {w0, w1};
     uint32_t o[4];
 #pragma unroll
@@ -296,8 +300,8 @@ sdpa_f16_kernel(const sdpa_params_t p) {
                 const uint32_t kw[2] = {pk[n].x ^ flip, pk[n].y ^ flip};
                 const uint32_t vw[2] = {pv[n].x ^ flip, pv[n].y ^ flip};
                 if (p.fastq) {
-                    kv = dequant8_f16(kw[0], kw[1], pks[n], kzb);
-                    vv = dequant8_f16(vw[0], vw[1], pvs[n], vzb);
+                    kv = dequant8_f16(kw[0], kw[1], twice(pks[n]), twice(1024.f + kzb));
+                    vv = dequant8_f16(vw[0], vw[1], twice(pvs[n]), twice(1024.f + vzb));
                 } else {
                 uint32_t kh[8], vh[8];
 #pragma unroll
@@ -504,48 +508,143 @@ sdpa_f16_kernel(const sdpa_params_t p) {
 
 
 // ---- few queries (at most 16 per head: the decode step) ----------------------
-// One workgroup per (head, key range); its four waves take the range's key
-// tiles in turn, each with its own running maximum, sum and accumulators and
-// its own piece of LDS (the V tile it transposes): no barrier until the end,
-// where wave 0 merges the four states. A launch is then heads x splits
-// workgroups streaming K and V once, instead of one workgroup per head walking
-// all keys. With more than one split the merged state goes to the scratchpad
-// (unnormalised accumulators, maximum, sum per query) and sdpa_combine_kernel
-// finishes.
-template <int DC, bool QUANT, bool MASKED, bool BF>
-__global__ void __launch_bounds__(SDPA_WAVES * 64)
+// Bound: HBM, one read of the cache; what it takes to get near is requests in
+// flight. One workgroup per (group of heads, key range); its four waves take the
+// range's 32-key tiles in turn, each with its own running maximum, sum and
+// accumulators and its own piece of LDS (the V tile it transposes): no barrier
+// until the end, where wave 0 merges the four states. With more than one range
+// the merged state goes to the scratchpad (unnormalised accumulators, maximum,
+// sum per query) and sdpa_combine_kernel finishes.
+//   * p.pack heads that share a K / V head ride in the 16 query columns of one
+//     MFMA (pack * Qn <= 16), so a grouped cache is read once per pack and not
+//     once per head;
+//   * a wave requests two tiles ahead (one where 16-bit head size 256 leaves no
+//     registers for two). The request has no branch: a load behind a run-time
+//     choice of its data type makes the compiler wait for every load before it.
+//     QUANT = 1 is the cache with f16 scales and byte zero points, QUANT = 2 the
+//     rest (f32 scales, s32 zero points, bf16 queries), which keeps the choices;
+//   * QUANT = 1: the lane that fetched a key's scale and zero point writes them to
+//     LDS as the packed f16 operands of the dequantization, one 8-byte read for
+//     each use; keys past the end are looked for in the last tile only.
+// 1 query, head size 128, launches back to back with the combining kernel, before /
+// after (us): 32 heads x 8191 keys, s8 29.2 / 24.0, f16 29.6 / 28.7; x 32768 keys, s8
+// 79.6 / 55.4 (4.9 TB/s), f16 100.6 / 98.4; 8 K / V heads, bf16, 8191 keys 29.8 / 15.6,
+// 32768 86.1 / 30.8; 4 K / V heads, s8, 32768 75.7 / 22.4.
+template <int DC, int QUANT, bool MASKED, bool BF>
+__global__ void __launch_bounds__(SDPA_WAVES * 64, DC > 4 ? 1 : 2)
 sdpa_decode_kernel(const sdpa_params_t p) {
     constexpr int D = 32 * DC;
     constexpr int DVB = D / 16;
     constexpr int V_PITCH = D * 2 + 32;
     constexpr int ST = D + 2; // floats of one query's state
-    __shared__ __attribute__((aligned(16))) uint8_t lds_v4[SDPA_WAVES][SDPA_KT * V_PITCH];
-    __shared__ float lds_st[SDPA_WAVES][16 * ST];
-    // a tile's 32 key scales and zero points of K and of V, per wave
-    __shared__ float lds_q[SDPA_WAVES][4 * SDPA_KT];
+    constexpr int SLOTS = !QUANT && DC > 4 ? 1 : 2; // tiles requested ahead
+    constexpr int V_BYTES = SDPA_KT * V_PITCH, ST_BYTES = 16 * ST * 4;
+    constexpr int W_BYTES = V_BYTES > ST_BYTES ? V_BYTES : ST_BYTES;
+    // per wave: the V tile while it walks, its state at the end
+    __shared__ __attribute__((aligned(16))) uint8_t lds_w[SDPA_WAVES][W_BYTES];
+    // a tile's 32 keys: {zero point, scale} operands of K, then of V, per wave
+    __shared__ __attribute__((aligned(16))) uint32_t lds_q[SDPA_WAVES][4 * SDPA_KT];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, c = lane >> 4;
-    const int head = blockIdx.x, split = blockIdx.y;
-    const int b1 = head % p.B1, b0 = head / p.B1;
-    const int kb0 = b0 / p.kv_div0, kb1 = b1 / p.kv_div1;
-    const uint16_t *Qb = p.Q + b0 * p.q.b0 + b1 * p.q.b1;
+    const int split = blockIdx.y;
+    const int packs = p.B1 / p.pack;
+    const int b1_0 = blockIdx.x % packs * p.pack, b0 = blockIdx.x / packs;
+    const int kb0 = b0 / p.kv_div0, kb1 = b1_0 / p.kv_div1;
+    // column r of the MFMAs: query q of head b1 (columns past the last repeat it)
+    const int rows = p.pack * p.Qn, rc = min(r, rows - 1);
+    const int b1 = b1_0 + rc / p.Qn, q = rc % p.Qn;
     const uint8_t *Kb8 = (const uint8_t *)p.K, *Vb8 = (const uint8_t *)p.V;
     const int64_t k_base = kb0 * p.k.b0 + kb1 * p.k.b1;
     const int64_t v_base = kb0 * p.v.b0 + kb1 * p.v.b1;
     const int64_t qz_base = kb0 * p.qz_b0 + kb1 * p.qz_b1;
-    uint8_t *lds_v = lds_v4[wave];
+    uint8_t *lds_v = lds_w[wave];
 
-    const int q = r; // the single 16-query block; rows past Qn repeat the last
-    v8h qf[DC];
+    int n_tiles = (p.S + SDPA_KT - 1) / SDPA_KT;
+    if (p.causal) n_tiles = min(n_tiles, (p.Qn - 1) / SDPA_KT + 1);
+    const int t_begin = split * p.tps, t_end = min(n_tiles, t_begin + p.tps);
+
+    // K fragments straight from memory in operand order (lane (r, c): key
+    // 16 kb + r, 8 values at 32 dc + 8 c); V rows through the wave's LDS piece
+    uint4 kr[SLOTS][2][DC], vr[SLOTS][D / 16];
+    uint32_t qsz[SLOTS][2]; // lanes 0..31: scale, zero point of K's key; 32..63: V's
+    const bool up = lane >= 32;
+    // (absent buffers: the cache stands in, the value is replaced below)
+    const void *const sp = up ? p.v_scale : p.k_scale, *const zp = up ? p.v_zp : p.k_zp;
+    const uint16_t *const sp1 = sp ? (const uint16_t *)sp + qz_base : nullptr;
+    const uint8_t *const zp1 = zp ? (const uint8_t *)zp + qz_base : nullptr;
+    auto fetch = [&](int kt, auto slot_tag) {
+        constexpr int sl = decltype(slot_tag)::value;
 #pragma unroll
-    for (int dc = 0; dc < DC; dc++)
-        qf[dc] = *(const v8h *)(Qb + (int64_t)min(q, p.Qn - 1) * p.q.row + dc * 32
-                + c * 8);
+        for (int kb = 0; kb < 2; kb++) {
+            const int key = min(kt * SDPA_KT + kb * 16 + r, p.S - 1);
+#pragma unroll
+            for (int dc = 0; dc < DC; dc++) {
+                if (!QUANT) {
+                    kr[sl][kb][dc] = *(const uint4 *)((const uint16_t *)Kb8 + k_base
+                            + key * p.k.row + dc * 32 + c * 8);
+                } else {
+                    const uint2 w = *(const uint2 *)(Kb8 + k_base + key * p.k.row
+                            + dc * 32 + c * 8);
+                    kr[sl][kb][dc] = make_uint4(w.x, w.y, 0, 0);
+                }
+            }
+        }
+        // V: the tile's 8-element pieces in turn (piece i: key i / (D / 8), chunk
+        // i % (D / 8)), lane l carries the pieces l, l + 64, ...
+#pragma unroll
+        for (int n = 0; n < D / 16; n++) {
+            const int i = lane + 64 * n;
+            const int kk = i / (D / 8), ch = i % (D / 8);
+            const int key = min(kt * SDPA_KT + kk, p.S - 1);
+            if (!QUANT) {
+                vr[sl][n] = *(const uint4 *)((const uint16_t *)Vb8 + v_base
+                        + key * p.v.row + ch * 8);
+            } else {
+                const uint2 w = *(const uint2 *)(Vb8 + v_base + key * p.v.row
+                        + ch * 8);
+                vr[sl][n] = make_uint4(w.x, w.y, 0, 0);
+            }
+        }
+        // one scale and one zero point per lane: the tile's 32 keys, K's in the
+        // lower half of the wave, V's in the upper
+        const int key = min(kt * SDPA_KT + (lane & 31), p.S - 1);
+        if constexpr (QUANT == 1) {
+            const uint16_t *const s1 = sp1 ? sp1 + key : (const uint16_t *)p.Q;
+            const uint8_t *const z1 = zp1 ? zp1 + key : (const uint8_t *)p.Q;
+            qsz[sl][0] = *s1;
+            qsz[sl][1] = *z1;
+        } else if constexpr (QUANT == 2) {
+            qsz[sl][0] = f2u(sp ? ld_scale(up ? p.vs_dt : p.ks_dt, sp, qz_base + key)
+                                : 1.f);
+            qsz[sl][1] = f2u(
+                    zp ? ld_zp(up ? p.vz_dt : p.kz_dt, zp, qz_base + key) : 0.f);
+        }
+    };
+    // Everything is requested before anything is looked at, in the order of use: a
+    // wait for a load is a wait for all loads before it.
+    const uint16_t *const sc_ptr = (const uint16_t *)(p.scale ? p.scale : p.Q);
+    const uint16_t sc_raw[2] = {sc_ptr[0], sc_ptr[p.scale_dt == dt_f32 ? 1 : 0]};
+    v8h qf[DC];
+    const uint16_t *Qb = p.Q + b0 * p.q.b0 + b1 * p.q.b1 + (int64_t)q * p.q.row;
+#pragma unroll
+    for (int dc = 0; dc < DC; dc++) qf[dc] = *(const v8h *)(Qb + dc * 32 + c * 8);
+    int kt = t_begin + wave;
+    using slot0 = std::integral_constant<int, 0>;
+    using slot1 = std::integral_constant<int, SLOTS - 1>;
+    if (kt < t_end) {
+        fetch(kt, slot0 {});
+        if (SLOTS > 1 && kt + SDPA_WAVES < t_end) fetch(kt + SDPA_WAVES, slot1 {});
+    }
+
     float sc = 1.f;
     if (p.scale) {
-        sc = load_float(p.scale_dt, p.scale, 0);
+        const uint32_t h = sc_raw[0], w = h | ((uint32_t)sc_raw[1] << 16);
+        sc = p.scale_dt == dt_f32 ? u2f(w)
+                : p.scale_dt == dt_bf16
+                ? u2f(h << 16)
+                : (float)__builtin_bit_cast(_Float16, (uint16_t)h);
         if (p.invert_scale) sc = 1.f / sc;
     }
     constexpr float L2E = 1.44269504088896340736f;
@@ -561,64 +660,17 @@ sdpa_decode_kernel(const sdpa_params_t p) {
     for (int d = 0; d < DVB; d++) oacc[d] = v4f {0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
 
-    int n_tiles = (p.S + SDPA_KT - 1) / SDPA_KT;
-    if (p.causal) n_tiles = min(n_tiles, (p.Qn - 1) / SDPA_KT + 1);
-    const int t_begin = split * p.tps, t_end = min(n_tiles, t_begin + p.tps);
-
-    // K fragments straight from memory in operand order (lane (r, c): key
-    // 16 kb + r, 8 values at 32 dc + 8 c); V rows through the wave's LDS piece
-    uint4 kr[2][DC], vr[D / 16];
-    float qsz[2]; // lanes 0..31: K scale, zero point of key lane; 32..63: V's
-    float *qz = lds_q[wave];
-    auto fetch = [&](int kt) {
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++) {
-            const int key = min(kt * SDPA_KT + kb * 16 + r, p.S - 1);
-#pragma unroll
-            for (int dc = 0; dc < DC; dc++) {
-                if (!QUANT) {
-                    kr[kb][dc] = *(const uint4 *)((const uint16_t *)Kb8 + k_base
-                            + key * p.k.row + dc * 32 + c * 8);
-                } else {
-                    const uint2 w = *(const uint2 *)(Kb8 + k_base + key * p.k.row
-                            + dc * 32 + c * 8);
-                    kr[kb][dc] = make_uint4(w.x, w.y, 0, 0);
-                }
-            }
-        }
-        if (QUANT) {
-            // one scale and one zero point per lane: the tile's 32 keys, K's in
-            // the lower half of the wave, V's in the upper
-            const int key = min(kt * SDPA_KT + (lane & 31), p.S - 1);
-            const bool up = lane >= 32;
-            const void *sp = up ? p.v_scale : p.k_scale;
-            const void *zp = up ? p.v_zp : p.k_zp;
-            qsz[0] = sp ? ld_scale(up ? p.vs_dt : p.ks_dt, sp, qz_base + key) : 1.f;
-            qsz[1] = zp ? ld_zp(up ? p.vz_dt : p.kz_dt, zp, qz_base + key) : 0.f;
-        }
-        // V: the tile's 8-element pieces in turn (piece i: key i / (D / 8), chunk
-        // i % (D / 8)), lane l carries the pieces l, l + 64, ...
-#pragma unroll
-        for (int n = 0; n < D / 16; n++) {
-            const int i = lane + 64 * n;
-            const int kk = i / (D / 8), ch = i % (D / 8);
-            const int key = min(kt * SDPA_KT + kk, p.S - 1);
-            if (!QUANT) {
-                vr[n] = *(const uint4 *)((const uint16_t *)Vb8 + v_base
-                        + key * p.v.row + ch * 8);
-            } else {
-                const uint2 w = *(const uint2 *)(Vb8 + v_base + key * p.v.row
-                        + ch * 8);
-                vr[n] = make_uint4(w.x, w.y, 0, 0);
-            }
-        }
-    };
-    auto dequant8 = [&](const uint4 &raw, float s1, float z1) {
-        const bool sgn = p.kv_dt == dt_s8;
-        const uint32_t flip = sgn ? 0x80808080u : 0u;
-        const float zb = z1 + (sgn ? 128.f : 0.f);
+    uint32_t *const qz = lds_q[wave];
+    const bool sgn = p.kv_dt == dt_s8;
+    const uint32_t flip = sgn ? 0x80808080u : 0u;
+    // eight cache bytes of tile key `kk` (row `half`: 0 K, 1 V) -> the 16-bit type
+    auto dequant8 = [&](const uint4 &raw, int half, int kk) {
         const uint32_t w[2] = {raw.x ^ flip, raw.y ^ flip};
-        if (p.fastq) return dequant8_f16(w[0], w[1], s1, zb);
+        const uint2 o = *(const uint2 *)&qz[(half * SDPA_KT + kk) * 2];
+        if constexpr (QUANT == 1)
+            return dequant8_f16(w[0], w[1], __builtin_bit_cast(h2, o.y),
+                    __builtin_bit_cast(h2, o.x));
+        const float zb = u2f(o.x), s1 = u2f(o.y);
         uint32_t h[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -629,36 +681,51 @@ sdpa_decode_kernel(const sdpa_params_t p) {
                 h[4] | (h[5] << 16), h[6] | (h[7] << 16));
     };
 
-    int kt = t_begin + wave;
-    if (kt < t_end) fetch(kt);
-    for (; kt < t_end; kt += SDPA_WAVES) {
+    auto tile = [&](int kt, auto slot_tag) {
+        constexpr int sl = decltype(slot_tag)::value;
         const int key0 = kt * SDPA_KT;
+        const bool last = key0 + SDPA_KT > p.S; // (wave-uniform)
         // this tile's operands out of the request registers
-        if (QUANT) {
-            // [K scale | V scale | K zero point | V zero point] x 32 keys
-            qz[lane] = qsz[0];
-            qz[64 + lane] = qsz[1];
+        if constexpr (QUANT == 1) {
+            const _Float16 one = (_Float16)1.f;
+            const _Float16 s = sp ? __builtin_bit_cast(_Float16, (uint16_t)qsz[sl][0])
+                                  : one;
+            const int zdt = up ? p.vz_dt : p.kz_dt;
+            const int z = !zp ? 0
+                    : zdt == dt_s8 ? (int)(int8_t)qsz[sl][1] : (int)qsz[sl][1];
+            const _Float16 o = (_Float16)(float)(1024 + z + (sgn ? 128 : 0));
+            *(uint2 *)&qz[lane * 2] = make_uint2(
+                    __builtin_bit_cast(uint32_t, h2 {o, o}),
+                    __builtin_bit_cast(uint32_t, h2 {s, s}));
+        } else if constexpr (QUANT == 2) {
+            *(uint2 *)&qz[lane * 2] = make_uint2(
+                    f2u(u2f(qsz[sl][1]) + (sgn ? 128.f : 0.f)), qsz[sl][0]);
         }
         v8h ka[2][DC];
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
             for (int dc = 0; dc < DC; dc++) {
-                uint4 w = QUANT ? dequant8(kr[kb][dc], qz[kb * 16 + r],
-                                          qz[64 + kb * 16 + r])
-                                : kr[kb][dc];
-                if (key0 + kb * 16 + r >= p.S) w = make_uint4(0, 0, 0, 0);
+                uint4 w = kr[sl][kb][dc];
+                if constexpr (QUANT != 0) w = dequant8(w, 0, kb * 16 + r);
                 ka[kb][dc] = __builtin_bit_cast(v8h, w);
             }
+        // (keys past the end: zero, so that probability 0 x V stays 0; their
+        // scores are replaced below)
+        auto v_to_lds = [&](auto last_tag) {
 #pragma unroll
-        for (int n = 0; n < D / 16; n++) {
-            const int i = lane + 64 * n;
-            const int kk = i / (D / 8), ch = i % (D / 8);
-            uint4 w = QUANT ? dequant8(vr[n], qz[32 + kk], qz[96 + kk]) : vr[n];
-            if (key0 + kk >= p.S) w = make_uint4(0, 0, 0, 0);
-            *(uint4 *)(lds_v + kk * V_PITCH + ch * 16) = w;
-        }
-        if (kt + SDPA_WAVES < t_end) fetch(kt + SDPA_WAVES);
+            for (int n = 0; n < D / 16; n++) {
+                const int i = lane + 64 * n;
+                const int kk = i / (D / 8), ch = i % (D / 8);
+                uint4 w = vr[sl][n];
+                if constexpr (QUANT != 0) w = dequant8(w, 1, kk);
+                if (decltype(last_tag)::value && key0 + kk >= p.S)
+                    w = make_uint4(0, 0, 0, 0);
+                *(uint4 *)(lds_v + kk * V_PITCH + ch * 16) = w;
+            }
+        };
+        if (last) v_to_lds(std::true_type {});
+        else v_to_lds(std::false_type {});
 
         v4f st[2] = {v4f {0.f, 0.f, 0.f, 0.f}, v4f {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -666,13 +733,14 @@ sdpa_decode_kernel(const sdpa_params_t p) {
 #pragma unroll
             for (int dc = 0; dc < DC; dc++)
                 st[kb] = mma16<BF>(ka[kb][dc], qf[dc], st[kb]);
+        if (kt + SLOTS * SDPA_WAVES < t_end) fetch(kt + SLOTS * SDPA_WAVES, slot_tag);
         float sv[8];
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
             for (int i = 0; i < 4; i++) sv[kb * 4 + i] = st[kb][i] * sc2;
         if (MASKED) {
-            const int64_t mrow = (int64_t)min(q, p.Qn - 1) * p.m.row;
+            const int64_t mrow = (int64_t)q * p.m.row;
 #pragma unroll
             for (int kb = 0; kb < 2; kb++)
 #pragma unroll
@@ -682,13 +750,16 @@ sdpa_decode_kernel(const sdpa_params_t p) {
                     sv[kb * 4 + i] += L2E * ld_mask(p.mask_dt, mask_b, mo);
                 }
         }
+        if (last || p.causal) {
 #pragma unroll
-        for (int kb = 0; kb < 2; kb++)
+            for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int key = key0 + kb * 16 + 4 * c + i;
-                if (key >= p.S || (p.causal && key > q)) sv[kb * 4 + i] = -INFINITY;
-            }
+                for (int i = 0; i < 4; i++) {
+                    const int key = key0 + kb * 16 + 4 * c + i;
+                    if (key >= p.S || (p.causal && key > q))
+                        sv[kb * 4 + i] = -INFINITY;
+                }
+        }
         float mt = sv[0];
 #pragma unroll
         for (int i = 1; i < 8; i++) mt = fmaxf(mt, sv[i]);
@@ -696,6 +767,7 @@ sdpa_decode_kernel(const sdpa_params_t p) {
         const float m_new = fmaxf(m_run, mt);
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const bool moved = m_new != m_run;
         m_run = m_new;
         float ls = 0.f;
         _Float16 ph[8];
@@ -706,10 +778,14 @@ sdpa_decode_kernel(const sdpa_params_t p) {
             ph[i] = cvt16<BF>(pv1);
         }
         l_run = l_run * alpha + ls;
+        // the accumulators only move when some query's maximum did
+        if (__builtin_amdgcn_ballot_w64(moved)) {
+#pragma unroll
+            for (int d = 0; d < DVB; d++) oacc[d] *= alpha;
+        }
         const v8h pb = v8h {ph[0], ph[1], ph[2], ph[3], ph[4], ph[5], ph[6], ph[7]};
 #pragma unroll
         for (int d = 0; d < DVB; d++) {
-            oacc[d] *= alpha;
             const uint8_t *va = lds_v + (4 * c + (r >> 2)) * V_PITCH
                     + (d * 16 + 4 * (r & 3)) * 2;
             const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -721,11 +797,16 @@ sdpa_decode_kernel(const sdpa_params_t p) {
                     v8s {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
             oacc[d] = mma16<BF>(a, pb, oacc[d]);
         }
+    };
+    for (; kt < t_end; kt += SLOTS * SDPA_WAVES) {
+        tile(kt, slot0 {});
+        if (SLOTS > 1 && kt + SDPA_WAVES < t_end) tile(kt + SDPA_WAVES, slot1 {});
     }
 
     // ---- merge the four waves' states: query r, accumulator rows d = 16 dv + 4 c + i
+    // (over the wave's own V tile, which it has read)
     const float l_wave = rows_sum(l_run);
-    float *mine = lds_st[wave] + r * ST;
+    float *mine = (float *)lds_w[wave] + r * ST;
 #pragma unroll
     for (int d = 0; d < DVB; d++)
 #pragma unroll
@@ -736,17 +817,20 @@ sdpa_decode_kernel(const sdpa_params_t p) {
     }
     __syncthreads();
     if (wave != 0) return;
+    const float *state[SDPA_WAVES];
+#pragma unroll
+    for (int w = 0; w < SDPA_WAVES; w++) state[w] = (const float *)lds_w[w] + r * ST;
     float m_all = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < SDPA_WAVES; w++) m_all = fmaxf(m_all, lds_st[w][r * ST + D]);
+    for (int w = 0; w < SDPA_WAVES; w++) m_all = fmaxf(m_all, state[w][D]);
     const float m_use = m_all == -INFINITY ? 0.f : m_all;
     float l_all = 0.f, wgt[SDPA_WAVES];
 #pragma unroll
     for (int w = 0; w < SDPA_WAVES; w++) {
-        wgt[w] = __builtin_amdgcn_exp2f(lds_st[w][r * ST + D] - m_use);
-        l_all += wgt[w] * lds_st[w][r * ST + D + 1];
+        wgt[w] = __builtin_amdgcn_exp2f(state[w][D] - m_use);
+        l_all += wgt[w] * state[w][D + 1];
     }
-    if (q >= p.Qn) return;
+    if (r >= rows) return;
     if (p.nsplit == 1) {
         uint16_t *Ob = p.dst + b0 * p.o.b0 + b1 * p.o.b1 + (int64_t)q * p.o.row;
 #pragma unroll
@@ -757,14 +841,15 @@ sdpa_decode_kernel(const sdpa_params_t p) {
                 float o = 0.f;
 #pragma unroll
                 for (int w = 0; w < SDPA_WAVES; w++)
-                    o += wgt[w] * lds_st[w][r * ST + d * 16 + 4 * c + i];
+                    o += wgt[w] * state[w][d * 16 + 4 * c + i];
                 h[i] = __builtin_bit_cast(uint16_t, cvt16<BF>(o / l_all));
             }
             *(uint2 *)(Ob + d * 16 + 4 * c) = make_uint2(
                     h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
         }
     } else {
-        float *out = p.part + (((int64_t)head * p.nsplit + split) * 16 + q) * ST;
+        const int64_t head = (int64_t)b0 * p.B1 + b1;
+        float *out = p.part + ((head * p.nsplit + split) * p.Qn + q) * ST;
 #pragma unroll
         for (int d = 0; d < DVB; d++)
 #pragma unroll
@@ -772,7 +857,7 @@ sdpa_decode_kernel(const sdpa_params_t p) {
                 float o = 0.f;
 #pragma unroll
                 for (int w = 0; w < SDPA_WAVES; w++)
-                    o += wgt[w] * lds_st[w][r * ST + d * 16 + 4 * c + i];
+                    o += wgt[w] * state[w][d * 16 + 4 * c + i];
                 out[d * 16 + 4 * c + i] = o;
             }
         if (c == 0) {
@@ -793,11 +878,13 @@ sdpa_combine_kernel(const sdpa_params_t p, const int D) {
     const int head = blockIdx.x, q = blockIdx.y, t = threadIdx.x;
     const int b1 = head % p.B1, b0 = head / p.B1;
     const int ST = D + 2;
-    const float *st = p.part + ((int64_t)head * p.nsplit * 16 + q) * ST;
+    // state of split s: row s * Qn + q of the head
+    const float *st = p.part + ((int64_t)head * p.nsplit * p.Qn + q) * ST;
+    const int64_t step = (int64_t)p.Qn * ST;
     // every thread finds the maximum itself (at most 256 values from L2)
     float m_all = -INFINITY;
     for (int s1 = t; s1 < p.nsplit; s1 += 128)
-        m_all = fmaxf(m_all, st[(int64_t)s1 * 16 * ST + D]);
+        m_all = fmaxf(m_all, st[s1 * step + D]);
 #pragma unroll
     for (int o = 32; o; o >>= 1) m_all = fmaxf(m_all, __shfl_xor(m_all, o));
     if ((t & 63) == 0) red[t >> 6] = m_all;
@@ -806,7 +893,7 @@ sdpa_combine_kernel(const sdpa_params_t p, const int D) {
     const float m_use = m_all == -INFINITY ? 0.f : m_all;
     float l_part = 0.f;
     for (int s1 = t; s1 < p.nsplit; s1 += 128) {
-        const float *e = st + (int64_t)s1 * 16 * ST;
+        const float *e = st + s1 * step;
         const float w = __builtin_amdgcn_exp2f(e[D] - m_use);
         w_s[s1] = w;
         l_part += w * e[D + 1];
@@ -821,7 +908,7 @@ sdpa_combine_kernel(const sdpa_params_t p, const int D) {
         float o = 0.f;
 #pragma unroll 8
         for (int s1 = 0; s1 < p.nsplit; s1++)
-            o += w_s[s1] * st[(int64_t)s1 * 16 * ST + d];
+            o += w_s[s1] * st[s1 * step + d];
         p.dst[b0 * p.o.b0 + b1 * p.o.b1 + (int64_t)q * p.o.row + d]
                 = p.bf ? f32_to_bf16(o / l_all)
                        : __builtin_bit_cast(uint16_t, (_Float16)(o / l_all));
@@ -830,16 +917,26 @@ sdpa_combine_kernel(const sdpa_params_t p, const int D) {
 
 // how a decode-sized problem is cut over the keys
 struct sdpa_split_t {
-    int nsplit, tps;
+    int nsplit, tps, pack;
 };
-sdpa_split_t decode_split(int64_t heads, int64_t S, int64_t Qn, bool causal) {
+sdpa_split_t decode_split(const sdpa_params_t &p) {
+    const int64_t S = p.S, Qn = p.Qn;
+    const bool causal = p.causal != 0;
+    sdpa_split_t r;
+    // the most heads of a group whose queries fit the MFMA's 16 columns
+    r.pack = 1;
+    for (int h = p.kv_div1; h > 1; h--)
+        if (p.kv_div1 % h == 0 && h * Qn <= 16) {
+            r.pack = h;
+            break;
+        }
+    const int64_t heads = (int64_t)p.B0 * p.B1 / r.pack;
     int64_t tiles = (S + SDPA_KT - 1) / SDPA_KT;
     if (causal) tiles = std::min<int64_t>(tiles, (Qn - 1) / SDPA_KT + 1);
     // enough workgroups to fill the chip twice, at least one tile per wave
     int64_t want = std::max<int64_t>(1, 512 / std::max<int64_t>(1, heads));
     int64_t tps = std::max<int64_t>(SDPA_WAVES, (tiles + want - 1) / want);
     tps = (tps + SDPA_WAVES - 1) / SDPA_WAVES * SDPA_WAVES;
-    sdpa_split_t r;
     r.tps = (int)tps;
     r.nsplit = (int)std::max<int64_t>(1, (tiles + tps - 1) / tps);
     if (r.nsplit > SDPA_MAX_SPLIT) {
@@ -1013,11 +1110,10 @@ const char *qmm_sdpa_impl_name(const qmm_sdpa_desc_t *desc) {
 size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc) {
     sdpa_params_t p;
     if (!desc || !supported(*desc, &p) || p.Qn > 16) return 0;
-    const sdpa_split_t sp
-            = decode_split((int64_t)p.B0 * p.B1, p.S, p.Qn, p.causal != 0);
+    const sdpa_split_t sp = decode_split(p);
     if (sp.nsplit <= 1) return 0;
     const int64_t D = desc->q.dims[desc->q.ndims - 1];
-    return (size_t)p.B0 * p.B1 * sp.nsplit * 16 * (D + 2) * sizeof(float);
+    return (size_t)p.B0 * p.B1 * sp.nsplit * p.Qn * (D + 2) * sizeof(float);
 }
 
 int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
@@ -1050,13 +1146,13 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
     const bool qn = p.kv_dt != desc->q.dt, mk = p.mask != nullptr;
     const bool bf = p.bf != 0;
     if (p.Qn <= 16) {
-        const sdpa_split_t sp
-                = decode_split((int64_t)p.B0 * p.B1, p.S, p.Qn, p.causal != 0);
+        const sdpa_split_t sp = decode_split(p);
         p.nsplit = sp.nsplit;
+        p.pack = sp.pack;
         p.tps = sp.tps;
         p.part = (float *)args->scratch;
         if (p.nsplit > 1 && !p.part) return QMM_INVALID_ARGUMENTS;
-        const dim3 dgrid((unsigned)(p.B0 * p.B1), (unsigned)p.nsplit);
+        const dim3 dgrid((unsigned)(p.B0 * (p.B1 / p.pack)), (unsigned)p.nsplit);
         auto god = [&](auto kern) {
             hipLaunchKernelGGL(kern, dgrid, dim3(SDPA_WAVES * 64), 0,
                     (hipStream_t)hip_stream, p);
@@ -1064,22 +1160,37 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
         // template arguments from the run-time choices
 #define SDPA_PICK(KERN, GO, DCV) \
     switch ((qn ? 4 : 0) | (bf ? 2 : 0) | (mk ? 1 : 0)) { \
-        case 0: GO(KERN<DCV, false, false, false>); break; \
-        case 1: GO(KERN<DCV, false, true, false>); break; \
-        case 2: GO(KERN<DCV, false, false, true>); break; \
-        case 3: GO(KERN<DCV, false, true, true>); break; \
-        case 4: GO(KERN<DCV, true, false, false>); break; \
-        case 5: GO(KERN<DCV, true, true, false>); break; \
-        case 6: GO(KERN<DCV, true, false, true>); break; \
-        case 7: GO(KERN<DCV, true, true, true>); break; \
+        case 0: GO(KERN<DCV, 0, false, false>); break; \
+        case 1: GO(KERN<DCV, 0, true, false>); break; \
+        case 2: GO(KERN<DCV, 0, false, true>); break; \
+        case 3: GO(KERN<DCV, 0, true, true>); break; \
+        case 4: GO(KERN<DCV, 1, false, false>); break; \
+        case 5: GO(KERN<DCV, 1, true, false>); break; \
+        case 6: GO(KERN<DCV, 1, false, true>); break; \
+        case 7: GO(KERN<DCV, 1, true, true>); break; \
+        default: return QMM_UNIMPLEMENTED; \
+    }
+// (a bf16 kernel has no packed dequantization: QUANT = 2 there)
+#define SDPA_PICK_DECODE(DCV) \
+    switch ((qn ? (p.fastq ? 4 : 8) : 0) | (bf ? 2 : 0) | (mk ? 1 : 0)) { \
+        case 0: god(sdpa_decode_kernel<DCV, 0, false, false>); break; \
+        case 1: god(sdpa_decode_kernel<DCV, 0, true, false>); break; \
+        case 2: god(sdpa_decode_kernel<DCV, 0, false, true>); break; \
+        case 3: god(sdpa_decode_kernel<DCV, 0, true, true>); break; \
+        case 4: god(sdpa_decode_kernel<DCV, 1, false, false>); break; \
+        case 5: god(sdpa_decode_kernel<DCV, 1, true, false>); break; \
+        case 8: god(sdpa_decode_kernel<DCV, 2, false, false>); break; \
+        case 9: god(sdpa_decode_kernel<DCV, 2, true, false>); break; \
+        case 10: god(sdpa_decode_kernel<DCV, 2, false, true>); break; \
+        case 11: god(sdpa_decode_kernel<DCV, 2, true, true>); break; \
         default: return QMM_UNIMPLEMENTED; \
     }
         switch (D) {
-            case 32: SDPA_PICK(sdpa_decode_kernel, god, 1) break;
-            case 64: SDPA_PICK(sdpa_decode_kernel, god, 2) break;
-            case 96: SDPA_PICK(sdpa_decode_kernel, god, 3) break;
-            case 128: SDPA_PICK(sdpa_decode_kernel, god, 4) break;
-            case 256: SDPA_PICK(sdpa_decode_kernel, god, 8) break;
+            case 32: SDPA_PICK_DECODE(1) break;
+            case 64: SDPA_PICK_DECODE(2) break;
+            case 96: SDPA_PICK_DECODE(3) break;
+            case 128: SDPA_PICK_DECODE(4) break;
+            case 256: SDPA_PICK_DECODE(8) break;
             default: return QMM_UNIMPLEMENTED;
         }
         if (p.nsplit > 1)
@@ -1117,6 +1228,7 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
         default: return QMM_UNIMPLEMENTED;
     }
 #undef SDPA_PICK
+#undef SDPA_PICK_DECODE
     return hipGetLastError() == hipSuccess ? QMM_OK : QMM_RUNTIME_ERROR;
 }
 

@@ -1,0 +1,62 @@
+"""Few queries against a grouped K / V cache: the heads of a group share a workgroup, their queries the 16 columns of
+one MFMA (as many whole divisors of the group as fit). Against float64 attention under the comparison rule of the
+reference's own SDPA test, as the cases beside this file."""
+import numpy as np
+import pytest
+
+import onednn_amd as dnnl
+from qmm_harness import dt
+from test_gpu_sdpa import attention64, f16, f16_to_f64, reference_rule, run_sdpa
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    eng = dnnl.engine(dnnl.engine.kind.gpu, 0)
+    return eng, dnnl.stream(eng)
+
+
+@pytest.mark.parametrize("qdt", [dt.f16, dt.bf16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("rep,Qn,S,D,mkind,quant", [
+    (16, 1, 1, 64, "none", None), (5, 3, 700, 128, "per_head", None), (6, 4, 300, 96, "causal", None),
+    (7, 1, 2049, 128, "per_head", "f16"), (4, 4, 33, 32, "none", "f32"), (8, 1, 4100, 256, "none", "f16"),
+    (32, 1, 640, 128, "per_head", "f32"), (3, 9, 129, 64, "causal", None),
+], ids=str)
+def test_heads_of_a_group_share_a_workgroup(ctx, rep, Qn, S, D, mkind, quant, qdt):
+    print("[case] sdpa grouped rep=%d Qn=%d S=%d D=%d %s %s %s" % (rep, Qn, S, D, mkind, quant, qdt), flush=True)
+    MB, KH = 2, 2
+    H = KH * rep
+    r = np.random.default_rng(rep * 100 + S)
+    q = f16(r.standard_normal((MB, H, Qn, D)), qdt)
+    scale = 1.0 / np.sqrt(D)
+    mask = None
+    if mkind == "per_head":
+        mask = (r.standard_normal((1, H, Qn, S)) * 2).astype(np.float32)
+        mask[..., 1::6] = -np.inf
+    kw = dict(scale=scale, mask=mask, causal=mkind == "causal", kv_heads=KH, qdt=qdt)
+    if quant is None:
+        k, v = f16(r.standard_normal((MB, KH, S, D)), qdt), f16(r.standard_normal((MB, KH, S, D)), qdt)
+        got = run_sdpa(ctx, q, k, v, **kw)
+        k64, v64 = f16_to_f64(k, qdt), f16_to_f64(v, qdt)
+    else:
+        k = r.integers(-128, 128, (MB, KH, S, D)).astype(np.int8)
+        v = r.integers(-128, 128, (MB, KH, S, D)).astype(np.int8)
+        sdt, zdt, znp = (dt.f16, dt.s8, np.int8) if quant == "f16" else (dt.f32, dt.s32, np.int32)
+        side = []
+        for x, groups in ((k, (D, 1)), (v, (1, D))):
+            sc = r.uniform(0.005, 0.02, (KH, S)).astype(np.float32)
+            raw = f16(sc) if quant == "f16" else sc
+            val = f16_to_f64(raw) if quant == "f16" else sc.astype(np.float64)
+            zp = r.integers(-6, 7, (KH, S)).astype(znp)
+            # the cache as the reorder to the queries' type gives it
+            x64 = f16_to_f64(f16((x - zp[None, ..., None].astype(np.float64)) * val[None, ..., None], qdt), qdt)
+            side.append((x64, (0b1110, groups, sdt, raw, zdt, zp)))
+        got = run_sdpa(ctx, q, k, v, kv_dt=dt.s8, k_q=side[0][1], v_q=side[1][1], **kw)
+        k64, v64 = side[0][0], side[1][0]
+    s_eff = float(f16_to_f64(f16(np.array([scale]), qdt), qdt)[0])
+    gold = attention64(f16_to_f64(q, qdt), np.swapaxes(k64, -1, -2), v64, s_eff,
+                       None if mask is None else mask.astype(np.float64), mkind == "causal", rep)
+    bad, total, worst = reference_rule(f16_to_f64(got, qdt), gold, 0.001466 if qdt == dt.f16 else 0.0079)
+    print("[sdpa grouped] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
+    assert bad <= total * 0.0006
