@@ -25,7 +25,9 @@
 //     in a group of 128) and the conversion, the subtraction of the bias and the
 //     product with the row scale are one fma: fma(f, ss, -1.5 * 2^23 * ss). The
 //     bias times a 16-bit scale is exact, so the one rounding is that of
-//     (float)sum * ss. Two vector instructions per result and group, not three;
+//     (float)sum * ss. Two vector instructions per result and group, not three.
+//     Where the product with the bias overflows (an infinite scale, a bf16 one of
+//     2^100 and more), the sums are formed again with (f - 1.5 * 2^23) * ss;
 //   * the row and column scales of the next group are fetched by the threads
 //     of the workgroup, one of each, and go through LDS as f32: no pre-pass.
 // Source rows come through LDS (double-buffered per group, direct loads), a
@@ -237,24 +239,28 @@ gemm_g128_kernel(const g128_params_t p) {
         }
     };
     constexpr float BIAS = 12582912.f; // 1.5 * 2^23, bits 0x4B400000
+    int huge = 0; // s8: a row scale whose product with BIAS is no number
     auto stage_x = [&](int g) { // s8: the fetched scales of group g to LDS
         if constexpr (S8) {
             float *x = (float *)(lds + G::X_OFF + (g & 1) * G::X_BYTES);
             const float s = half_bits(raw_row, p.ss_f16);
             if (tid < BM) *(float2 *)(x + 2 * tid) = make_float2(s, -BIAS * s);
+            huge |= !(__builtin_fabsf(s) < 0x1p100f);
             x[2 * BM + tid] = half_bits(raw_col[0], p.sw_f16) * 0.0625f;
         }
     };
 
     float res[FM][FN][4]; // (scalars: as vectors they must lie in aligned tuples)
+    const v4f p0 = S8 ? v4f {BIAS, BIAS, BIAS, BIAS} : v4f {0.f, 0.f, 0.f, 0.f};
+
+    auto sum_groups = [&](auto any_scale) {
+    constexpr bool ANY_SCALE = decltype(any_scale)::value;
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
         for (int j = 0; j < FN; j++)
 #pragma unroll
             for (int e = 0; e < 4; e++) res[i][j][e] = 0.f;
-
-    const v4f p0 = S8 ? v4f {BIAS, BIAS, BIAS, BIAS} : v4f {0.f, 0.f, 0.f, 0.f};
 
     fetch_x(0);
     fetch_a(0);
@@ -398,7 +404,9 @@ gemm_g128_kernel(const g128_params_t p) {
                         const int jf = q / 4, e = q % 4;
                         const float v = P[u & 1][jf][e];
                         float &o = res[i][j0 + jf][e];
-                        if constexpr (S8)
+                        if constexpr (S8 && ANY_SCALE)
+                            o = __builtin_fmaf((v - BIAS) * ss[i & 1].x, sw[jf][e], o);
+                        else if constexpr (S8)
                             o = __builtin_fmaf(
                                     __builtin_fmaf(v, ss[i & 1].x, ss[i & 1].y),
                                     sw[jf][e], o);
@@ -416,7 +424,17 @@ gemm_g128_kernel(const g128_params_t p) {
         }
         stage_x(g + 1);
     }
-    __syncthreads(); // LDS is reused by the epilogue
+    };
+    sum_groups(std::false_type {});
+    // LDS is reused behind this barrier, by the sums once more or the epilogue
+    if constexpr (S8) {
+        if (__syncthreads_or(huge)) {
+            sum_groups(std::true_type {});
+            __syncthreads();
+        }
+    } else {
+        __syncthreads();
+    }
 
     // ---- epilogue: up to 64 rows at a time through a wave-private LDS tile, so that a
     // lane gets four neighbouring columns of a row and 16 lanes a whole row piece

@@ -56,6 +56,29 @@ def test_s8_extreme_sums(ctx):
     assert_bit_exact(got, p.run_oracle(), "extremes")
 
 
+@pytest.mark.parametrize("name", ["bf16_2e110", "f16_inf"])
+@pytest.mark.parametrize("M", [129, 640])
+def test_s8_huge_row_scales(ctx, M, name):
+    """Row scales whose product with the bias of the sums is no f32 number: finite results stay exact, an infinite
+    scale gives infinities of the sums' signs (NaN where a sum is 0)."""
+    eng, strm = ctx
+    print("[case] g128 s8 huge row scales %d %s" % (M, name), flush=True)
+    finite = name == "bf16_2e110"
+    p = dynamic_quant(M, 256, 16640, 23, exact=True, scale_dt=dt.bf16 if finite else dt.f16)
+    mask, code, group, ss = p.scales["src"]
+    ss = np.array(ss, dtype=np.float64)
+    ss[5, 0] = ss[M - 1, 1] = 2.0 ** 110 if finite else np.inf
+    p.scales["src"] = (mask, code, group, ss)
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == W4A8
+    want = p.run_oracle()
+    got, want = O.to_f32(p.dst.dt, got).reshape(M, -1), O.to_f32(p.dst.dt, want).reshape(M, -1)
+    assert np.isfinite(want).all() == finite
+    if finite:  # (a row's two groups lie 2^100 apart: one of them is lost in the rounding of the sum)
+        assert np.abs(want[5]).max() > 2.0 ** 100
+    np.testing.assert_array_equal(got, want)
+
+
 def test_s8_arbitrary_scales_and_post_ops(ctx):
     eng, strm = ctx
     print("[case] g128 s8 arbitrary scales", flush=True)
