@@ -283,6 +283,13 @@ QMM_API int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc,
  * reference. */
 QMM_API int qmm_gemm_stamps_read(void *host, size_t bytes);
 
+/* Rows of the tile (64, 96 or 128) with which the tiled kernel for 4-bit weights
+ * takes an M x N x K problem with groups of 128 k under src_dt activations (s8,
+ * f16, bf16), or 0 where its sizes leave it to the other kernels of
+ * hip:gfx950:mfma_w4a8 / hip:gfx950:decode_w4. Both kinds of kernel carry the same
+ * implementation name; this tells them apart. */
+QMM_API int qmm_gemm_g128_rows(int src_dt, int64_t M, int64_t N, int64_t K);
+
 /* ---- measurement aid ----
  * Launches a kernel that only reads: up to three byte ranges (16-byte aligned,
  * lengths rounded down to 16), pulled with 16-byte vector loads by

@@ -42,7 +42,7 @@ void launch_gemm_w4a8_small(const w4a8_small_t &p, bool has_zp,
         hipStream_t stream);
 bool gemm_w4a8_small_takes(const w4a8_prep_t &q);
 void launch_gemm_g128_s8(const g128_params_t &p, int rows, hipStream_t stream);
-int gemm_g128_rows(int M, int N, bool s8);
+int gemm_g128_rows(int M, int N, int K, int kind);
 void launch_gemm_w4a8_tiny(const w4a8_small_t &p, bool has_zp, int nwv,
         hipStream_t stream);
 int gemm_w4a8_tiny_max_groups(bool half);
@@ -1315,7 +1315,7 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
         // sides: the kernel with the tall wave tiles, which needs no pre-pass
         // (its sums start from the bits of 1.5 * 2^23, which times a 16-bit scale
         // is an f32 number; direct 16-byte loads, 32-bit offsets inside a tile)
-        const int g128_rows = gemm_g128_rows(q.M, q.N, true);
+        const int g128_rows = gemm_g128_rows(q.M, q.N, q.K, G_S8);
         auto is16 = [](int dt) { return dt == dt_f16 || dt == dt_bf16; };
         if (g128_rows && w4a8_variant == 0 && !sc.has_zp && q.gk == 128 && q.ss && q.sw
                 && is16(q.ss_dt) && is16(q.sw_dt) && q.ss_g == 128 && q.sw_g == 128

@@ -40,9 +40,11 @@
 // parts switched off (1000 rows, s8, 88 us): no MFMAs 66, no fold 64, neither 43 us
 // (prologue, expanding, LDS reads, epilogue), no loads inside the loop 88: the parts
 // add up, whether the fold stands behind a row block's MFMAs or between them.
+#include <algorithm>
 #include <type_traits>
 
 #include "qmm_device.hpp"
+#include "qmm_hip.h"
 #include "qmm_plan.hpp"
 
 namespace qmm {
@@ -56,7 +58,6 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
-enum : int { G_S8 = 0, G_F16 = 1, G_BF16 = 2 };
 constexpr int WAVES = 4, FN = 4, WN = 16 * FN, BN = WAVES * WN;
 constexpr int B_WAVE = FN * 1024; // a wave's packed weights of one group
 constexpr int STG_PITCH = WN + 4; // floats per staged row of results
@@ -538,9 +539,24 @@ void launch_gemm_g128_bf16(const g128_params_t &p, int rows, hipStream_t stream)
 }
 #endif
 #else
-// Rows of the tile for an M x N problem, 0: the other kernels are as fast.
-// Measured per group of 128 k (us), one / two workgroups on a CU (a CU that has n
-// takes n / 2 pairs and n % 2 single ones, one after the other):
+// us per group of 128 k for so many tiles, one / two workgroups on a CU (a CU that
+// has n takes n / 2 pairs and n % 2 single ones, one after the other)
+static double group_us(int64_t tiles, double one, double two) {
+    const int64_t n = (tiles + 255) / 256;
+    return (double)(n / 2) * two + (double)(n % 2) * one;
+}
+// us of the kernels of qmm_gemv_w4.hip (up to 16 rows) and qmm_gemm_w4f.hip for few
+// rows. Up to 16 rows: per 1000 columns what launching their workgroups takes, or
+// reading their weights; 17 to 32 rows: rounds of 32 x 128 tiles, one on a CU.
+static double few_rows_us(int M, int N, int groups) {
+    if (M > 16) return (double)(((int64_t)N + 32767) / 32768) * (5.5 + 0.68 * groups);
+    const double launch = M <= 4 ? 0.31 : M <= 8 ? 0.43 : 0.93;
+    const double read = M <= 4 ? 0.012 : M <= 8 ? 0.017 : 0.0178;
+    return 1e-3 * N * std::max(launch, read * groups);
+}
+
+// Rows of the tile for an M x N x K problem, 0: the other kernels are as fast.
+// Measured per group of 128 k (us), one / two workgroups on a CU:
 //   s8:   64 rows 1.10 / 1.45, 128 rows 1.75 / 2.45
 //   f16:  64 rows 1.75 / 2.35,  96 rows 2.2  / 2.7 (bf16 a tenth more on each)
 // The gates: the kernel of qmm_gemm_w4f.hip takes 1.85 us for a 64 x 256 block and
@@ -548,18 +564,40 @@ void launch_gemm_g128_bf16(const g128_params_t &p, int rows, hipStream_t stream)
 // 512 rows, 448 blocks, 117 against 82 us); that of qmm_gemm_w4a8.hip was faster by
 // up to 5 % at 64 ... 128 blocks and slower from 224 on (200 rows 49.4 against
 // 42.2 us; 128 rows 40.9 against 40.9 us; 65 rows x 4096 columns 38.0 against 39.9).
-int gemm_g128_rows(int M, int N, bool s8) {
-    const int64_t tn = (N + 255) / 256;
+// f16 / bf16 with at most 32 rows pass the gate where there are more than 65536
+// columns, and are then a question of time against time: most of a 64-row tile is
+// padding, but the other kernels pay by the column. bf16, other kernels / this one:
+// 4096 x 128256 weights, 1 row 49 / 84, 8 rows 74 / 85, 16 rows 119 / 87, 32 rows
+// 109 / 91; 4096 x 65792, 1 row 26 / 82, 16 rows 73 / 84, 32 rows 79 / 86, 33 rows
+// 121 / 87; 1024 x 128256, 1 row 39 / 25 us. (s8: up to 64
+// rows have kernels of their own, which the launch takes before it asks here.)
+int gemm_g128_rows(int M, int N, int K, int kind) {
+    const bool s8 = kind == G_S8;
+    const int64_t tn = ((int64_t)N + 255) / 256;
     const int tall = s8 ? 128 : 96;
-    const int64_t t64 = (M + 63) / 64 * tn, tt = (M + tall - 1) / tall * tn;
-    if (t64 <= (s8 ? 192 : 256)) return 0;
-    auto cost = [](int64_t tiles, double one, double two) {
-        const int64_t n = (tiles + 255) / 256;
-        return (double)(n / 2) * two + (double)(n % 2) * one;
-    };
-    const double c64 = s8 ? cost(t64, 1.10, 1.45) : cost(t64, 1.75, 2.35);
-    const double ct = s8 ? cost(tt, 1.75, 2.45) : cost(tt, 2.2, 2.7);
+    const int64_t t64 = ((int64_t)M + 63) / 64 * tn;
+    const int64_t tt = ((int64_t)M + tall - 1) / tall * tn;
+    if (t64 <= (s8 ? 192 : 256) || (s8 && M <= 64)) return 0;
+    const double c64 = s8 ? group_us(t64, 1.10, 1.45) : group_us(t64, 1.75, 2.35);
+    const double ct = s8 ? group_us(tt, 1.75, 2.45) : group_us(tt, 2.2, 2.7);
+    if (!s8 && M <= 32) {
+        const int groups = K / 128;
+        const double us
+                = 5.0 + groups * std::min(c64, ct) * (kind == G_BF16 ? 1.1 : 1.0);
+        if (few_rows_us(M, N, groups) <= us) return 0;
+    }
     return c64 < ct ? 64 : tall;
 }
 #endif
 } // namespace qmm
+
+#if !defined(QMM_G128_PART)
+extern "C" int qmm_gemm_g128_rows(int src_dt, int64_t M, int64_t N, int64_t K) {
+    using namespace qmm;
+    if (M < 1 || N < 1 || K < 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX)
+        return 0;
+    if (src_dt != dt_s8 && src_dt != dt_f16 && src_dt != dt_bf16) return 0;
+    return gemm_g128_rows((int)M, (int)N, (int)K,
+            src_dt == dt_s8 ? G_S8 : src_dt == dt_f16 ? G_F16 : G_BF16);
+}
+#endif

@@ -876,7 +876,7 @@ void launch_gemm_w4f(const gemv_params_t &p, int shifts, int flags_m,
 bool gemm_w4f_wins(const gemv_params_t &p);
 void launch_gemm_g128_f16(const g128_params_t &p, int rows, hipStream_t stream);
 void launch_gemm_g128_bf16(const g128_params_t &p, int rows, hipStream_t stream);
-int gemm_g128_rows(int M, int N, bool s8);
+int gemm_g128_rows(int M, int N, int K, int kind);
 
 // Returns false when no kernel takes the problem (nothing is launched then).
 bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
@@ -939,10 +939,11 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
         // an absent zero-point buffer is never dereferenced past its first
         // byte: the weights stand in for it
         const uint8_t *zp = p.zps ? (const uint8_t *)p.zps : p.B;
-        // 4-bit weights at many rows: the kernel whose wave tile is up to 96 rows
-        // tall (direct 16-byte loads: rows on 16-byte boundaries, whole groups of
+        // 4-bit weights at many rows (few: where it is the faster one, over very
+        // wide weights): the kernel whose wave tile is up to 96 rows tall (direct 16-byte loads: rows on 16-byte boundaries, whole groups of
         // 128 k, 32-bit offsets inside a tile of rows)
-        const int g128_rows = gemm_g128_rows(p.M, p.N, false);
+        const int g128_rows
+                = gemm_g128_rows(p.M, p.N, p.K, p.act_f16 ? G_F16 : G_BF16);
         if (g128_rows && !p.w8 && p.K == Kpad && p.lda % 8 == 0 && p.lda < (1 << 23)
                 && ((uintptr_t)p.A & 15) == 0) {
             g128_params_t t;

@@ -267,6 +267,7 @@ struct w4a8_prep_t {
 };
 
 // ---- 4-bit weights with groups of 128 k, many rows (qmm_gemm_g128.hip) --------
+enum : int { G_S8 = 0, G_F16 = 1, G_BF16 = 2 }; // its activations
 struct g128_params_t {
     const uint8_t *A; // s8, f16 or bf16 rows, K-contiguous
     int64_t lda; // bytes

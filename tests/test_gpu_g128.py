@@ -11,6 +11,7 @@ import pytest
 import onednn_amd as dnnl
 import oracle as O
 import test_gpu_parity as parity
+from onednn_amd import _capi
 from qmm_harness import assert_bf16_within_1ulp, assert_bit_exact, assert_f32_close, dt
 from test_gpu_w4a8 import W4A8, dynamic_quant
 
@@ -102,16 +103,9 @@ W4_CASES = {
 }
 
 
-@pytest.mark.parametrize("name", sorted(W4_CASES))
-def test_16bit_activations(ctx, name):
-    eng, strm = ctx
-    print("[case] g128 %s" % name, flush=True)
-    kw = W4_CASES[name]
-    p = parity.decode_w4(seed=600 + len(name), **kw)
-    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
-    assert pd.impl_info_str() == parity.DECODE
+def check_16bit(p, M, N, got, name):
     want = p.run_oracle()
-    code, M, N = p.dst.dt, kw["M"], kw["N"]
+    code = p.dst.dt
     terms = parity.decode_term_scale(p).reshape(M, N)
     if code == dt.bf16:
         assert_bf16_within_1ulp(got, want, name, abs_slack=2e-5 * terms.reshape(-1))
@@ -120,3 +114,36 @@ def test_16bit_activations(ctx, name):
     # f32 sums in another order: 2e-5 of the summed magnitudes; an f16 result one step (2^-10) more
     bar = 2e-5 * terms + (np.abs(w) * 2.0 ** -10 if code == dt.f16 else 0)
     assert np.all(np.abs(g.astype(np.float64) - w) <= bar), name
+
+
+@pytest.mark.parametrize("name", sorted(W4_CASES))
+def test_16bit_activations(ctx, name):
+    eng, strm = ctx
+    print("[case] g128 %s" % name, flush=True)
+    kw = W4_CASES[name]
+    p = parity.decode_w4(seed=600 + len(name), **kw)
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == parity.DECODE
+    check_16bit(p, kw["M"], kw["N"], got, name)
+
+
+# One row of tiles over more than 65536 columns: the tiled kernel where it is the faster one, else the decode kernels.
+FEW_ROWS = {
+    "f16_1_row_decode": (dict(M=1, K=2048, N=65552, act_dt=dt.f16), 0),
+    "bf16_8_rows_decode": (dict(M=8, K=2048, N=65552), 0),
+    "f16_5_rows_tiled": (dict(M=5, K=128, N=65552, act_dt=dt.f16), 64),
+    "bf16_16_rows_tiled": (dict(M=16, K=256, N=65590, with_zp=False, wei_dt=dt.s4), 64),
+    "f16_33_rows_tiled": (dict(M=33, K=256, N=65544, act_dt=dt.f16), 64),
+}
+
+
+@pytest.mark.parametrize("name", sorted(FEW_ROWS))
+def test_few_rows_of_wide_weights(ctx, name):
+    eng, strm = ctx
+    print("[case] g128 few rows %s" % name, flush=True)
+    kw, tile = FEW_ROWS[name]
+    p = parity.decode_w4(seed=700 + len(name), **kw)
+    assert _capi.lib().qmm_gemm_g128_rows(p.src.dt, kw["M"], kw["N"], kw["K"]) == tile
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == parity.DECODE
+    check_16bit(p, kw["M"], kw["N"], got, name)
