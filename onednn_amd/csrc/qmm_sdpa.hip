@@ -919,7 +919,7 @@ sdpa_combine_kernel(const sdpa_params_t p, const int D) {
 struct sdpa_split_t {
     int nsplit, tps, pack;
 };
-sdpa_split_t decode_split(const sdpa_params_t &p) {
+sdpa_split_t decode_split(const sdpa_params_t &p, int64_t D) {
     const int64_t S = p.S, Qn = p.Qn;
     const bool causal = p.causal != 0;
     sdpa_split_t r;
@@ -933,8 +933,17 @@ sdpa_split_t decode_split(const sdpa_params_t &p) {
     const int64_t heads = (int64_t)p.B0 * p.B1 / r.pack;
     int64_t tiles = (S + SDPA_KT - 1) / SDPA_KT;
     if (causal) tiles = std::min<int64_t>(tiles, (Qn - 1) / SDPA_KT + 1);
-    // enough workgroups to fill the chip twice, at least one tile per wave
-    int64_t want = std::max<int64_t>(1, 512 / std::max<int64_t>(1, heads));
+    // Few tiles stay one range, however few workgroups that is: a second range costs
+    // the combining launch. How many that are depends on what a tile takes a wave
+    // (1 query, us, one range / several: head size 64, 256 keys 5.2 / 7.4, 512 keys
+    // 6.2 / 7.5; head size 128, 256 keys 7.7 / 8.5, s8 8.7 / 9.2, 384 keys 8.6 / 8.6,
+    // s8 10.0 / 9.2, bf16 queries over s8, 256 keys 11.0 / 10.6; head size 256, 256
+    // keys 13.2 / 12.0).
+    const bool unpacked = p.kv_dt != (p.bf ? dt_bf16 : dt_f16) && !p.fastq;
+    const int64_t w = unpacked ? 2 * D : D;
+    const int64_t alone = SDPA_WAVES * (w <= 64 ? 4 : w <= 128 ? 2 : 1);
+    // else enough workgroups to fill the chip twice, at least one tile per wave
+    int64_t want = tiles <= alone ? 1 : std::max<int64_t>(1, 512 / std::max<int64_t>(1, heads));
     int64_t tps = std::max<int64_t>(SDPA_WAVES, (tiles + want - 1) / want);
     tps = (tps + SDPA_WAVES - 1) / SDPA_WAVES * SDPA_WAVES;
     r.tps = (int)tps;
@@ -1110,9 +1119,9 @@ const char *qmm_sdpa_impl_name(const qmm_sdpa_desc_t *desc) {
 size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc) {
     sdpa_params_t p;
     if (!desc || !supported(*desc, &p) || p.Qn > 16) return 0;
-    const sdpa_split_t sp = decode_split(p);
-    if (sp.nsplit <= 1) return 0;
     const int64_t D = desc->q.dims[desc->q.ndims - 1];
+    const sdpa_split_t sp = decode_split(p, D);
+    if (sp.nsplit <= 1) return 0;
     return (size_t)p.B0 * p.B1 * sp.nsplit * p.Qn * (D + 2) * sizeof(float);
 }
 
@@ -1146,7 +1155,7 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
     const bool qn = p.kv_dt != desc->q.dt, mk = p.mask != nullptr;
     const bool bf = p.bf != 0;
     if (p.Qn <= 16) {
-        const sdpa_split_t sp = decode_split(p);
+        const sdpa_split_t sp = decode_split(p, D);
         p.nsplit = sp.nsplit;
         p.pack = sp.pack;
         p.tps = sp.tps;
