@@ -96,7 +96,8 @@ struct sdpa_params_t {
     int32_t nsplit, tps;
     int32_t fastq, bf; // f16 scales and 8-bit zero points: f16 dequantisation
     int32_t pack; // few queries: heads of one K / V head that share a workgroup
-    float *part; // [head][split][query][D + 2]: O (unnormalised), m, l
+    int32_t packs; // B1 / pack
+    float *part; // [head][split], part_pitch each: [query][D + 2]: O (unnormalised), m, l
 };
 
 // Lanes that differ only in their 16-lane row hold parts of one query. The two
@@ -507,6 +508,13 @@ sdpa_f16_kernel(const sdpa_params_t p) {
 }
 
 
+// Floats of one range's states of one head in the scratchpad (a query's: D
+// accumulators, maximum, sum), up to whole 128-byte lines: the states of other ranges
+// and heads are written by other XCDs.
+QMM_HD int part_pitch(int Qn, int D) {
+    return (Qn * (D + 2) + 31) / 32 * 32;
+}
+
 // ---- few queries (at most 16 per head: the decode step) ----------------------
 // Bound: HBM, one read of the cache; what it takes to get near is requests in
 // flight. One workgroup per (group of heads, key range); its four waves take the
@@ -549,8 +557,7 @@ sdpa_decode_kernel(const sdpa_params_t p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, c = lane >> 4;
     const int split = blockIdx.y;
-    const int packs = p.B1 / p.pack;
-    const int b1_0 = blockIdx.x % packs * p.pack, b0 = blockIdx.x / packs;
+    const int b1_0 = blockIdx.x % p.packs * p.pack, b0 = blockIdx.x / p.packs;
     const int kb0 = b0 / p.kv_div0, kb1 = b1_0 / p.kv_div1;
     // column r of the MFMAs: query q of head b1 (columns past the last repeat it)
     const int rows = p.pack * p.Qn, rc = min(r, rows - 1);
@@ -849,7 +856,7 @@ sdpa_decode_kernel(const sdpa_params_t p) {
         }
     } else {
         const int64_t head = (int64_t)b0 * p.B1 + b1;
-        float *out = p.part + ((head * p.nsplit + split) * p.Qn + q) * ST;
+        float *out = p.part + (head * p.nsplit + split) * part_pitch(p.Qn, D) + q * ST;
 #pragma unroll
         for (int d = 0; d < DVB; d++)
 #pragma unroll
@@ -869,18 +876,21 @@ sdpa_decode_kernel(const sdpa_params_t p) {
 
 // the splits' states of one (head, query) -> dst. The weights of the splits
 // are formed once in LDS; a thread then owns one d (two of 256) and adds the splits'
-// accumulators with independent loads.
+// accumulators with independent loads, eight at a time and what is left over at once.
+// The first head of every pack comes first, then the second, ...: with a multiple of 8
+// packs, as with so many heads of their own, a head's states lie in the L2 of the XCD
+// that reads them.
 constexpr int SDPA_MAX_SPLIT = 256;
 __global__ void __launch_bounds__(128)
 sdpa_combine_kernel(const sdpa_params_t p, const int D) {
     __shared__ float w_s[SDPA_MAX_SPLIT];
     __shared__ float red[2];
-    const int head = blockIdx.x, q = blockIdx.y, t = threadIdx.x;
-    const int b1 = head % p.B1, b0 = head / p.B1;
-    const int ST = D + 2;
-    // state of split s: row s * Qn + q of the head
-    const float *st = p.part + ((int64_t)head * p.nsplit * p.Qn + q) * ST;
-    const int64_t step = (int64_t)p.Qn * ST;
+    const int q = blockIdx.y, t = threadIdx.x;
+    const int b0 = blockIdx.x / p.packs;
+    const int b1 = blockIdx.x % p.packs * p.pack + blockIdx.z;
+    const int64_t head = (int64_t)b0 * p.B1 + b1;
+    const int step = part_pitch(p.Qn, D); // one split to the next
+    const float *st = p.part + head * p.nsplit * step + q * (D + 2);
     // every thread finds the maximum itself (at most 256 values from L2)
     float m_all = -INFINITY;
     for (int s1 = t; s1 < p.nsplit; s1 += 128)
@@ -906,9 +916,23 @@ sdpa_combine_kernel(const sdpa_params_t p, const int D) {
     const float l_all = red[0] + red[1];
     for (int d = t; d < D; d += 128) { // head sizes up to 256: two per thread
         float o = 0.f;
-#pragma unroll 8
-        for (int s1 = 0; s1 < p.nsplit; s1++)
-            o += w_s[s1] * st[s1 * step + d];
+        const float *x = st + d;
+        int s1 = 0;
+        for (; s1 + 8 <= p.nsplit; s1 += 8, x += 8 * step)
+#pragma unroll
+            for (int u = 0; u < 8; u++) o += w_s[s1 + u] * x[u * step];
+        const int left = p.nsplit - s1;
+        if (left > 0) { // (past the end: the last split again, not added)
+            float v[7], w[7];
+#pragma unroll
+            for (int u = 0; u < 7; u++) {
+                v[u] = x[min(u, left - 1) * step];
+                w[u] = w_s[s1 + min(u, left - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < 7; u++)
+                if (u < left) o += w[u] * v[u];
+        }
         p.dst[b0 * p.o.b0 + b1 * p.o.b1 + (int64_t)q * p.o.row + d]
                 = p.bf ? f32_to_bf16(o / l_all)
                        : __builtin_bit_cast(uint16_t, (_Float16)(o / l_all));
@@ -1122,7 +1146,7 @@ size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc) {
     const int64_t D = desc->q.dims[desc->q.ndims - 1];
     const sdpa_split_t sp = decode_split(p, D);
     if (sp.nsplit <= 1) return 0;
-    return (size_t)p.B0 * p.B1 * sp.nsplit * p.Qn * (D + 2) * sizeof(float);
+    return (size_t)p.B0 * p.B1 * sp.nsplit * part_pitch(p.Qn, (int)D) * sizeof(float);
 }
 
 int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
@@ -1158,10 +1182,11 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
         const sdpa_split_t sp = decode_split(p, D);
         p.nsplit = sp.nsplit;
         p.pack = sp.pack;
+        p.packs = p.B1 / p.pack;
         p.tps = sp.tps;
         p.part = (float *)args->scratch;
         if (p.nsplit > 1 && !p.part) return QMM_INVALID_ARGUMENTS;
-        const dim3 dgrid((unsigned)(p.B0 * (p.B1 / p.pack)), (unsigned)p.nsplit);
+        const dim3 dgrid((unsigned)(p.B0 * p.packs), (unsigned)p.nsplit);
         auto god = [&](auto kern) {
             hipLaunchKernelGGL(kern, dgrid, dim3(SDPA_WAVES * 64), 0,
                     (hipStream_t)hip_stream, p);
@@ -1204,8 +1229,8 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
         }
         if (p.nsplit > 1)
             hipLaunchKernelGGL(sdpa_combine_kernel,
-                    dim3((unsigned)(p.B0 * p.B1), (unsigned)p.Qn), dim3(128), 0,
-                    (hipStream_t)hip_stream, p, D);
+                    dim3((unsigned)(p.B0 * p.packs), (unsigned)p.Qn, (unsigned)p.pack),
+                    dim3(128), 0, (hipStream_t)hip_stream, p, D);
         return hipGetLastError() == hipSuccess ? QMM_OK : QMM_RUNTIME_ERROR;
     }
     const dim3 grid((unsigned)(p.B0 * p.B1),

@@ -60,3 +60,21 @@ def test_heads_of_a_group_share_a_workgroup(ctx, rep, Qn, S, D, mkind, quant, qd
     bad, total, worst = reference_rule(f16_to_f64(got, qdt), gold, 0.001466 if qdt == dt.f16 else 0.0079)
     print("[sdpa grouped] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
     assert bad <= total * 0.0006
+
+
+@pytest.mark.parametrize("ranges", [3, 4, 5, 6, 7, 8, 9, 15, 16, 17, 23])
+@pytest.mark.parametrize("H,KH,Qn", [(2, 2, 1), (8, 2, 2), (15, 3, 1)], ids=str)
+def test_every_count_of_ranges_is_combined(ctx, ranges, H, KH, Qn):
+    """128 keys a range at these head counts; the combining kernel adds eight ranges at a time, then the rest."""
+    print("[case] sdpa combine ranges=%d H=%d KH=%d Qn=%d" % (ranges, H, KH, Qn), flush=True)
+    MB, D, S = 2, 128, 128 * ranges - 5
+    r = np.random.default_rng(ranges * 10 + H)
+    q = f16(r.standard_normal((MB, H, Qn, D)))
+    k, v = f16(r.standard_normal((MB, KH, S, D))), f16(r.standard_normal((MB, KH, S, D)))
+    scale = 1.0 / np.sqrt(D)
+    got = run_sdpa(ctx, q, k, v, scale=scale, kv_heads=KH)
+    s_eff = float(f16_to_f64(f16(np.array([scale])))[0])
+    gold = attention64(f16_to_f64(q), np.swapaxes(f16_to_f64(k), -1, -2), f16_to_f64(v), s_eff, None, False, H // KH)
+    bad, total, worst = reference_rule(f16_to_f64(got), gold, 0.001466)
+    print("[sdpa combine] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
+    assert bad <= total * 0.0006

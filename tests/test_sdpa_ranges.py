@@ -44,3 +44,10 @@ def test_an_8_bit_cache_without_packed_dequantization_is_cut_earlier():
     assert scratch_bytes(1, 32, 8, 1, 257, 64, dt.bf16, dt.s8) > 0
     assert scratch_bytes(1, 32, 8, 1, 129, 128, dt.bf16, dt.s8) > 0
     assert scratch_bytes(1, 32, 8, 1, 256, 128, dt.f16, dt.s8) == 0
+
+
+@pytest.mark.parametrize("D,one,three", [(64, 384, 896), (96, 512, 1280), (128, 640, 1664), (256, 1152, 3200)])
+def test_states_lie_on_lines_of_their_own(D, one, three):
+    # 20 tiles, five ranges; per query D accumulators, maximum and sum; a range's, up to whole 128-byte lines
+    assert scratch_bytes(1, 1, 1, 1, 640, D) == 5 * one
+    assert scratch_bytes(2, 4, 2, 3, 640, D) == 2 * 4 * 5 * three
