@@ -947,14 +947,6 @@ sdpa_split_t decode_split(const sdpa_params_t &p, int64_t D) {
     const int64_t S = p.S, Qn = p.Qn;
     const bool causal = p.causal != 0;
     sdpa_split_t r;
-    // the most heads of a group whose queries fit the MFMA's 16 columns
-    r.pack = 1;
-    for (int h = p.kv_div1; h > 1; h--)
-        if (p.kv_div1 % h == 0 && h * Qn <= 16) {
-            r.pack = h;
-            break;
-        }
-    const int64_t heads = (int64_t)p.B0 * p.B1 / r.pack;
     int64_t tiles = (S + SDPA_KT - 1) / SDPA_KT;
     if (causal) tiles = std::min<int64_t>(tiles, (Qn - 1) / SDPA_KT + 1);
     // Few tiles stay one range, however few workgroups that is: a second range costs
@@ -966,7 +958,21 @@ sdpa_split_t decode_split(const sdpa_params_t &p, int64_t D) {
     const bool unpacked = p.kv_dt != (p.bf ? dt_bf16 : dt_f16) && !p.fastq;
     const int64_t w = unpacked ? 2 * D : D;
     const int64_t alone = SDPA_WAVES * (w <= 64 ? 4 : w <= 128 ? 2 : 1);
-    // else enough workgroups to fill the chip twice, at least one tile per wave
+    // The most heads of a group whose queries fit the MFMA's 16 columns. Up to 2048 keys
+    // in several ranges, no more than leave 8 packs: a head's states then stay on one
+    // XCD, which is worth more than reading a short cache once (1 x 32 heads over 4 K /
+    // V heads, packs of 4 / 8: 512 keys of 128 8.0 / 8.3 us, 2048 keys of 256 11.7 /
+    // 12.3, 8192 keys of 128 11.8 / 10.1).
+    const int64_t all = (int64_t)p.B0 * p.B1;
+    const int64_t packs = tiles > alone && tiles <= 64 && all >= 8 ? 8 : 1;
+    r.pack = 1;
+    for (int h = p.kv_div1; h > 1; h--)
+        if (p.kv_div1 % h == 0 && h * Qn <= 16 && all / h >= packs) {
+            r.pack = h;
+            break;
+        }
+    const int64_t heads = all / r.pack;
+    // enough workgroups to fill the chip twice, at least one tile per wave
     int64_t want = tiles <= alone ? 1 : std::max<int64_t>(1, 512 / std::max<int64_t>(1, heads));
     int64_t tps = std::max<int64_t>(SDPA_WAVES, (tiles + want - 1) / want);
     tps = (tps + SDPA_WAVES - 1) / SDPA_WAVES * SDPA_WAVES;

@@ -78,3 +78,21 @@ def test_every_count_of_ranges_is_combined(ctx, ranges, H, KH, Qn):
     bad, total, worst = reference_rule(f16_to_f64(got), gold, 0.001466)
     print("[sdpa combine] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
     assert bad <= total * 0.0006
+
+
+@pytest.mark.parametrize("H,KH,Qn", [(32, 4, 1), (24, 2, 1), (12, 1, 2), (14, 2, 1), (4, 1, 3)], ids=str)
+@pytest.mark.parametrize("S", [256, 257, 2048, 2049])
+def test_heads_in_a_pack_by_the_number_of_keys(ctx, H, KH, Qn, S):
+    """Fewer heads share a workgroup up to 2048 keys in several ranges (more than 256 keys here) than past either end."""
+    print("[case] sdpa packs H=%d KH=%d Qn=%d S=%d" % (H, KH, Qn, S), flush=True)
+    D = 128
+    r = np.random.default_rng(H * 100 + S)
+    q = f16(r.standard_normal((1, H, Qn, D)))
+    k, v = f16(r.standard_normal((1, KH, S, D))), f16(r.standard_normal((1, KH, S, D)))
+    scale = 1.0 / np.sqrt(D)
+    got = run_sdpa(ctx, q, k, v, scale=scale, kv_heads=KH)
+    s_eff = float(f16_to_f64(f16(np.array([scale])))[0])
+    gold = attention64(f16_to_f64(q), np.swapaxes(f16_to_f64(k), -1, -2), f16_to_f64(v), s_eff, None, False, H // KH)
+    bad, total, worst = reference_rule(f16_to_f64(got), gold, 0.001466)
+    print("[sdpa packs] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
+    assert bad <= total * 0.0006
