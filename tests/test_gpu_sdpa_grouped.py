@@ -96,3 +96,28 @@ def test_heads_in_a_pack_by_the_number_of_keys(ctx, H, KH, Qn, S):
     bad, total, worst = reference_rule(f16_to_f64(got), gold, 0.001466)
     print("[sdpa packs] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
     assert bad <= total * 0.0006
+
+
+@pytest.mark.parametrize("Qn,H", [(1, 4), (1, 8), (64, 4)], ids=str)
+def test_u8_cache_with_negative_zero_points(ctx, Qn, H):
+    """Zero points of the other sign than the cache's type: 1024 + z lies below the range of the bytes' own exponent, and
+    every difference is still an exact f16 number (the whole range -128 ... 127 in turn)."""
+    print("[case] sdpa u8 cache s8 zero points Qn=%d H=%d" % (Qn, H), flush=True)
+    KH, S, D = 4, 260, 128
+    r = np.random.default_rng(Qn + H)
+    q = f16(r.standard_normal((1, H, Qn, D)))
+    zp = ((np.arange(KH * S).reshape(KH, S) * 5) % 256 - 128).astype(np.int8)
+    side = []
+    for groups in ((D, 1), (1, D)):
+        # bytes around their zero point where the type holds them, so that the scores stay of order one
+        x = np.clip(zp[..., None].astype(np.int64) + r.integers(-60, 61, (KH, S, D)), 0, 255).astype(np.uint8)[None]
+        sc = f16(r.uniform(0.005, 0.02, (KH, S)))
+        x64 = f16_to_f64(f16((x - zp[None, ..., None].astype(np.float64)) * f16_to_f64(sc)[None, ..., None]))
+        side.append((x, x64, (0b1110, groups, dt.f16, sc, dt.s8, zp)))
+    scale = 1.0 / np.sqrt(D)
+    got = run_sdpa(ctx, q, side[0][0], side[1][0], scale=scale, kv_heads=KH, kv_dt=dt.u8, k_q=side[0][2], v_q=side[1][2])
+    s_eff = float(f16_to_f64(f16(np.array([scale])))[0])
+    gold = attention64(f16_to_f64(q), np.swapaxes(side[0][1], -1, -2), side[1][1], s_eff, None, False, H // KH)
+    bad, total, worst = reference_rule(f16_to_f64(got), gold, 0.001466)
+    print("[sdpa u8 zp] %d of %d outside the threshold, max diff %.2e" % (bad, total, worst))
+    assert bad <= total * 0.0006
