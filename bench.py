@@ -1049,7 +1049,7 @@ def bench_w4a8(A, memory, dt, tag, T, eng, strm, hs, hiprt):
                           "algorithmic_bytes": nbytes, "GBps": round(nbytes / (ms * 1e-3) / 1e9, 1),
                           "frac_of_hbm_peak": round(nbytes / (ms * 1e-3) / 1e9 / PEAK_HBM, 4),
                           "impl": pd.impl_info_str(),
-                          "includes": "scale pre-pass%s + GEMM" % (" with weights column sums" if szp else "")}
+                          "includes": "scale pre-pass with weights column sums + GEMM" if szp else "one launch"}
     return res
 
 

@@ -2,17 +2,22 @@
 // for many rows: hip:gfx950:decode_w4 (f16 / bf16 activations, f32 sums) and
 // hip:gfx950:mfma_w4a8 (s8 activations, s32 sums inside a group of 128 k). The
 // arithmetic is that of qmm_gemm_w4f.hip / qmm_gemm_w4a8.hip, operation for
-// operation; what differs is the shape of the work.
+// operation but for one: bf16 takes the offset off the group's sum in one fma, where
+// qmm_gemm_w4f.hip rounds the product first. What differs is the shape of the work.
 //
 // Both problems are bound by instruction issue: next to its MFMAs a wave has to
 // expand the nibbles of its columns and to fold a finished group into f32
 // accumulators, and the vector ALU shares its issue slots with the matrix
-// cores. So the wave tile is as tall as 256 registers allow (128 rows for s8, 96
-// for f16 / bf16, whose expanded weights take twice the registers; 64 for smaller
-// problems), which is two waves per SIMD:
+// cores. So the wave tile is as tall as 256 registers allow with two waves per SIMD:
+// 128 rows for s8, 96 for f16 / bf16, whose expanded weights take twice the
+// registers; or 64, where the taller one leaves more of the last round empty. Three
+// forms stand one step over: s8 with 128 rows spills 4 registers (20 bytes of scratch
+// a lane, from the second pass over the groups that huge row scales need; without it
+// 247 registers), bf16 with 96 rows 1 (s4 weights 4).
 //   * four waves side by side own 16 FM rows x 256 columns, a wave all the rows
 //     of its 64 columns: a nibble is expanded once for up to 128 rows, where the
-//     other kernels expand it once for 64;
+//     other kernels expand it once for 64 (the 64-row form has none of this gain: its
+//     comes from the next point and from two workgroups on a CU);
 //   * the group is the unit of the loop: a 16 x 16 fragment of the result runs
 //     its MFMAs over the whole group (4 of 16 x 16 x 32 f16, 2 of 16 x 16 x 64
 //     i8) in four registers and is folded into the f32 accumulators at once, so
@@ -34,10 +39,12 @@
 // wave's packed weights through a private piece of LDS that is refilled as soon
 // as its nibbles are in registers. One barrier per group.
 //
-// Measured on 4096 x 14336 weights, launches back to back: s8 x s4, 2176 rows 229 ->
-// 161 us, 4096 rows 393 -> 281 us (1.71 POP/s); f16 x u4, 1000 rows 230 -> 157 us,
-// 2048 rows 402 -> 256 us (0.94 PFLOP/s); bf16 x u4, 1000 rows 256 -> 175 us. With
-// parts switched off (1000 rows, s8, 88 us): no MFMAs 66, no fold 64, neither 43 us
+// Measured on 4096 x 14336 weights, launches back to back, the kernels named above /
+// this one: s8 x s4, 1000 rows 121 / 87 us, 2176 rows 230 / 163 us, 4096 rows 407 / 284
+// us (1.69 POP/s); f16 x u4, 1000 rows (64-row tiles) 230 / 158 us, 2048 rows 402 / 259
+// us (0.93 PFLOP/s); bf16 x u4, 1000 rows 256 / 178 us. The second pass of the s8 form
+// costs 3 % where it is not taken (2176 rows 155 us without). With parts switched off
+// (1000 rows, s8, without that pass, 88 us): no MFMAs 66, no fold 64, neither 43 us
 // (prologue, expanding, LDS reads, epilogue), no loads inside the loop 88: the parts
 // add up, whether the fold stands behind a row block's MFMAs or between them.
 #include <algorithm>
@@ -556,9 +563,14 @@ static double few_rows_us(int M, int N, int groups) {
 }
 
 // Rows of the tile for an M x N x K problem, 0: the other kernels are as fast.
-// Measured per group of 128 k (us), one / two workgroups on a CU:
+// us per group of 128 k, one / two workgroups on a CU, prologue and epilogue of a
+// 4096-k problem shared out over its groups:
 //   s8:   64 rows 1.10 / 1.45, 128 rows 1.75 / 2.45
 //   f16:  64 rows 1.75 / 2.35,  96 rows 2.2  / 2.7 (bf16 a tenth more on each)
+// Over 530 problems (100 ... 4096 rows, 4096 ... 28672 columns, 1024 and 4096 k) the
+// tile chosen with these is 0.9 % (s8), 0.2 % (f16), 0.5 % (bf16) behind the better one
+// on average, 15 % (s8, 257 rows x 28672 columns), 3 % and 5 % at most. Costs from the
+// slope over K alone (s8 0.84 / 1.28 and 1.27 / 2.26) choose worse (s8: 4.6 %).
 // The gates: the kernel of qmm_gemm_w4f.hip takes 1.85 us for a 64 x 256 block and
 // runs one on a CU (4096 x 14336 weights: 256 rows, 224 blocks, 62 against 63 us;
 // 512 rows, 448 blocks, 117 against 82 us); that of qmm_gemm_w4a8.hip was faster by

@@ -146,8 +146,9 @@ QMM_D float ld_zp(int dt, const void *p, int64_t i) {
 // significant bits, so rounding the f16 product is the same single rounding as
 // f16(f32 product): the values of the reference's dequantizing reorder, at 1.5
 // instructions per element. `raw`: bytes with the sign bit already flipped for
-// s8; sc: the scale twice; off: 1024 + zero point (+ 128 for s8), an integer within
-// [1024, 2047], twice.
+// s8; sc: the scale twice; off: 1024 + zero point (+ 128 for s8), twice: an integer
+// within [896, 1407], so that off and every difference (at most 383 away from 0) are
+// f16 numbers.
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 QMM_D h2 twice(float v) {
     return h2 {(_Float16)v, (_Float16)v};
@@ -534,10 +535,12 @@ QMM_HD int part_pitch(int Qn, int D) {
 //   * QUANT = 1: the lane that fetched a key's scale and zero point writes them to
 //     LDS as the packed f16 operands of the dequantization, one 8-byte read for
 //     each use; keys past the end are looked for in the last tile only.
-// 1 query, head size 128, launches back to back with the combining kernel, before /
-// after (us): 32 heads x 8191 keys, s8 29.2 / 24.0, f16 29.6 / 28.7; x 32768 keys, s8
-// 79.6 / 55.4 (4.9 TB/s), f16 100.6 / 98.4; 8 K / V heads, bf16, 8191 keys 29.8 / 15.6,
-// 32768 86.1 / 30.8; 4 K / V heads, s8, 32768 75.7 / 22.4.
+// 1 query, head size 128, launches back to back with the combining kernel, one head to
+// a workgroup and one tile ahead / this kernel (us): 32 heads x 8191 keys, s8 28.2 /
+// 23.4, f16 29.2 / 28.4; x 32768 keys, s8 79.8 / 55.0 (5.0 TB/s), f16 102.1 / 100.3;
+// 8 K / V heads, bf16, 8191 keys 30.5 / 14.8, 32768 85.9 / 29.9; 4 K / V heads, s8,
+// 32768 75.2 / 20.1. 1024 keys, 32 heads over 8 K / V heads, f16: 1 sequence 8.0 / 7.9,
+// 16 42.3 / 17.6, 64 156 / 43.
 template <int DC, int QUANT, bool MASKED, bool BF>
 __global__ void __launch_bounds__(SDPA_WAVES * 64, DC > 4 ? 1 : 2)
 sdpa_decode_kernel(const sdpa_params_t p) {
@@ -577,7 +580,7 @@ sdpa_decode_kernel(const sdpa_params_t p) {
     uint4 kr[SLOTS][2][DC], vr[SLOTS][D / 16];
     uint32_t qsz[SLOTS][2]; // lanes 0..31: scale, zero point of K's key; 32..63: V's
     const bool up = lane >= 32;
-    // (absent buffers: the cache stands in, the value is replaced below)
+    // (absent buffers: the queries stand in, the value is replaced below)
     const void *const sp = up ? p.v_scale : p.k_scale, *const zp = up ? p.v_zp : p.k_zp;
     const uint16_t *const sp1 = sp ? (const uint16_t *)sp + qz_base : nullptr;
     const uint8_t *const zp1 = zp ? (const uint8_t *)zp + qz_base : nullptr;
@@ -879,7 +882,9 @@ sdpa_decode_kernel(const sdpa_params_t p) {
 // accumulators with independent loads, eight at a time and what is left over at once.
 // The first head of every pack comes first, then the second, ...: with a multiple of 8
 // packs, as with so many heads of their own, a head's states lie in the L2 of the XCD
-// that reads them.
+// that reads them. Bound: latency. 768 keys of 128, six ranges, 32 heads over 8 K / V
+// heads, both launches 7.9 us; with the heads in their own order 8.8, the six ranges
+// added one after the other 8.7, the states packed without gaps 8.4.
 constexpr int SDPA_MAX_SPLIT = 256;
 __global__ void __launch_bounds__(128)
 sdpa_combine_kernel(const sdpa_params_t p, const int D) {
