@@ -955,13 +955,16 @@ sdpa_split_t decode_split(const sdpa_params_t &p, int64_t D) {
     int64_t tiles = (S + SDPA_KT - 1) / SDPA_KT;
     if (causal) tiles = std::min<int64_t>(tiles, (Qn - 1) / SDPA_KT + 1);
     // Few tiles stay one range, however few workgroups that is: a second range costs
-    // the combining launch. How many that are depends on what a tile takes a wave
-    // (1 query, us, one range / several: head size 64, 256 keys 5.2 / 7.4, 512 keys
-    // 6.2 / 7.5; head size 128, 256 keys 7.7 / 8.5, s8 8.7 / 9.2, 384 keys 8.6 / 8.6,
-    // s8 10.0 / 9.2, bf16 queries over s8, 256 keys 11.0 / 10.6; head size 256, 256
-    // keys 13.2 / 12.0).
+    // the combining launch. How many that are depends on what a tile takes a wave; a
+    // cache without packed dequantization counts as a head size 64 larger. 1 query, 32
+    // heads over 8 K / V heads, us, one range / several: head size 64, 256 keys 5.2 /
+    // 6.5, 512 keys 6.2 / 6.5; head size 128, 256 keys 7.7 / 7.8, s8 8.6 / 8.3, 384
+    // keys 8.6 / 7.9, bf16 over s8, 256 keys 10.8 / 9.5; bf16 over s8 of 32, 256 keys
+    // 5.1 / 6.5, 512 keys 7.1 / 6.5; head size 256, 256 keys 13.5 / 11.3. With more
+    // workgroups one range is better for longer (8 x 32 heads, 256 keys of 128 8.4 /
+    // 10.5, 384 keys 12.2 / 14.9).
     const bool unpacked = p.kv_dt != (p.bf ? dt_bf16 : dt_f16) && !p.fastq;
-    const int64_t w = unpacked ? 2 * D : D;
+    const int64_t w = unpacked ? D + 64 : D;
     const int64_t alone = SDPA_WAVES * (w <= 64 ? 4 : w <= 128 ? 2 : 1);
     // The most heads of a group whose queries fit the MFMA's 16 columns. Up to 2048 keys
     // in several ranges, no more than leave 8 packs: a head's states then stay on one

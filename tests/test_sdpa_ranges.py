@@ -42,6 +42,8 @@ def test_few_keys_are_one_range(batch, heads, kv_heads, D, keys):
 def test_an_8_bit_cache_without_packed_dequantization_is_cut_earlier():
     assert scratch_bytes(1, 32, 8, 1, 256, 64, dt.bf16, dt.s8) == 0
     assert scratch_bytes(1, 32, 8, 1, 257, 64, dt.bf16, dt.s8) > 0
+    assert scratch_bytes(1, 32, 8, 1, 256, 32, dt.bf16, dt.s8) == 0
+    assert scratch_bytes(1, 32, 8, 1, 512, 32, dt.bf16, dt.s8) > 0
     assert scratch_bytes(1, 32, 8, 1, 129, 128, dt.bf16, dt.s8) > 0
     assert scratch_bytes(1, 32, 8, 1, 256, 128, dt.f16, dt.s8) == 0
 
