@@ -1,0 +1,93 @@
+"""The many-queries attention kernel (two groups of waves over the keys, 128 queries a workgroup and 64 keys a tile)
+at the sizes where its tiles end, against float64 attention under the reference test's rule."""
+import numpy as np
+import pytest
+
+import onednn_amd as dnnl
+from onednn_amd import memory
+from qmm_harness import T, dt
+from test_gpu_sdpa import attention64, ctx, f16, f16_to_f64, reference_rule, run_sdpa, say  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+THR = {dt.f16: 0.001466, dt.bf16: 0.0079}
+
+
+def check(got, q, k, v, qdt, scale, causal, rep):
+    gold = attention64(f16_to_f64(q, qdt), np.swapaxes(f16_to_f64(k, qdt), -1, -2), f16_to_f64(v, qdt), scale, None, causal,
+                       rep)
+    bad, total, worst = reference_rule(f16_to_f64(got, qdt), gold, THR[qdt])
+    print("[sdpa prefill] %d of %d outside, max diff %.2e" % (bad, total, worst))
+    assert bad <= total * 0.0006
+
+
+CASES = [
+    # heads, kv heads, queries, keys, D, causal: one tile and less; one row past the 32 queries of a wave and the 128
+    # of a workgroup; 32 / 64 / 128 keys and one more or less; fewer keys than queries and more
+    (2, 2, 17, 1, 64, False), (2, 1, 31, 31, 128, True), (3, 3, 33, 64, 64, True), (2, 2, 32, 65, 128, False),
+    (1, 1, 128, 127, 128, True), (4, 2, 129, 129, 64, True), (2, 2, 129, 400, 128, False), (2, 2, 300, 63, 128, True),
+    (2, 2, 65, 192, 64, False), (2, 2, 257, 513, 64, True), (1, 1, 1100, 1100, 128, True), (2, 2, 600, 2305, 64, False),
+    # more query tiles than workgroups: two rounds, the second one backwards; a third, partial one
+    (40, 8, 1000, 1000, 64, True), (40, 40, 1000, 130, 128, False), (100, 4, 700, 70, 64, True),
+]
+
+
+@pytest.mark.parametrize("qdt", [dt.f16, dt.bf16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_ends_of_tiles(ctx, case, qdt):  # noqa: F811
+    H, KV, Qn, S, D, causal = case
+    say("sdpa prefill %s %r" % (qdt, case))
+    r = np.random.default_rng(Qn * 3 + S)
+    q = f16(r.standard_normal((1, H, Qn, D)), qdt)
+    k, v = f16(r.standard_normal((1, KV, S, D)), qdt), f16(r.standard_normal((1, KV, S, D)), qdt)
+    got = run_sdpa(ctx, q, k, v, scale=0.125, causal=causal, kv_heads=KV, qdt=qdt)
+    check(got, q, k, v, qdt, 0.125, causal, H // KV)
+
+
+@pytest.mark.parametrize("scale", [-0.125, 4.0], ids=str)
+def test_scales_that_are_not_the_usual(ctx, scale):  # noqa: F811
+    """A negative scale (the maximum of the raw products is not that of the scores); scores far apart, so that the
+    running maximum grows late and the probabilities before it vanish."""
+    H, Qn, S, D = 2, 160, 4200, 64
+    say("sdpa prefill scale %g" % scale)
+    r = np.random.default_rng(3)
+    q = f16(r.standard_normal((1, H, Qn, D)))
+    k = r.standard_normal((1, H, S, D))
+    k *= np.linspace(0.05, 1.0, S)[:, None]
+    k, v = f16(k), f16(r.standard_normal((1, H, S, D)))
+    got = run_sdpa(ctx, q, k, v, scale=scale)
+    check(got, q, k, v, dt.f16, scale, False, 1)
+
+
+def test_rows_of_all_heads_side_by_side(ctx):  # noqa: F811
+    """Q, K, V and dst as [token][head][D] buffers."""
+    eng, strm = ctx
+    H, Qn, S, D = 3, 150, 140, 128
+    say("sdpa prefill interleaved heads")
+    r = np.random.default_rng(9)
+    q, k, v = (f16(r.standard_normal((1, n, H, D))) for n in (Qn, S, S))
+    q_md = memory.desc([1, H, Qn, D], dt.f16, T("acbd"))
+    kt_md = memory.desc([1, H, D, S], dt.f16, T("adbc"))
+    v_md = memory.desc([1, H, S, D], dt.f16, T("acbd"))
+    out = memory(q_md, eng)
+    pd = dnnl.sdpa.primitive_desc(eng, q_md, kt_md, v_md, None, dt.undef, q_md, False, 0, True)
+    dnnl.sdpa(pd).execute(strm, {dnnl.DNNL_ARG_QUERIES: memory(q_md, eng).write(q), dnnl.DNNL_ARG_KEYS: memory(kt_md, eng).write(k),
+                                 dnnl.DNNL_ARG_VALUES: memory(v_md, eng).write(v), dnnl.DNNL_ARG_DST: out})
+    strm.wait()
+    got = np.swapaxes(out.read(np.uint16, (1, Qn, H, D)), 1, 2)
+    q, k, v = (np.swapaxes(x, 1, 2) for x in (q, k, v))
+    check(got, q, k, v, dt.f16, 1.0, True, 1)
+
+
+def test_infinite_values_stay_with_the_queries_that_see_them(ctx):  # noqa: F811
+    """An infinite value at the last key, not a multiple of anything: queries that cannot see the key in a tile of
+    their own stay finite, those that do are infinite, and none is NaN through the keys past the end."""
+    H, Qn, S, D = 2, 200, 101, 64
+    say("sdpa prefill infinite value")
+    r = np.random.default_rng(11)
+    q, k, v = (f16(r.standard_normal((1, H, n, D))) for n in (Qn, S, S))
+    v[:, :, S - 1, 0] = 0x7C00
+    got = f16_to_f64(run_sdpa(ctx, q, k, v, scale=0.125))
+    assert np.isposinf(got[..., 0]).all() and np.isfinite(got[..., 1:]).all()
+    got = f16_to_f64(run_sdpa(ctx, q, k, v, scale=0.125, causal=True))
+    assert np.isposinf(got[:, :, S - 1:, 0]).all() and np.isfinite(got[..., 1:]).all()
+    assert np.isfinite(got[:, :, :64]).all()  # whole tiles of 64 keys
