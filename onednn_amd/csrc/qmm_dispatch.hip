@@ -29,7 +29,8 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream);
 void launch_quantize_rows(const quant_rows_params_t &p, hipStream_t stream);
 void launch_quantize_transpose(const quant_tr_params_t &p, hipStream_t stream);
 void launch_w4a8_prep(const w4a8_prep_t &p, hipStream_t stream);
-void launch_gemv_b8(const gemm_params_t &p, hipStream_t stream);
+void launch_gemv_b8(const gemm_params_t &p, bool f8, hipStream_t stream);
+bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256);
 void launch_gemm_f16(const gemm16_params_t &p, hipStream_t stream);
 void launch_rowsum_b8(const void *src, int32_t *dst, int64_t batch, int64_t M,
         int64_t K, int64_t lda, int64_t a_sb, bool a_is_u8, const void *src_zp,
@@ -1122,9 +1123,13 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
         g.batch = (int32_t)P.batch;
         g.kb32 = (int32_t)geom.kb32;
         g.nb32 = (int32_t)geom.nb32;
-        // at most 64 rows of one matrix: the streaming kernel (it forms the
+        // few rows of one matrix, or few results: the streaming kernel (it forms the
         // row sums a weights zero point needs itself)
-        if (!f8 && P.M <= 64 && P.batch == 1 && gemm_variant == 0) {
+        if (P.batch == 1 && gemm_variant == 0 && (!f8 || P.K % 64 == 0)
+                && ((!f8 && P.M <= 64)
+                        || (plan->b8x_variant == 1 && !plan->measure
+                                && gemv_b8_takes(P.M, P.N, P.K, f8,
+                                        gemm_b8_uses_tile256(g, f8, 0))))) {
             if (b8_needs_rowsum(D)) {
                 const qmm_quant_t &wz = D.zps[QMM_WEI];
                 g.wei_zp = wz.set ? args->zps[QMM_WEI] : nullptr;
@@ -1132,7 +1137,7 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
                 g.wei_zp_sn = wz.set && (wz.mask & (1 << (nd - 1))) ? 1 : 0;
                 g.w_off = D.wei.dt == dt_u8 ? 128 : 0;
             }
-            launch_gemv_b8(g, stream);
+            launch_gemv_b8(g, f8, stream);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(e, "kernel launch");
             return QMM_OK;
