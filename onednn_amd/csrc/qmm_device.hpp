@@ -796,6 +796,134 @@ QMM_D void epilogue_fast4(const epilogue_t &ep, float (&d)[4], bool has_ss,
     }
 }
 
+// Rows m_first ... + nv - 1 of a staged tile through an EP_FAST_* shape (no bias, no dst
+// scale or zero point) where the straight-line loops do not apply: rows or columns end
+// inside the tile, or rows do not start on a vector's boundary. A wave visits RPI rows
+// at a time (lane: row lrow of them, columns n ... n + nvalid - 1), NIT times; what a
+// post-op reads from memory is requested BATCH visits ahead of the stores, whole
+// vectors at any address: one row at a time is a trip to memory per row (16 heads x
+// 1361 x 1361 scores with a mask 141 -> 68 us).
+// staged(row, d, ss): the four results and the row's source scale. PACK: the wave
+// flushes f32 denormals, bf16 by v_cvt_pk_bf16_f32. Operation for operation
+// epilogue_fast4().
+template <int BATCH, int NIT, int RPI, bool PACK, typename F>
+QMM_D void epilogue_fast_rows(const epilogue_t &ep, bool has_ss, bool has_ws,
+        const float (&ws)[4], int64_t b, int64_t m_first, int nv, int lrow, int64_t n,
+        int nvalid, F staged) {
+    typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+    typedef unsigned v4u_any __attribute__((ext_vector_type(4), aligned(4)));
+    typedef unsigned v2u_any __attribute__((ext_vector_type(2), aligned(2)));
+    const int fast = ep.fast;
+    const bool bf = ep.dst.dt == dt_bf16;
+    const bool f32 = fast == EP_FAST_ADD || !bf; // the second operand's type
+    if (nvalid <= 0) return;
+#pragma unroll 1
+    for (int it0 = 0; it0 < NIT; it0 += BATCH) {
+        if (it0 * RPI >= nv) break;
+        // the bits only: nothing here needs a load's result, and no load is behind a
+        // choice of its own (a conversion or a join would wait for every load)
+        v4u_any y[BATCH];
+        if (fast == EP_FAST_ADD || fast == EP_FAST_SUM) {
+            const uint8_t *const base = fast == EP_FAST_ADD
+                    ? (const uint8_t *)ep.po[0].t.ptr + (b * ep.po[0].t.sb + n) * 4
+                    : (const uint8_t *)ep.dst.ptr + (b * ep.dst.sb + n) * (f32 ? 4 : 2);
+            const int64_t pitch = fast == EP_FAST_ADD ? ep.po[0].t.sm * 4
+                                                      : ep.dst.sm * (f32 ? 4 : 2);
+            const uint8_t *q[BATCH];
+#pragma unroll
+            for (int k = 0; k < BATCH; k++)
+                q[k] = base + (m_first + min((it0 + k) * RPI + lrow, nv - 1)) * pitch;
+            if (nvalid == 4 && f32) {
+#pragma unroll
+                for (int k = 0; k < BATCH; k++) y[k] = *(const v4u_any *)q[k];
+            } else if (nvalid == 4) {
+#pragma unroll
+                for (int k = 0; k < BATCH; k++) {
+                    const v2u_any v = *(const v2u_any *)q[k];
+                    y[k][0] = v[0], y[k][1] = v[1];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+                    if (i < nvalid) {
+#pragma unroll
+                        for (int k = 0; k < BATCH; k++)
+                            y[k][i] = f32 ? ((const uint32_t *)q[k])[i]
+                                          : ((const uint16_t *)q[k])[i];
+                    }
+            }
+        }
+        auto operand = [&](const v4u_any &v, int i) {
+            if (f32) return u2f(v[i]);
+            if (nvalid == 4)
+                return u2f(i & 1 ? v[i >> 1] & 0xffff0000u : v[i >> 1] << 16);
+            return u2f(v[i] << 16);
+        };
+#pragma unroll
+        for (int k = 0; k < BATCH; k++) {
+            const int row = (it0 + k) * RPI + lrow;
+            if (row >= nv) continue;
+            float d[4], ss;
+            staged(row, d, ss);
+            if (has_ss) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] *= ss;
+            }
+            if (has_ws) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] *= ws[i];
+            }
+            if (fast == EP_FAST_RELU) {
+                const float alpha = ep.po[0].alpha;
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] = d[i] > 0 ? d[i] : d[i] * alpha;
+            } else if (fast == EP_FAST_SWISH) {
+                const float na = -ep.po[0].alpha * 1.44269504088896340736f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float e = __builtin_amdgcn_exp2f(d[i] * na);
+                    d[i] = d[i] * __builtin_amdgcn_rcpf(1.0f + e);
+                }
+            } else if (fast == EP_FAST_ADD) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] += operand(y[k], i);
+            } else if (fast == EP_FAST_SUM) {
+                const float sc = ep.po[0].scale;
+#pragma unroll
+                for (int i = 0; i < 4; i++) d[i] += sc * (operand(y[k], i) - 0.f);
+            }
+            const int64_t off = b * ep.dst.sb + (m_first + row) * ep.dst.sm + n;
+            if (bf) {
+                uint16_t *q = (uint16_t *)ep.dst.ptr + off;
+                uint32_t h0, h1;
+                if constexpr (PACK) {
+                    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h0) : "v"(d[0]), "v"(d[1]));
+                    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h1) : "v"(d[2]), "v"(d[3]));
+                } else {
+                    h0 = f32_to_bf16(d[0]) | (uint32_t)f32_to_bf16(d[1]) << 16;
+                    h1 = f32_to_bf16(d[2]) | (uint32_t)f32_to_bf16(d[3]) << 16;
+                }
+                if (nvalid == 4) {
+                    *(v2u_any *)q = v2u_any {h0, h1};
+                } else {
+                    q[0] = (uint16_t)h0;
+                    if (nvalid > 1) q[1] = (uint16_t)(h0 >> 16);
+                    if (nvalid > 2) q[2] = (uint16_t)h1;
+                }
+            } else {
+                float *q = (float *)ep.dst.ptr + off;
+                if (nvalid == 4) {
+                    *(v4f_any *)q = v4f_any {d[0], d[1], d[2], d[3]};
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 3; i++)
+                        if (i < nvalid) q[i] = d[i];
+                }
+            }
+        }
+    }
+}
+
 // Straight-line epilogue of four neighbouring results of one row when nothing
 // has to be checked per lane: the four columns exist, dst (and a binary
 // operand) can be accessed as one vector. FAST is the recognised shape, BF16

@@ -337,6 +337,16 @@ gemm_b8_kernel(const gemm_params_t p) {
     const float ws4[4] = {cols.ws[0], cols.ws[1], cols.ws[2], cols.ws[3]};
     static_for<FM>([&](auto I) {
         constexpr int i = decltype(I)::value;
+        const int m_first = m0 + wm0 + i * 32, nv = min(32, p.M - m_first);
+        const int lrow = lane / (WN / 4);
+        // the source scales of the rows the lane visits, requested ahead of the staging
+        float ssr[32 / ROWS_PER_IT];
+#pragma unroll
+        for (int it = 0; it < 32 / ROWS_PER_IT; it++)
+            ssr[it] = has_ss && nv > 0
+                    ? ep_load(p.ep.src_scale, bz,
+                            m_first + min(it * ROWS_PER_IT + lrow, nv - 1), 0)
+                    : 1.f;
         // weights zero points: the row sums of the lane's 16 rows (s32
         // arithmetic wraps as the reference's int accumulation does)
         int rsr[16];
@@ -365,19 +375,29 @@ gemm_b8_kernel(const gemm_params_t p) {
                 stg[row * WN + j * 32 + (lane & 31)] = v;
             }
         }
+        float *const ssl = (float *)lds + WGM * WGN * 32 * WN + wave * 32;
+        if (ecol == 0) {
+#pragma unroll
+            for (int it = 0; it < 32 / ROWS_PER_IT; it++)
+                ssl[it * ROWS_PER_IT + lrow] = ssr[it];
+        }
+        if (p.ep.fast != EP_FAST_NONE && !p.ep.fast_ext) {
+            auto staged = [&](int row, float (&v)[4], float &ss) {
+                const float4 t = *(const float4 *)&stg[row * WN + ecol];
+                v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
+                ss = ssl[row];
+            };
+            epilogue_fast_rows<32 / ROWS_PER_IT, 32 / ROWS_PER_IT, ROWS_PER_IT, false>(
+                    p.ep, has_ss, has_ws, ws4, bz, m_first, nv, lrow, en, envalid, staged);
+        } else {
 #pragma unroll 1
-        for (int it = 0; it < 32 / ROWS_PER_IT; it++) {
-            const int row = it * ROWS_PER_IT + lane / (WN / 4);
-            const float4 t = *(const float4 *)&stg[row * WN + ecol];
-            const int m = m0 + wm0 + i * 32 + row;
-            if (m < p.M && en < p.N) {
-                float v[4] = {t.x, t.y, t.z, t.w};
-                const float ss = has_ss ? ep_load(p.ep.src_scale, bz, m, 0) : 1.f;
-                if (p.ep.fast != EP_FAST_NONE && !p.ep.fast_ext)
-                    epilogue_fast4(
-                            p.ep, v, has_ss, ss, has_ws, ws4, bz, m, en, envalid);
-                else
-                    epilogue_rows4(epk, cols, v, has_ss, ss, bz, m, en, envalid);
+            for (int it = 0; it < 32 / ROWS_PER_IT; it++) {
+                const int row = it * ROWS_PER_IT + lrow;
+                const float4 t = *(const float4 *)&stg[row * WN + ecol];
+                if (row < nv && en < p.N) {
+                    float v[4] = {t.x, t.y, t.z, t.w};
+                    epilogue_rows4(epk, cols, v, has_ss, ssl[row], bz, m_first + row, en, envalid);
+                }
             }
         }
     });
@@ -394,7 +414,7 @@ static void launch_cfg(const gemm_params_t &p, hipStream_t stream) {
     const int grid_x = ntiles >= 64 ? ((ntiles + 7) / 8) * 8 : ntiles;
     constexpr size_t lds_main = (size_t)STAGES * (BM + BN) * BK;
     constexpr size_t lds_ep
-            = (size_t)WGM * WGN * 32 * (BN / WGN) * sizeof(float);
+            = (size_t)WGM * WGN * 32 * (BN / WGN + 1) * sizeof(float); // results, scales
     constexpr size_t lds = lds_main > lds_ep ? lds_main : lds_ep;
     auto kern = gemm_b8_kernel<BM, BN, BK, WGM, WGN, STAGES, F8, U8A>;
     ensure_dynamic_lds((const void *)kern, (int)lds);
@@ -466,13 +486,21 @@ bool gemm_b8_uses_tile256(const gemm_params_t &p, bool f8, int variant) {
     const int64_t tm = (p.M + 255) / 256;
     const int64_t tiles256 = tm * ((p.N + 255) / 256) * p.batch;
     if (tiles256 >= 192) return true;
+    // fp8: fewer tiles too, unless K is long and two 128 x 128 tiles for every large
+    // one would not even fill the CUs once (us, 128 x 128 / 256 x 256: 2048 x 1024 x
+    // 1024 26.1 / 23.0, 2048 x 2048 x 2048 35.1 / 31.9, 1024 x 4096 x 4096 46.0 / 46.4,
+    // 256 x 8192 x 8192 60.4 / 75.1, 512 x 14336 x 4096 86.6 / 119.8, 2048 x 4096 x 4096
+    // 58.4 / 49.6, 1300 x 8192 x 5120 82.7 / 77.1)
+    if (f8)
+        return p.K < 4096
+                || (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch > 256;
     // int8 with an s8 source also has the 256 x 128 kernel with two workgroups
     // per CU, which beats the tiles below from 32 such tiles on, unless the row
     // tiles are mostly padding and the tiles are few (measured with a swish /
     // bf16 epilogue: 256 x 4096 x 4096 29 against 37 us, 2048 x 4096 x 4096 40
     // against 67, 1024 x 512 x 1024 13 against 21; 512 x 1024 x 1024 (16 tiles)
     // 15 against 10 and 128 x 4096 x 4096 (half-empty row tiles) 29 against 18)
-    if (f8 || (p.switches & (GEMM_ONE_PER_CU | GEMM_MFMA32))) return false;
+    if (p.switches & (GEMM_ONE_PER_CU | GEMM_MFMA32)) return false;
     const int64_t tiles128 = tm * ((p.N + 127) / 128) * p.batch;
     const bool rows_full = 4 * (int64_t)p.M >= 3 * tm * 256;
     return tiles128 >= 32 && (rows_full || tiles128 >= 96);
@@ -492,7 +520,8 @@ void launch_gemm_b8(const gemm_params_t &p, bool f8, int variant,
         const int64_t mid = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128)
                 * p.batch;
         // small problems: more, smaller tiles keep more CUs busy
-        variant = big >= 256 ? 1 : (mid >= 64 ? 2 : 3);
+        // (fp8 on 256 x 128: 88.5 instead of 58.4 us, 2048 x 4096 x 4096)
+        variant = big >= 256 && !f8 ? 1 : (mid >= 64 ? 2 : 3);
     }
     switch (variant) {
         case 1: launch_gemm_b8_v1(p, f8, stream); break;

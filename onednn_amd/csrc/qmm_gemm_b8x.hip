@@ -213,62 +213,6 @@ QMM_D int a_swz16(int row, int q) {
     QX_MF(2, 0, CB); QX_MF(2, 1, CB); QX_MF(2, 2, CB); QX_MF(2, 3, CB); \
     QX_MF(3, 0, CB); QX_MF(3, 1, CB); QX_MF(3, 2, CB); QX_MF(3, 3, CB);
 
-// epilogue_fast4 for a full group of four bf16 results: same arithmetic, the
-// conversion done by v_cvt_pk_bf16_f32 (round to nearest even; the caller runs
-// with f32 denormals flushed, which reproduces the reference's subnormal -> 0).
-QMM_D void epilogue_fast4_bf16(const epilogue_t &ep, float (&d)[4], bool has_ss,
-        float ss, bool has_ws, const float (&ws)[4], int64_t b, int64_t m,
-        int64_t n) {
-    if (has_ss) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            d[i] *= ss;
-    }
-    if (has_ws) {
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            d[i] *= ws[i];
-    }
-    const int64_t dst_off = b * ep.dst.sb + m * ep.dst.sm + n;
-    uint16_t *q = (uint16_t *)ep.dst.ptr + dst_off;
-    const int fast = ep.fast;
-    if (fast == EP_FAST_RELU) {
-        const float alpha = ep.po[0].alpha;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            d[i] = d[i] > 0 ? d[i] : d[i] * alpha;
-    } else if (fast == EP_FAST_SWISH) {
-        const float na = -ep.po[0].alpha * 1.44269504088896340736f;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float e = __builtin_amdgcn_exp2f(d[i] * na);
-            d[i] = d[i] * __builtin_amdgcn_rcpf(1.0f + e);
-        }
-    } else if (fast == EP_FAST_ADD) {
-        const float *y = (const float *)ep.po[0].t.ptr + b * ep.po[0].t.sb
-                + m * ep.po[0].t.sm + n;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            d[i] += y[i];
-    } else if (fast == EP_FAST_SUM) {
-        const float sc = ep.po[0].scale;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            d[i] += sc * (bf16_to_f32(q[i]) - 0.f);
-    }
-    uint32_t h0, h1;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h0) : "v"(d[0]), "v"(d[1]));
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(h1) : "v"(d[2]), "v"(d[3]));
-    if ((((uintptr_t)q) & 7) == 0) {
-        *(uint2 *)q = make_uint2(h0, h1);
-    } else {
-        q[0] = (uint16_t)h0;
-        q[1] = (uint16_t)(h0 >> 16);
-        q[2] = (uint16_t)h1;
-        q[3] = (uint16_t)(h1 >> 16);
-    }
-}
-
 // Epilogue of 64 staged rows when the wave's 128 x 128 tile lies fully inside
 // the matrix and the dst rows are vector-aligned: no per-lane conditions, so
 // the rows pipeline. FAST is the recognised epilogue shape, DSTK the dst type,
@@ -487,7 +431,7 @@ QMM_D void tile_epilogue(const gemm_params_t &p, AccT (&acc)[NFI][NFJ],
                                    : 0)
                         - p.w_off;
     }
-    const bool full = m0 + wm0 + 128 <= p.M && n0 + wn0 + WN <= p.N
+    const bool full = n0 + wn0 + WN <= p.N
             && ep.fast != EP_FAST_NONE && epilogue_full4_ok(ep)
             && (!LEAN || (ep.fast <= EP_FAST_SUM && dstk <= EP_DST_F16));
     static_for<2>([&](auto H) {
@@ -535,7 +479,7 @@ QMM_D void tile_epilogue(const gemm_params_t &p, AccT (&acc)[NFI][NFJ],
                 *(int4 *)&stg_m[row * PITCH + ecol] = t;
             }
         }
-        if (full) {
+        if (full && m0 + wm0 + h * 64 + 64 <= p.M) {
             const int64_t m_first = m0 + wm0 + h * 64;
             const float *const ssh = ssl + h * 64;
 #define QX_EP_ROWS(F, D, X) \
@@ -580,35 +524,35 @@ QMM_D void tile_epilogue(const gemm_params_t &p, AccT (&acc)[NFI][NFJ],
 #undef QX_EP_DST
 #undef QX_EP_CASE
         } else {
-#pragma unroll 2
-            for (int it = 0; it < 64 / RPI; it++) {
-                const int row = it * RPI + lane / LPR;
+            auto staged = [&](int row, float (&v)[4], float &ss) {
                 const int4 t = *(const int4 *)&stg_r[row * PITCH + ecol];
-                const int lrow = h * 64 + row;
-                const int m = m0 + wm0 + lrow;
-                const float ss = ssl[lrow];
-                if (m < p.M && envalid > 0) {
-                    float v[4];
-                    if constexpr (F8) {
-                        v[0] = u2f((uint32_t)t.x);
-                        v[1] = u2f((uint32_t)t.y);
-                        v[2] = u2f((uint32_t)t.z);
-                        v[3] = u2f((uint32_t)t.w);
-                    } else {
-                        v[0] = (float)(int32_t)((uint32_t)t.x + (uint32_t)cs4[0]);
-                        v[1] = (float)(int32_t)((uint32_t)t.y + (uint32_t)cs4[1]);
-                        v[2] = (float)(int32_t)((uint32_t)t.z + (uint32_t)cs4[2]);
-                        v[3] = (float)(int32_t)((uint32_t)t.w + (uint32_t)cs4[3]);
+                ss = ssl[h * 64 + row];
+                if constexpr (F8) {
+                    v[0] = u2f((uint32_t)t.x);
+                    v[1] = u2f((uint32_t)t.y);
+                    v[2] = u2f((uint32_t)t.z);
+                    v[3] = u2f((uint32_t)t.w);
+                } else {
+                    v[0] = (float)(int32_t)((uint32_t)t.x + (uint32_t)cs4[0]);
+                    v[1] = (float)(int32_t)((uint32_t)t.y + (uint32_t)cs4[1]);
+                    v[2] = (float)(int32_t)((uint32_t)t.z + (uint32_t)cs4[2]);
+                    v[3] = (float)(int32_t)((uint32_t)t.w + (uint32_t)cs4[3]);
+                }
+            };
+            const int m_first = m0 + wm0 + h * 64, nv = min(64, p.M - m_first);
+            if (ep.fast != EP_FAST_NONE && !ext) {
+                epilogue_fast_rows<LEAN ? 8 : 4, 64 / RPI, RPI, true>(ep, has_ss, has_ws,
+                        ws4, bz, m_first, nv, lane / LPR, en, envalid, staged);
+            } else {
+#pragma unroll 2
+                for (int it = 0; it < 64 / RPI; it++) {
+                    const int row = it * RPI + lane / LPR;
+                    if (row < nv && envalid > 0) {
+                        float v[4], ss;
+                        staged(row, v, ss);
+                        epilogue_rows4(epk, cols, v, has_ss, ss, bz, m_first + row, en,
+                                envalid);
                     }
-                    if (ep.fast == EP_FAST_NONE || ext)
-                        epilogue_rows4(
-                                epk, cols, v, has_ss, ss, bz, m, en, envalid);
-                    else if (to_bf16 && envalid == 4)
-                        epilogue_fast4_bf16(
-                                ep, v, has_ss, ss, has_ws, ws4, bz, m, en);
-                    else
-                        epilogue_fast4(ep, v, has_ss, ss, has_ws, ws4, bz, m,
-                                en, envalid);
                 }
             }
         }
