@@ -382,18 +382,23 @@ void launch_gemm_w4f_part2(const gemv_params_t &, int, int, hipStream_t);
 void launch_gemm_w4f_part3(const gemv_params_t &, int, int, hipStream_t);
 
 // Whether the tiled kernel is the better way to run p.M > 16 rows, against the
-// decode kernel once per block of 16 rows. Both walk K at about the same pace;
-// measured at K = 4096: a pass of the decode kernel over 4096 columns 4.3 us, a
-// round of 128-column workgroups 26 us (32 rows) or 40 us (64 rows).
+// decode kernel once per block of 16 rows. Measured (us, f16 x u4): a round of
+// 128-column workgroups of 32 rows 10.5 / 15.7 / 26 / 47 at K = 1024 / 2048 / 4096 /
+// 8192, of 64 rows 15.4 / 21.9 / 36 / 64; a pass of the decode kernel over 4096 columns
+// 4.3 up to K = 4096 (what is left of a short K is its start and end), 7.8 at 8192. Decode
+// kernel / tiled: 100 x 1024 x 4096 30.0 / 15.4, 20 x 1024 x 10576 22.6 / 10.6, 232 x 1024
+// x 1280 23.2 / 15.1, 100 x 1024 x 1280 13.5 / 15.4, 100 x 8192 x 4096 54.4 / 64.1; u8
+// weights alike (100 x 1024 x 4096 34.3 / 18.3).
 bool gemm_w4f_wins(const gemv_params_t &p) {
     if (p.M <= 16) return false;
     const int64_t wide = (int64_t)((p.M + 63) / 64) * ((p.N + 255) / 256);
     if (p.M > 64 && wide >= 128) return true;
     const int bm = p.M <= 32 ? 32 : 64;
+    const double k = p.K / 1024.0;
     const double wgs = (double)((p.M + bm - 1) / bm) * ((p.N + 127) / 128);
     const double rounds = wgs <= 256 ? 1.0 : wgs / 256;
-    const double tiled = (bm == 32 ? 26.0 : 40.0) * rounds;
-    const double passes = (double)((p.M + 15) / 16) * 4.3 * p.N / 4096.0;
+    const double tiled = (bm == 32 ? 5.3 + 5.1 * k : 8.6 + 6.9 * k) * rounds;
+    const double passes = (double)((p.M + 15) / 16) * 4.3 * p.N / 4096.0 * (k > 4 ? k / 4 : 1);
     return tiled < passes;
 }
 
