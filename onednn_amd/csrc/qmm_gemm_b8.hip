@@ -326,6 +326,8 @@ gemm_b8_kernel(const gemm_params_t p) {
     const int envalid = min(4, p.N - en);
     const bool has_ss = p.ep.src_scale.ptr != nullptr;
     const bool has_ws = p.ep.wei_scale.ptr != nullptr;
+    const bool ss_row = has_ss && p.ep.src_scale.sm != 0; // else one for the batch entry
+    const float ss0 = has_ss && !ss_row ? ep_load(p.ep.src_scale, bz, 0, 0) : 1.f;
     // what depends on the lane's 4 columns only, fetched once
     ep_cols_t cols;
     epilogue_cols_load(p.ep, cols, bz, en, envalid > 0 ? envalid : 0);
@@ -343,7 +345,7 @@ gemm_b8_kernel(const gemm_params_t p) {
         float ssr[32 / ROWS_PER_IT];
 #pragma unroll
         for (int it = 0; it < 32 / ROWS_PER_IT; it++)
-            ssr[it] = has_ss && nv > 0
+            ssr[it] = ss_row && nv > 0
                     ? ep_load(p.ep.src_scale, bz,
                             m_first + min(it * ROWS_PER_IT + lrow, nv - 1), 0)
                     : 1.f;
@@ -376,7 +378,7 @@ gemm_b8_kernel(const gemm_params_t p) {
             }
         }
         float *const ssl = (float *)lds + WGM * WGN * 32 * WN + wave * 32;
-        if (ecol == 0) {
+        if (ss_row && ecol == 0) {
 #pragma unroll
             for (int it = 0; it < 32 / ROWS_PER_IT; it++)
                 ssl[it * ROWS_PER_IT + lrow] = ssr[it];
@@ -385,7 +387,7 @@ gemm_b8_kernel(const gemm_params_t p) {
             auto staged = [&](int row, float (&v)[4], float &ss) {
                 const float4 t = *(const float4 *)&stg[row * WN + ecol];
                 v[0] = t.x, v[1] = t.y, v[2] = t.z, v[3] = t.w;
-                ss = ssl[row];
+                ss = ss_row ? ssl[row] : ss0;
             };
             epilogue_fast_rows<32 / ROWS_PER_IT, 32 / ROWS_PER_IT, ROWS_PER_IT, false>(
                     p.ep, has_ss, has_ws, ws4, bz, m_first, nv, lrow, en, envalid, staged);
@@ -396,7 +398,8 @@ gemm_b8_kernel(const gemm_params_t p) {
                 const float4 t = *(const float4 *)&stg[row * WN + ecol];
                 if (row < nv && en < p.N) {
                     float v[4] = {t.x, t.y, t.z, t.w};
-                    epilogue_rows4(epk, cols, v, has_ss, ssl[row], bz, m_first + row, en, envalid);
+                    epilogue_rows4(epk, cols, v, has_ss, ss_row ? ssl[row] : ss0, bz,
+                            m_first + row, en, envalid);
                 }
             }
         }
