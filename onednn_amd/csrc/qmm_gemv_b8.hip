@@ -111,7 +111,11 @@ QMM_D void gb8_tail_store(const gemm_params_t &p, const epilogue_t &epk,
 }
 
 // F8: f8_e4m3 on both sides, f32 sums (two fragments to an MFMA of 64 k)
-template <int MR, bool F8>
+// QUADS: the end takes four columns per thread; else, for at most 16 rows, a thread per
+// result: a long post-op is one chain of them and not four (16 x 4096 x 4096 8.3 / 8.8,
+// 1 x 1024 x 4096 with a swish 6.0 / 6.7 us; 32 x 4096 x 4096 9.9 / 9.4 the other way).
+// Kernels of their own: either end behind a branch cost the few rows 0.4 us.
+template <int MR, bool F8, bool QUADS>
 __global__ void __launch_bounds__(GB8_WAVES * 64)
 gemv_b8_kernel(const gemm_params_t p) {
     typedef typename std::conditional<F8, v16f, v16i>::type acc_t;
@@ -130,7 +134,7 @@ gemv_b8_kernel(const gemm_params_t p) {
     };
     // column block and first row. A column block's row blocks are 8 workgroups apart:
     // on one XCD, close in time, so that its weights come from memory once
-    const int nrb = MR == 32 ? (p.M + 31) / 32 : 1;
+    const int nrb = QUADS ? (p.M + 31) / 32 : 1;
     int nb = blockIdx.x, m0 = 0;
     if (nrb > 1) {
         nb = blockIdx.x / (8 * nrb) * 8 + blockIdx.x % 8;
@@ -264,13 +268,47 @@ gemv_b8_kernel(const gemm_params_t p) {
         const int tot = rsum[rb] + __shfl_xor(rsum[rb], 32);
         if (lane < (MR < 32 ? MR : 32)) red_rs(wave, 32 * rb + lane) = tot;
     }
-    const int tid = threadIdx.x, tr = tid >> 3, tn = nb * 32 + (tid & 7) * 4;
-    gb8_tail_t tail;
-    if (tr < MR) gb8_tail_load(p, need_rs, m0 + tr, tn, tail);
-    __syncthreads();
-    const epilogue_t &epk
-            = ((const gemm_params_t *)__builtin_amdgcn_kernarg_segment_ptr())->ep;
-    if (tr < MR) gb8_tail_store<F8>(p, epk, tail, lds_raw, WAVE_LDS, MR, tr, m0 + tr, tn);
+    const int tid = threadIdx.x;
+    if constexpr (!QUADS) {
+        __syncthreads();
+        const int r = tid >> 5, n = nb * 32 + (tid & 31);
+        if (r >= rows || r >= MR || n >= p.N) return;
+        float d = 0.f;
+        uint32_t v = 0, rs = 0;
+#pragma unroll
+        for (int w = 0; w < GB8_WAVES; w++) {
+            const int x = red(w, r, tid & 31);
+            if constexpr (F8) {
+                d += u2f((uint32_t)x);
+            } else {
+                v += (uint32_t)x;
+                rs += (uint32_t)red_rs(w, r);
+            }
+        }
+        if constexpr (!F8) {
+            int comp = p.a_is_u8 ? 128 : 0;
+            if (p.src_zp) comp -= load_int(p.src_zp_dt, p.src_zp, 0);
+            const int cs = comp != 0 && p.colsum ? comp * p.colsum[n] : 0;
+            const int zw = need_rs
+                    ? (p.wei_zp ? load_int(p.wei_zp_dt, p.wei_zp, (int64_t)n * p.wei_zp_sn)
+                                : 0)
+                            - p.w_off
+                    : 0;
+            // s32 arithmetic that wraps as the reference's int accumulation
+            v += (uint32_t)cs - (uint32_t)zw * (rs + (uint32_t)p.K * (uint32_t)comp);
+            d = (float)(int32_t)v;
+        }
+        epilogue_apply_store(p.ep, d, 0, m0 + r, n);
+    } else {
+        const int tr = tid >> 3, tn = nb * 32 + (tid & 7) * 4;
+        gb8_tail_t tail;
+        if (tr < MR) gb8_tail_load(p, need_rs, m0 + tr, tn, tail);
+        __syncthreads();
+        const epilogue_t &epk
+                = ((const gemm_params_t *)__builtin_amdgcn_kernarg_segment_ptr())->ep;
+        if (tr < MR)
+            gb8_tail_store<F8>(p, epk, tail, lds_raw, WAVE_LDS, MR, tr, m0 + tr, tn);
+    }
 }
 
 // 33 ... 64 rows: a workgroup owns CB blocks of 32 columns, so that the source rows,
@@ -404,7 +442,7 @@ bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256) {
 void launch_gemv_b8(const gemm_params_t &p, bool f8, hipStream_t stream) {
     if (p.M <= 0 || p.N <= 0) return;
     auto go = [&](auto kern, int64_t blocks, int lds) {
-        ensure_dynamic_lds((const void *)kern, lds);
+        if (lds > 65536) ensure_dynamic_lds((const void *)kern, lds);
         hipLaunchKernelGGL(
                 kern, dim3((unsigned)blocks), dim3(GB8_WAVES * 64), lds, stream, p);
     };
@@ -412,14 +450,17 @@ void launch_gemv_b8(const gemm_params_t &p, bool f8, hipStream_t stream) {
     const int64_t nrb = (p.M + 31) / 32;
     const int64_t grid32 = nrb > 1 ? (p.nb32 + 7) / 8 * 8 * nrb : p.nb32;
     if (p.M <= 4)
-        f8 ? go(gemv_b8_kernel<4, true>, p.nb32, lds4)
-           : go(gemv_b8_kernel<4, false>, p.nb32, lds4);
+        f8 ? go(gemv_b8_kernel<4, true, false>, p.nb32, lds4)
+           : go(gemv_b8_kernel<4, false, false>, p.nb32, lds4);
+    else if (p.M <= 16)
+        f8 ? go(gemv_b8_kernel<32, true, false>, p.nb32, lds32)
+           : go(gemv_b8_kernel<32, false, false>, p.nb32, lds32);
     // 33 ... 64 rows as two blocks of 32 where these are at most one workgroup to a CU
     // (64 rows, us, two blocks / one of 64: 4096 x 4096 8.6 / 11.6, 14336 x 4096 20.8 /
     // 28.5, 1024 x 6144 7.5 / 6.5, 8192 x 8192 23.7 / 21.7, 4096 x 14336 23.1 / 22.6)
     else if (f8 || p.M <= 32 || p.M > 64 || p.nb32 <= 128)
-        f8 ? go(gemv_b8_kernel<32, true>, grid32, lds32)
-           : go(gemv_b8_kernel<32, false>, grid32, lds32);
+        f8 ? go(gemv_b8_kernel<32, true, true>, grid32, lds32)
+           : go(gemv_b8_kernel<32, false, true>, grid32, lds32);
     else
         go(gemv_b8_rows64_kernel, p.nb32, GB8_WAVES * 64 * (4 * 32 + 16));
 }
