@@ -489,14 +489,18 @@ bool gemm_b8_uses_tile256(const gemm_params_t &p, bool f8, int variant) {
     const int64_t tm = (p.M + 255) / 256;
     const int64_t tiles256 = tm * ((p.N + 255) / 256) * p.batch;
     if (tiles256 >= 192) return true;
-    // fp8: fewer tiles too, unless K is long and two 128 x 128 tiles for every large
-    // one would not even fill the CUs once (us, 128 x 128 / 256 x 256: 2048 x 1024 x
-    // 1024 26.1 / 23.0, 2048 x 2048 x 2048 35.1 / 31.9, 1024 x 4096 x 4096 46.0 / 46.4,
-    // 256 x 8192 x 8192 60.4 / 75.1, 512 x 14336 x 4096 86.6 / 119.8, 2048 x 4096 x 4096
-    // 58.4 / 49.6, 1300 x 8192 x 5120 82.7 / 77.1)
-    if (f8)
-        return p.K < 4096
-                || (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch > 256;
+    // fp8 with fewer tiles: time against time. Measured (us, into a bf16 residual): one
+    // round of 256 x 256 tiles 23 / 32 / 46 / 75 / 120 at K = 1024 / 2048 / 4096 / 8192 /
+    // 14336, about 20 more where columns end inside a wave's 128; 128 x 128 tiles 26 / 35
+    // / 45 / 60 / 87 while every CU has one at most, 58 / 83 (4096 / 8192) with two
+    // (2048 x 4096 x 4096 58.4 / 49.6, 512 x 14336 x 4096 86.6 / 119.8, 1100 x 2048 x 4000
+    // 48.0 / 55.3)
+    if (f8) {
+        const double k = p.K / 1024.0;
+        const double mid = (double)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+        const double t128 = (mid <= 256 ? 22 + 5 * k : 33 + 6.2 * k) * (mid > 512 ? mid / 512 : 1);
+        return 16 + 7.3 * k + (p.N % 128 ? 20 : 0) < t128;
+    }
     // int8 with an s8 source also has the 256 x 128 kernel with two workgroups
     // per CU, which beats the tiles below from 32 such tiles on, unless the row
     // tiles are mostly padding and the tiles are few (measured with a swish /
