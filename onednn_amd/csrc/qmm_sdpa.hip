@@ -9,8 +9,8 @@
 // reorder does: f16(scale * (x - zero_point)), in f32 arithmetic for bf16
 // queries and for f32 scales / s32 zero points.
 //
-// Many queries without an explicit mask over an unquantized cache of head size 64 or
-// 128 run on the kernel of qmm_sdpa_prefill.hip; the rest here.
+// Many queries without an explicit mask at head sizes 64 and 128 run on the kernel of
+// qmm_sdpa_prefill.hip (an 8-bit cache from 257 queries on); the rest here.
 //
 // The scores never leave the CU. A workgroup owns 128 queries of one head (four
 // waves of 32) and walks the keys 32 at a time:
@@ -1040,8 +1040,9 @@ const char *qmm_sdpa_impl_name(const qmm_sdpa_desc_t *desc) {
 
 size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc) {
     sdpa_params_t p;
-    if (!desc || !supported(*desc, &p) || p.Qn > 16) return 0;
+    if (!desc || !supported(*desc, &p)) return 0;
     const int64_t D = desc->q.dims[desc->q.ndims - 1];
+    if (p.Qn > 16) return sdpa_prefill_scratch(p, (int)D);
     const sdpa_split_t sp = decode_split(p, D);
     if (sp.nsplit <= 1) return 0;
     return (size_t)p.B0 * p.B1 * sp.nsplit * part_pitch(p.Qn, (int)D) * sizeof(float);
@@ -1132,7 +1133,8 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
         return hipGetLastError() == hipSuccess ? QMM_OK : QMM_RUNTIME_ERROR;
     }
     if (sdpa_prefill_takes(p, D)) {
-        if (!sdpa_prefill_launch(p, D, hip_stream)) return QMM_UNIMPLEMENTED;
+        if (sdpa_prefill_scratch(p, D) && !args->scratch) return QMM_INVALID_ARGUMENTS;
+        if (!sdpa_prefill_launch(p, D, args->scratch, hip_stream)) return QMM_UNIMPLEMENTED;
         return hipGetLastError() == hipSuccess ? QMM_OK : QMM_RUNTIME_ERROR;
     }
     const dim3 grid((unsigned)(p.B0 * p.B1),

@@ -129,9 +129,11 @@ QMM_D uint4 dequant8_f16(uint32_t w0, uint32_t w1, const h2 &sc, const h2 &off) 
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// many queries without an explicit mask, K / V in their type (qmm_sdpa_prefill.hip)
+// many queries without an explicit mask (qmm_sdpa_prefill.hip); scratch: what
+// sdpa_prefill_scratch asks for, an 8-bit cache in the queries' type
 bool sdpa_prefill_takes(const sdpa_params_t &p, int D);
-bool sdpa_prefill_launch(const sdpa_params_t &p, int D, void *hip_stream);
+size_t sdpa_prefill_scratch(const sdpa_params_t &p, int D);
+bool sdpa_prefill_launch(const sdpa_params_t &p, int D, void *scratch, void *hip_stream);
 
 } // namespace qmm
 

@@ -1,6 +1,6 @@
 // Scaled dot-product attention over many queries, K and V in the queries' 16-bit
-// type, head sizes 64 and 128, causal or not, no explicit mask (the rest:
-// qmm_sdpa.hip, which also describes the arithmetic).
+// type (or written in it first), head sizes 64 and 128, causal or not, no explicit
+// mask (the rest: qmm_sdpa.hip, which also describes the arithmetic).
 //
 // A workgroup owns 128 queries of a head; its eight waves are two groups of four,
 // a wave 32 queries, and the groups take the keys' tiles of 64 in turn, each with
@@ -461,21 +461,89 @@ sdpa_prefill_kernel(const sdpa_params_t p) {
         }
 }
 
-} // namespace
-
-// Whether the kernel above takes a problem: wherever it can, it was the faster one at
-// every size tried (see the top); byte offsets inside a head have 32 bits here
-bool sdpa_prefill_takes(const sdpa_params_t &p, int D) {
-    if (D != 64 && D != 128) return false;
-    if (p.mask_dt != dt_undef || p.kv_dt != (p.bf ? dt_bf16 : dt_f16)) return false;
-    return (int64_t)p.S * p.k.row * 2 < (int64_t)1 << 31
-            && (int64_t)p.S * p.v.row * 2 < (int64_t)1 << 31;
+// An 8-bit cache for the kernel above: K and V as dense [head][key][D] arrays of the
+// queries' type, with the values (and the arithmetic) of the kernels that dequantize
+// while they stage. Bound: HBM; one pass here instead of one per 128 queries there.
+template <bool BF>
+__global__ void __launch_bounds__(256)
+sdpa_dequant_kernel(const sdpa_params_t p, int D, int kv1, uint16_t *K, uint16_t *V) {
+    const int per_row = D / 8;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)p.S * per_row) return;
+    const int key = (int)(i / per_row), ch = (int)(i % per_row);
+    const int kb0 = blockIdx.y / kv1, kb1 = blockIdx.y % kv1;
+    const bool v = blockIdx.z != 0;
+    const sdpa_strides_t &st = v ? p.v : p.k;
+    const uint2 w = *(const uint2 *)((const uint8_t *)(v ? p.V : p.K) + kb0 * st.b0
+            + kb1 * st.b1 + (int64_t)key * st.row + ch * 8);
+    const int64_t qi = kb0 * p.qz_b0 + kb1 * p.qz_b1 + key;
+    const void *sp = v ? p.v_scale : p.k_scale, *zp = v ? p.v_zp : p.k_zp;
+    const float s = sp ? ld_scale(v ? p.vs_dt : p.ks_dt, sp, qi) : 1.f;
+    const float z = zp ? ld_zp(v ? p.vz_dt : p.kz_dt, zp, qi) : 0.f;
+    const bool sgn = p.kv_dt == dt_s8;
+    const uint32_t flip = sgn ? 0x80808080u : 0u;
+    const float zb = z + (sgn ? 128.f : 0.f);
+    const uint32_t b[2] = {w.x ^ flip, w.y ^ flip};
+    uint4 o;
+    if (p.fastq) {
+        o = dequant8_f16(b[0], b[1], twice(s), twice(1024.f + zb));
+    } else {
+        float f[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            f[j] = s * ((float)((b[j >> 2] >> (8 * (j & 3))) & 0xff) - zb);
+        o = make_uint4(cvt_pair<BF>(f[0], f[1]), cvt_pair<BF>(f[2], f[3]),
+                cvt_pair<BF>(f[4], f[5]), cvt_pair<BF>(f[6], f[7]));
+    }
+    *(uint4 *)((v ? V : K) + ((int64_t)blockIdx.y * p.S * D + i * 8)) = o;
 }
 
-bool sdpa_prefill_launch(const sdpa_params_t &p, int D, void *hip_stream) {
+} // namespace
+
+// Whether the kernel takes a problem: wherever it can, it was the faster one at every
+// size tried (see the top); byte offsets inside a head have 32 bits here. An 8-bit cache
+// is dequantized into the scratchpad first (up to 256 MiB of it), from 257 queries on: a
+// second launch and the scratchpad's order cost 8 us, dequantizing while staging once per
+// 128 queries (us, there / here, s8, f16: 32 heads x 200 of 64 13.9 / 17.3, 32 x 130 of
+// 128 15.5 / 17.6, 8 x 300 of 128 26.8 / 19.9, 4 x 500 of 64 25.9 / 19.2, 16 over 4 K / V
+// heads x 1005 of 128 79.4 / 29.4, 32 x 2048 175 / 67).
+bool sdpa_prefill_takes(const sdpa_params_t &p, int D) {
+    if ((D != 64 && D != 128) || p.mask_dt != dt_undef || p.Qn <= 16) return false;
+    if (p.kv_dt == (p.bf ? dt_bf16 : dt_f16))
+        return (int64_t)p.S * p.k.row * 2 < (int64_t)1 << 31
+                && (int64_t)p.S * p.v.row * 2 < (int64_t)1 << 31;
+    const int64_t heads = (int64_t)(p.B0 / p.kv_div0) * (p.B1 / p.kv_div1);
+    return p.Qn > 256 && heads <= 65535 && heads * p.S * D * 4 <= (int64_t)256 << 20;
+}
+
+size_t sdpa_prefill_scratch(const sdpa_params_t &p, int D) {
+    if (!sdpa_prefill_takes(p, D) || p.kv_dt == (p.bf ? dt_bf16 : dt_f16)) return 0;
+    return (size_t)(p.B0 / p.kv_div0) * (p.B1 / p.kv_div1) * p.S * D * 4;
+}
+
+bool sdpa_prefill_launch(
+        const sdpa_params_t &p0, int D, void *scratch, void *hip_stream) {
     constexpr int QW = 4, KT = 64;
+    sdpa_params_t p = p0;
     const dim3 grid((unsigned)(p.B0 * p.B1), (unsigned)((p.Qn + 32 * QW - 1) / (32 * QW)));
     if (grid.y > 65535) return false;
+    if (p.kv_dt != (p.bf ? dt_bf16 : dt_f16)) {
+        if (!scratch) return false;
+        const int kv0 = p.B0 / p.kv_div0, kv1 = p.B1 / p.kv_div1;
+        uint16_t *const K = (uint16_t *)scratch, *const V = K + (int64_t)kv0 * kv1 * p.S * D;
+        const dim3 dq((unsigned)(((int64_t)p.S * (D / 8) + 255) / 256), (unsigned)(kv0 * kv1), 2);
+        if (p.bf)
+            hipLaunchKernelGGL(sdpa_dequant_kernel<true>, dq, dim3(256), 0,
+                    (hipStream_t)hip_stream, p, D, kv1, K, V);
+        else
+            hipLaunchKernelGGL(sdpa_dequant_kernel<false>, dq, dim3(256), 0,
+                    (hipStream_t)hip_stream, p, D, kv1, K, V);
+        p.K = K;
+        p.V = V;
+        p.k.row = p.v.row = D;
+        p.k.b1 = p.v.b1 = (int64_t)p.S * D;
+        p.k.b0 = p.v.b0 = (int64_t)kv1 * p.S * D;
+    }
     const int lds = 8 / QW * 4 * KT * D * 2 + 2048;
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(512), lds, (hipStream_t)hip_stream, p);

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import onednn_amd as dnnl
+import oracle as O
 from onednn_amd import memory
 from qmm_harness import T, dt
 from test_gpu_sdpa import attention64, ctx, f16, f16_to_f64, reference_rule, run_sdpa, say  # noqa: F401
@@ -91,3 +92,28 @@ def test_infinite_values_stay_with_the_queries_that_see_them(ctx):  # noqa: F811
     got = f16_to_f64(run_sdpa(ctx, q, k, v, scale=0.125, causal=True))
     assert np.isposinf(got[:, :, S - 1:, 0]).all() and np.isfinite(got[..., 1:]).all()
     assert np.isfinite(got[:, :, :64]).all()  # whole tiles of 64 keys
+
+
+@pytest.mark.parametrize("kv_dt,sdt,zdt", [(dt.s8, dt.f16, dt.s8), (dt.u8, dt.f16, dt.u8), (dt.s8, dt.f16, None), (dt.s8, dt.f32, dt.s32)], ids=str)
+@pytest.mark.parametrize("Qn,S,D,qdt", [(257, 100, 128, dt.f16), (300, 301, 64, dt.bf16), (260, 65, 64, dt.f16)], ids=str)
+def test_8_bit_cache_under_many_queries(ctx, Qn, S, D, qdt, kv_dt, sdt, zdt):  # noqa: F811
+    """The cache is written in the queries' type to the scratchpad first: the oracle's reorder gives the same values."""
+    MB, H, KV = 2, 4, 2
+    say("sdpa prefill 8-bit cache %r" % ((Qn, S, D, qdt, kv_dt, sdt, zdt),))
+    r = np.random.default_rng(Qn + D)
+    q = f16(r.standard_normal((MB, H, Qn, D)), qdt)
+    lo, hi, npdt = (-128, 128, np.int8) if kv_dt == dt.s8 else (0, 256, np.uint8)
+    kq, vq = (r.integers(lo, hi, (MB, KV, S, D)).astype(npdt) for _ in range(2))
+    scale = [r.uniform(0.005, 0.02, (KV, S)) for _ in range(2)]
+    ksc, vsc = [f16(x) if sdt == dt.f16 else x.astype(np.float32) for x in scale]
+    znp = {dt.s8: np.int8, dt.u8: np.uint8, dt.s32: np.int32, None: np.int8}[zdt]
+    kzp, vzp = [(r.integers(-6, 7, (KV, S)) + (100 if zdt == dt.u8 else 0)).astype(znp) for _ in range(2)]
+    side = [(0b1110, g, sdt, sc, zdt, zp if zdt is not None else None)
+            for g, sc, zp in (((D, 1), ksc, kzp), ((1, D), vsc, vzp))]
+    got = run_sdpa(ctx, q, kq, vq, scale=0.125, causal=True, kv_heads=KV, kv_dt=kv_dt, k_q=side[0], v_q=side[1], qdt=qdt)
+    kd, vd = np.zeros((MB, KV, S, D), np.uint16), np.zeros((MB, KV, S, D), np.uint16)
+    for raw, sc, zp, outd in ((kq, ksc, kzp, kd), (vq, vsc, vzp, vd)):
+        O.reorder(O.Tensor(kv_dt, [MB, KV, S, D], raw), O.Tensor(qdt, [MB, KV, S, D], outd),
+                  src_scale=O.Quant(0b1110, sdt, sc, (1, D)),
+                  src_zp=O.Quant(0b1110, zdt, zp, (1, D)) if zdt is not None else None)
+    check(got, q, kd, vd, qdt, 0.125, True, H // KV)
