@@ -17,11 +17,10 @@
 //   * K and V tiles come by direct global -> LDS loads, two buffers each, requested in
 //     the vector slot before the one they are needed in; the fragments of a matrix
 //     slot are read four products ahead;
-//   * the accumulators are rescaled when a maximum grew. From 2048 keys on only when
-//     it grew by 2^8: the probabilities then reach 256 at most, and what is lost is
-//     that the largest one is no longer exactly 1 (distance from float64 over the
-//     last half of 4096 keys; in the first 2048 it would show: 2.58 instead of
-//     2.52e-4 at f16).
+//   * the accumulators are rescaled whenever a maximum grew, so that the largest
+//     probability is exactly 1. Letting it lag (up to 2^8) from 2048 keys on gained
+//     2 ... 4 % at 4096 ... 16384 keys and cost precision: where one late key outweighs
+//     the rest, its rounded weight no longer is what the sum has of it.
 // Bound: the power limit (1.5 GHz in a long run, matrix cores busy 57 % of its
 // cycles) and, below that, the vector ALU: a wave alone issues one instruction in
 // about 5 cycles, and the probabilities of a slot are about 190 of them next to
@@ -306,7 +305,7 @@ sdpa_prefill_kernel(const sdpa_params_t p) {
                 const v2u x = __builtin_amdgcn_permlane32_swap(u, u, false, false);
                 mx = fmaxf(u2f(x.x), u2f(x.y)) * mul;
             }
-            if (__builtin_amdgcn_ballot_w64(mx > m_run + (t < 16 ? 0.f : 8.f))) {
+            if (__builtin_amdgcn_ballot_w64(mx > m_run)) {
                 const float m_new = fmaxf(m_run, mx);
                 const float alpha = m_new == -INFINITY
                         ? 1.f

@@ -117,3 +117,26 @@ def test_8_bit_cache_under_many_queries(ctx, Qn, S, D, qdt, kv_dt, sdt, zdt):  #
                   src_scale=O.Quant(0b1110, sdt, sc, (1, D)),
                   src_zp=O.Quant(0b1110, zdt, zp, (1, D)) if zdt is not None else None)
     check(got, q, kd, vd, qdt, 0.125, True, H // KV)
+
+
+@pytest.mark.parametrize("qdt", [dt.f16, dt.bf16], ids=["f16", "bf16"])
+def test_a_late_key_that_outweighs_the_rest(ctx, qdt):  # noqa: F811
+    """Past 2048 keys one key's weight is 2^6.3 ... 2^7.7 of the largest before it. Its probability is exactly 1, as that
+    of every maximum, so the result is off by its own rounding and by what the other keys' rounded weights add: together
+    0.07 of the result (2^-6.3 and 4350 x 2^-16), each within half a unit of its own last place and independent of the
+    others. Against the float64 result rounded to the type that is at most sqrt(1 + 0.07^2) = 1.003 of the error; a
+    rounded weight of the late key would be as large as the result's own rounding (1.2 ... 1.4)."""
+    H, Qn, S, D = 1, 256, 4352, 64
+    say("sdpa prefill late key %s" % qdt)
+    r = np.random.default_rng(21)
+    q, k = np.zeros((1, H, Qn, D)), np.zeros((1, H, S, D))
+    q[..., 0] = np.linspace(0.9, 1.1, Qn)
+    k[..., 0] = -16 * np.log(2.0)
+    k[:, :, 5, 0] = 0.0
+    k[:, :, 66 * 64 + 10, 0] = 7 * np.log(2.0)  # (tiles of 64 keys go to two groups of waves in turn: the same group)
+    q, k, v = f16(q, qdt), f16(k, qdt), f16(r.standard_normal((1, H, S, D)), qdt)
+    got = f16_to_f64(run_sdpa(ctx, q, k, v, scale=1.0, qdt=qdt), qdt)
+    gold = attention64(f16_to_f64(q, qdt), np.swapaxes(f16_to_f64(k, qdt), -1, -2), f16_to_f64(v, qdt), 1.0, None, False, 1)
+    off, own = np.linalg.norm(got - gold), np.linalg.norm(f16_to_f64(f16(gold, qdt), qdt) - gold)
+    print("[sdpa prefill] error %.3e, rounding alone %.3e" % (off / np.linalg.norm(gold), own / np.linalg.norm(gold)))
+    assert off <= 1.01 * own
