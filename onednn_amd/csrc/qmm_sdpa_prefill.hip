@@ -213,7 +213,7 @@ sdpa_prefill_kernel(const sdpa_params_t p) {
         for (int i = 0; i < 16; i++) oacc[d][i] = 0.f;
     v8h pb[2 * KB];
     float m_run = -INFINITY, l_run = 0.f;
-    bool have_p = false;
+    bool have_p = false, half = false;
 
     // ---- one slot of matrix work: the scores of tile t, then the values of t - 1
     auto scores = [&](auto par_tag) {
@@ -260,8 +260,7 @@ sdpa_prefill_kernel(const sdpa_params_t p) {
 #pragma unroll
             for (int i = 0; i < 16; i++) st[kb][i] = 0.f;
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < N; i++) {
+        auto product = [&](int i) {
             if (i < NS)
                 st[i % KB] = mma32<BF>(f[i % AHEAD], qf[i / KB], st[i % KB]);
             else
@@ -269,7 +268,12 @@ sdpa_prefill_kernel(const sdpa_params_t p) {
                         f[i % AHEAD], pb[(i - NS) / DC], oacc[(i - NS) % DC]);
             if (i + AHEAD < N) f[i % AHEAD] = fragment(i + AHEAD);
             __builtin_amdgcn_sched_barrier(0);
-        }
+        };
+#pragma unroll
+        for (int i = 0; i < N - 2 * DC; i++) product(i);
+        if (half) return;
+#pragma unroll
+        for (int i = N - 2 * DC; i < N; i++) product(i);
     };
 
     // ---- one slot of vector work: the probabilities of tile t
@@ -278,6 +282,9 @@ sdpa_prefill_kernel(const sdpa_params_t p) {
         load_v(t + 1);
         load_k(t + 2);
         have_p = wanted(t * KG + g);
+        // the tile's last 32 keys, hidden from every query of the wave, stay out of the
+        // products: probability 0 times a value that is not finite would be NaN
+        half = p.causal && key0 + 32 > q_wave + 31;
         if (have_p) {
             const bool edge = key0 + KT > p.S
                     || (p.causal && key0 + KT - 1 > q_wave) || !(sc2 > 0.f);

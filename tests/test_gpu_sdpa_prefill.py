@@ -140,3 +140,20 @@ def test_a_late_key_that_outweighs_the_rest(ctx, qdt):  # noqa: F811
     off, own = np.linalg.norm(got - gold), np.linalg.norm(f16_to_f64(f16(gold, qdt), qdt) - gold)
     print("[sdpa prefill] error %.3e, rounding alone %.3e" % (off / np.linalg.norm(gold), own / np.linalg.norm(gold)))
     assert off <= 1.01 * own
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bits", [0x7C00, 0x7E00], ids=["inf", "nan"])
+def test_values_past_a_block_of_32_keys_stay_out(ctx, D, bits):  # noqa: F811
+    """A causal mask hides the second 32 of a tile's 64 keys from a wave's 32 queries, whatever the values there hold
+    (rows of a cache that are not written yet): those queries' results are finite and the same."""
+    H, Qn, S = 2, 96, 160
+    say("sdpa prefill hidden block %d %x" % (D, bits))
+    r = np.random.default_rng(31)
+    q, k, v = (f16(r.standard_normal((1, H, n, D))) for n in (Qn, S, S))
+    for first in (32, 96):
+        want = run_sdpa(ctx, q, k, v, scale=0.125, causal=True)
+        bad = v.copy()
+        bad[:, :, first:] = bits
+        got = run_sdpa(ctx, q, k, bad, scale=0.125, causal=True)
+        assert (got[:, :, :first] == want[:, :, :first]).all()
