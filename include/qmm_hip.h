@@ -250,6 +250,12 @@ QMM_API size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc);
 QMM_API int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc,
         const qmm_sdpa_args_t *args, void *hip_stream);
 
+/* Whether attention over more than 16 queries without an explicit mask takes the
+ * kernel of many queries (1), with dense rows of head_size, or its sizes leave it to
+ * the other one (0). Both carry the same implementation name; this tells them apart. */
+QMM_API int qmm_sdpa_pipelined(int head_size, int causal, int64_t heads, int64_t kv_heads,
+        int64_t queries, int64_t keys, int cache_8bit);
+
 /* ---- kernel-selection overrides ----
  * For A/B measurements and for tests that must reach a particular kernel at
  * sizes the oracle finishes quickly. Environment variables, read once when a

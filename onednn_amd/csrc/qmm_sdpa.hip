@@ -10,7 +10,8 @@
 // queries and for f32 scales / s32 zero points.
 //
 // Many queries without an explicit mask at head sizes 64 and 128 run on the kernel of
-// qmm_sdpa_prefill.hip (an 8-bit cache from 257 queries on); the rest here.
+// qmm_sdpa_prefill.hip where the keys are enough (an 8-bit cache from 257 queries on); the
+// rest here.
 //
 // The scores never leave the CU. A workgroup owns 128 queries of one head (four
 // waves of 32) and walks the keys 32 at a time:

@@ -506,18 +506,40 @@ sdpa_dequant_kernel(const sdpa_params_t p, int D, int kv1, uint16_t *K, uint16_t
 
 } // namespace
 
-// Whether the kernel takes a problem: wherever it can, it was the faster one at every
-// size tried (see the top); byte offsets inside a head have 32 bits here. An 8-bit cache
-// is dequantized into the scratchpad first (up to 256 MiB of it), from 257 queries on: a
-// second launch and the scratchpad's order cost 8 us, dequantizing while staging once per
-// 128 queries (us, there / here, s8, f16: 32 heads x 200 of 64 13.9 / 17.3, 32 x 130 of
-// 128 15.5 / 17.6, 8 x 300 of 128 26.8 / 19.9, 4 x 500 of 64 25.9 / 19.2, 16 over 4 K / V
-// heads x 1005 of 128 79.4 / 29.4, 32 x 2048 175 / 67).
+// Keys from which the kernel beats that of qmm_sdpa.hip. Its workgroups of eight waves
+// take longer to start and to merge, two fit a CU at head size 64 and one at 128, and
+// what they gain is the shorter walk: alone on a CU one wins from 97 keys on (causal 33;
+// 8 heads x 512, us, there / here: 64 keys of 128 7.9 / 8.2, 128 10.3 / 9.2, 700 32.7 /
+// 17.0), with n of them to a CU only from a longer walk on, since the other kernel's
+// small workgroups then hide each other's latency. Head size 64: 512 workgroups x 320
+// keys 16.2 / 17.2, x 512 22.4 / 21.0; 768 x 640 35.4 / 35.6; 1024 x 512 38.2 / 40.7,
+// x 1024 64.9 / 63.2; 2048 x 1024 119.7 / 124.0, x 2048 226.4 / 218.8; causal, 256 heads
+// x 256 13.7 / 16.8, 512 x 512 50.7 / 72.1, 64 x 2048 70.8 / 67.3, 128 x 2048 127.1 /
+// 134.9, x 4096 470 / 462. Head size 128: 512 x 256 22.5 / 23.5, x 400 30.4 / 30.3;
+// 1024 x 512 61.0 / 61.9, x 640 72.6 / 70.4; 2048 x 700 149.9 / 157.1, x 1024 206 / 199;
+// causal, 256 heads x 512 46.7 / 61.5, 128 x 700 40.0 / 47.0, 64 x 1400 65.3 / 57.8,
+// 256 x 2048 461 / 461, 128 x 4096 802 / 724. bf16 alike.
+static bool walk_is_long(const sdpa_params_t &p, int D) {
+    const int64_t n = ((int64_t)p.B0 * p.B1 * ((p.Qn + 127) / 128) + 255) / 256;
+    const double S = p.causal ? std::min(p.S, p.Qn) : p.S;
+    if (n <= 1) return S > (p.causal ? 32 : 96);
+    // the mean over the workgroups
+    const double walk = p.causal ? S * (1 - S / (2.0 * p.Qn)) + 64 : S;
+    if (D == 64) return walk > (n == 2 ? (p.causal ? 264 : 420) : std::min(1800.0, 275.0 * n - 250));
+    return walk > (n == 2 ? 315 : n == 3 ? 570 : std::min(1000.0, 120.0 * n + 100));
+}
+
+// Byte offsets inside a head have 32 bits here. An 8-bit cache is dequantized into the
+// scratchpad first (up to 256 MiB of it), from 257 queries on: a second launch and the
+// scratchpad's order cost 8 us, dequantizing while staging once per 128 queries (us,
+// there / here, s8, f16: 32 heads x 200 of 64 13.9 / 17.3, 32 x 130 of 128 15.5 / 17.6,
+// 8 x 300 of 128 26.8 / 19.9, 4 x 500 of 64 25.9 / 19.2, 16 over 4 K / V heads x 1005 of
+// 128 79.4 / 29.4, 32 x 2048 175 / 67).
 bool sdpa_prefill_takes(const sdpa_params_t &p, int D) {
     if ((D != 64 && D != 128) || p.mask_dt != dt_undef || p.Qn <= 16) return false;
     if (p.kv_dt == (p.bf ? dt_bf16 : dt_f16))
         return (int64_t)p.S * p.k.row * 2 < (int64_t)1 << 31
-                && (int64_t)p.S * p.v.row * 2 < (int64_t)1 << 31;
+                && (int64_t)p.S * p.v.row * 2 < (int64_t)1 << 31 && walk_is_long(p, D);
     const int64_t heads = (int64_t)(p.B0 / p.kv_div0) * (p.B1 / p.kv_div1);
     return p.Qn > 256 && heads <= 65535 && heads * p.S * D * 4 <= (int64_t)256 << 20;
 }
@@ -564,3 +586,22 @@ bool sdpa_prefill_launch(
 }
 
 } // namespace qmm
+
+extern "C" int qmm_sdpa_pipelined(int head_size, int causal, int64_t heads, int64_t kv_heads,
+        int64_t queries, int64_t keys, int cache_8bit) {
+    const int64_t top = 1 << 30;
+    if (heads < 1 || kv_heads < 1 || heads > top || heads % kv_heads || queries < 1
+            || queries > top || keys < 1 || keys > top)
+        return 0;
+    qmm::sdpa_params_t p = {};
+    p.B0 = p.kv_div0 = 1;
+    p.B1 = (int32_t)heads;
+    p.kv_div1 = (int32_t)(heads / kv_heads);
+    p.Qn = (int32_t)queries;
+    p.S = (int32_t)keys;
+    p.causal = causal;
+    p.mask_dt = qmm::dt_undef;
+    p.kv_dt = cache_8bit ? qmm::dt_s8 : qmm::dt_f16;
+    p.k.row = p.v.row = head_size;
+    return qmm::sdpa_prefill_takes(p, head_size);
+}

@@ -44,6 +44,16 @@ def test_ends_of_tiles(ctx, case, qdt):  # noqa: F811
     check(got, q, k, v, qdt, 0.125, causal, H // KV)
 
 
+@pytest.mark.parametrize("qdt", [dt.f16, dt.bf16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("case", [
+    # the sizes at which one kernel takes over from the other: 96 and 97 keys (causal 32 and 33) with at most one
+    # workgroup to a CU, and one head more than 256 workgroups
+    (2, 2, 40, 96, 128, False), (2, 1, 40, 97, 128, False), (2, 2, 33, 32, 64, True), (2, 2, 33, 33, 64, True),
+    (256, 8, 20, 40, 64, True), (257, 257, 20, 40, 64, True), (130, 13, 300, 420, 64, False), (130, 13, 300, 421, 64, False)], ids=str)
+def test_either_side_of_the_rule(ctx, case, qdt):  # noqa: F811
+    test_ends_of_tiles(ctx, case, qdt)
+
+
 @pytest.mark.parametrize("scale", [-0.125, 4.0], ids=str)
 def test_scales_that_are_not_the_usual(ctx, scale):  # noqa: F811
     """A negative scale (the maximum of the raw products is not that of the scores); scores far apart, so that the
