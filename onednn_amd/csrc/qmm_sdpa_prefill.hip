@@ -519,29 +519,38 @@ sdpa_dequant_kernel(const sdpa_params_t p, int D, int kv1, uint16_t *K, uint16_t
 // 1024 x 512 61.0 / 61.9, x 640 72.6 / 70.4; 2048 x 700 149.9 / 157.1, x 1024 206 / 199;
 // causal, 256 heads x 512 46.7 / 61.5, 128 x 700 40.0 / 47.0, 64 x 1400 65.3 / 57.8,
 // 256 x 2048 461 / 461, 128 x 4096 802 / 724. bf16 alike.
-static bool walk_is_long(const sdpa_params_t &p, int D) {
+//
+// An 8-bit cache is dequantized into the scratchpad first, from 257 queries on: a second
+// launch and the scratchpad's order cost 8 us, dequantizing while staging, which the
+// other kernel does once per 128 queries, more the more keys there are (us, there / here,
+// s8, f16). Head size 64: 8 heads x 300 queries x 64 keys 7.0 / 13.9, x 256 14.6 / 15.3,
+// x 300 17.6 / 16.8; causal, 128 heads x 400 24.3 / 25.2, x 600 38.2 / 33.7, 256 x 600
+// 48.2 / 57.9, x 900 92.0 / 102, x 2048 319 / 297, 64 x 4096 queries x 384 67.9 / 74.2,
+// x 512 85.0 / 84.3. Head size 128: 32 over 8 heads x 300 x 64 10.1 / 17.7, x 150 17.1 /
+// 19.2, x 200 21.4 / 19.7, x 4096 343 / 67; 64 x 4096 x 128 72.8 / 76.0, x 256 116 / 93.9.
+static bool walk_is_long(const sdpa_params_t &p, int D, bool dequant) {
     const int64_t n = ((int64_t)p.B0 * p.B1 * ((p.Qn + 127) / 128) + 255) / 256;
     const double S = p.causal ? std::min(p.S, p.Qn) : p.S;
-    if (n <= 1) return S > (p.causal ? 32 : 96);
     // the mean over the workgroups
     const double walk = p.causal ? S * (1 - S / (2.0 * p.Qn)) + 64 : S;
+    if (dequant) {
+        if (D == 128) return walk > 160;
+        return n <= 1 ? S > 280 : walk > std::min(p.causal ? 800.0 : 500.0, 70.0 * n + 150);
+    }
+    if (n <= 1) return S > (p.causal ? 32 : 96);
     if (D == 64) return walk > (n == 2 ? (p.causal ? 264 : 420) : std::min(1800.0, 275.0 * n - 250));
     return walk > (n == 2 ? 315 : n == 3 ? 570 : std::min(1000.0, 120.0 * n + 100));
 }
 
-// Byte offsets inside a head have 32 bits here. An 8-bit cache is dequantized into the
-// scratchpad first (up to 256 MiB of it), from 257 queries on: a second launch and the
-// scratchpad's order cost 8 us, dequantizing while staging once per 128 queries (us,
-// there / here, s8, f16: 32 heads x 200 of 64 13.9 / 17.3, 32 x 130 of 128 15.5 / 17.6,
-// 8 x 300 of 128 26.8 / 19.9, 4 x 500 of 64 25.9 / 19.2, 16 over 4 K / V heads x 1005 of
-// 128 79.4 / 29.4, 32 x 2048 175 / 67).
+// byte offsets inside a head have 32 bits here; at most 256 MiB of scratchpad
 bool sdpa_prefill_takes(const sdpa_params_t &p, int D) {
     if ((D != 64 && D != 128) || p.mask_dt != dt_undef || p.Qn <= 16) return false;
     if (p.kv_dt == (p.bf ? dt_bf16 : dt_f16))
         return (int64_t)p.S * p.k.row * 2 < (int64_t)1 << 31
-                && (int64_t)p.S * p.v.row * 2 < (int64_t)1 << 31 && walk_is_long(p, D);
+                && (int64_t)p.S * p.v.row * 2 < (int64_t)1 << 31 && walk_is_long(p, D, false);
     const int64_t heads = (int64_t)(p.B0 / p.kv_div0) * (p.B1 / p.kv_div1);
-    return p.Qn > 256 && heads <= 65535 && heads * p.S * D * 4 <= (int64_t)256 << 20;
+    return p.Qn > 256 && heads <= 65535 && heads * p.S * D * 4 <= (int64_t)256 << 20
+            && walk_is_long(p, D, true);
 }
 
 size_t sdpa_prefill_scratch(const sdpa_params_t &p, int D) {

@@ -105,9 +105,11 @@ def test_infinite_values_stay_with_the_queries_that_see_them(ctx):  # noqa: F811
 
 
 @pytest.mark.parametrize("kv_dt,sdt,zdt", [(dt.s8, dt.f16, dt.s8), (dt.u8, dt.f16, dt.u8), (dt.s8, dt.f16, None), (dt.s8, dt.f32, dt.s32)], ids=str)
-@pytest.mark.parametrize("Qn,S,D,qdt", [(257, 100, 128, dt.f16), (300, 301, 64, dt.bf16), (260, 65, 64, dt.f16)], ids=str)
+@pytest.mark.parametrize("Qn,S,D,qdt", [(257, 100, 128, dt.f16), (300, 301, 64, dt.bf16), (260, 65, 64, dt.f16),
+                                        (257, 195, 128, dt.f16), (390, 281, 64, dt.f16), (290, 333, 128, dt.bf16)], ids=str)
 def test_8_bit_cache_under_many_queries(ctx, Qn, S, D, qdt, kv_dt, sdt, zdt):  # noqa: F811
-    """The cache is written in the queries' type to the scratchpad first: the oracle's reorder gives the same values."""
+    """From 161 keys a workgroup (head size 64: 281) on the cache is written in the queries' type to the scratchpad first:
+    the oracle's reorder gives the same values."""
     MB, H, KV = 2, 4, 2
     say("sdpa prefill 8-bit cache %r" % ((Qn, S, D, qdt, kv_dt, sdt, zdt),))
     r = np.random.default_rng(Qn + D)

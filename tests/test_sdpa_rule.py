@@ -44,6 +44,24 @@ def test_keys_from_which_the_pipelined_kernel_takes_16_bit_values(D, causal, hea
     assert pipelined(D, causal, heads, queries, keys) == taken
 
 
+@pytest.mark.parametrize("D,causal,heads,kv,queries,keys,taken", [
+    (64, 0, 8, 8, 256, 4096, False), (128, 0, 32, 8, 257, 16, False),  # 8.3 / 18.1
+    (64, 0, 8, 8, 300, 256, False),  # 14.6 / 15.3
+    (64, 0, 8, 8, 300, 300, True),  # 17.6 / 16.8
+    (64, 1, 128, 32, 400, 400, False),  # 24.3 / 25.2
+    (64, 1, 128, 32, 600, 600, True),  # 38.2 / 33.7
+    (64, 1, 256, 64, 900, 900, False),  # 92 / 102
+    (64, 0, 64, 8, 4096, 384, False),  # 67.9 / 74.2
+    (64, 0, 64, 8, 4096, 512, True),  # 85.0 / 84.3
+    (128, 0, 32, 8, 300, 150, False),  # 17.1 / 19.2
+    (128, 0, 32, 8, 300, 200, True),  # 21.4 / 19.7
+    (128, 0, 64, 8, 4096, 128, False),  # 72.8 / 76.0
+    (128, 1, 8, 8, 257, 257, True),  # 24.1 / 18.3
+])
+def test_keys_from_which_an_8_bit_cache_is_dequantized_first(D, causal, heads, kv, queries, keys, taken):
+    assert pipelined(D, causal, heads, queries, keys, kv, True) == taken
+
+
 def test_fewer_keys_than_queries():
     # a causal mask over fewer keys: most workgroups walk all of them
     assert not pipelined(64, 1, 64, 4096, 256) and pipelined(64, 1, 64, 8192, 2560)
