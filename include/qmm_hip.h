@@ -239,14 +239,18 @@ typedef struct {
     void *dst;
     const void *mask, *scale;
     const void *k_scale, *k_zp, *v_scale, *v_zp;
-    void *scratch; /* qmm_sdpa_scratch_size() bytes, or NULL when 0 */
+    void *scratch; /* qmm_sdpa_scratch_size() bytes, or NULL: see there */
 } qmm_sdpa_args_t;
 
 QMM_API int qmm_sdpa_supports(const qmm_sdpa_desc_t *desc);
 QMM_API const char *qmm_sdpa_impl_name(const qmm_sdpa_desc_t *desc);
-/* Bytes of scratch a launch needs: non-zero only for at most 16 queries with
- * enough keys to be cut into several ranges (partial results per range). */
+/* Bytes of scratch for a launch. At most 16 queries with enough keys to be cut into
+ * several ranges: the ranges' partial results, without which the launch fails
+ * (qmm_sdpa_needs_scratch() is 1). Many queries and keys of an 8-bit cache: the cache in
+ * 16 bits; without it the launch
+ * dequantizes while it stages the keys, which takes longer. */
 QMM_API size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc);
+QMM_API int qmm_sdpa_needs_scratch(const qmm_sdpa_desc_t *desc);
 QMM_API int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc,
         const qmm_sdpa_args_t *args, void *hip_stream);
 

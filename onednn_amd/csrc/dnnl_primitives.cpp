@@ -1505,12 +1505,22 @@ dnnl_status_t dnnl_primitive_create(
     }
     if (p->pd->kind == kind_sdpa && p->pd->scratch_bytes
             && p->pd->attr.scratchpad_mode == dnnl_scratchpad_mode_library) {
-        const dnnl_engine *eng = p->pd->engine;
-        if (eng->device < 0 || hipSetDevice(eng->device) != hipSuccess
-                || hipMalloc(&p->lib_scratch, p->pd->scratch_bytes)
-                        != hipSuccess) {
+        const int dev = p->pd->engine->device;
+        const bool needed = qmm_sdpa_needs_scratch(&p->pd->sd) != 0;
+        // one that only makes the launch faster is asked for, and done without where
+        // there is none to have; the attempt leaves a capture under way on this thread
+        // and the runtime's last error as they are
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (!needed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        const bool have = dev >= 0 && hipSetDevice(dev) == hipSuccess
+                && hipMalloc(&p->lib_scratch, p->pd->scratch_bytes) == hipSuccess;
+        if (!have) p->lib_scratch = nullptr;
+        if (!needed) {
+            if (!have) (void)hipGetLastError();
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+        } else if (!have) {
             delete p;
-            return eng->device < 0 ? dnnl_runtime_error : dnnl_out_of_memory;
+            return dev < 0 ? dnnl_runtime_error : dnnl_out_of_memory;
         }
     }
     *primitive = p;

@@ -1049,6 +1049,11 @@ size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc) {
     return (size_t)p.B0 * p.B1 * sp.nsplit * part_pitch(p.Qn, (int)D) * sizeof(float);
 }
 
+int qmm_sdpa_needs_scratch(const qmm_sdpa_desc_t *desc) {
+    sdpa_params_t p;
+    return desc && supported(*desc, &p) && p.Qn <= 16 && qmm_sdpa_scratch_size(desc) != 0;
+}
+
 int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
         void *hip_stream) {
     if (!desc || !args) return QMM_INVALID_ARGUMENTS;

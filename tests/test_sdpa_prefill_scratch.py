@@ -29,3 +29,26 @@ def test_room_for_the_cache(queries, keys, D, cache, masked, want):
     pd = dnnl.sdpa.primitive_desc(eng, q, kt, v, mask, dt.f16, q, False, 4, False, attr)
     md = pd.scratchpad_desc()
     assert (0 if md.is_zero() else md.get_size()) == (2 * 4 * keys * D * 2 if want else 0)
+
+
+def test_a_primitive_is_created_without_room_for_the_cache():
+    """The room only makes the launch faster: where it cannot be had (no device here, no memory elsewhere) the primitive
+    is created all the same. The ranges of few queries need theirs."""
+    eng = dnnl.engine(dnnl.engine.kind.gpu, 0)
+    T = lambda name: 2 + tag._plain.index(name)  # noqa: E731
+
+    def create(queries, keys, cache):
+        q = memory.desc([1, 8, queries, 64], dt.f16, T("abcd"))
+        pd = dnnl.sdpa.primitive_desc(eng, q, memory.desc([1, 8, 64, keys], cache, T("abdc")),
+                                      memory.desc([1, 8, keys, 64], cache, T("abcd")), None, dt.f16, q, False, 8, False)
+        return dnnl.sdpa(pd)
+
+    create(300, 400, dt.s8)
+    if eng_has_no_device():
+        with pytest.raises(dnnl.error):
+            create(1, 4096, dt.f16)
+
+
+def eng_has_no_device():
+    import torch
+    return not torch.cuda.is_available()
