@@ -182,6 +182,7 @@ struct pd_impl_t {
     dnnl_memory_desc sdpa_k, sdpa_v, sdpa_mask; // src = queries
     dnnl_prop_kind_t prop_kind = dnnl_forward_inference;
     size_t scratch_bytes = 0;
+    bool scratch_needed = true; // false: the launch is only faster with it
     // matmul whose descriptors hold DNNL_RUNTIME_DIM_VAL: no implementation is
     // chosen until execute sees the memory objects' own descriptors
     bool runtime = false;

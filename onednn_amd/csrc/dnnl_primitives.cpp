@@ -798,6 +798,12 @@ scratch_guard_t::~scratch_guard_t() {
 }
 
 namespace {
+bool is_capturing(void *hip_stream) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hip_stream && hipStreamIsCapturing((hipStream_t)hip_stream, &cs) == hipSuccess
+            && cs != hipStreamCaptureStatusNone;
+}
+
 // Holds the guard's mutex from before the launch until the event behind it is
 // recorded. A stream under capture is left alone (an event recorded outside the
 // capture cannot be waited for inside it): whoever captures orders the launches.
@@ -806,12 +812,8 @@ struct scratch_order_t {
     hipStream_t stream = nullptr;
     bool active = false;
     scratch_order_t(scratch_guard_t *guard, void *hip_stream) {
-        if (!guard) return;
+        if (!guard || is_capturing(hip_stream)) return;
         stream = (hipStream_t)hip_stream;
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (stream && hipStreamIsCapturing(stream, &cs) == hipSuccess
-                && cs != hipStreamCaptureStatusNone)
-            return;
         g = guard;
         g->mu.lock();
         active = true;
@@ -1463,6 +1465,7 @@ dnnl_status_t sdpa_primitive_desc_create(dnnl_primitive_desc_t *out,
     pd->impl = 0;
     pd->impl_name = qmm_sdpa_impl_name(&S);
     pd->scratch_bytes = qmm_sdpa_scratch_size(&S);
+    pd->scratch_needed = qmm_sdpa_needs_scratch(&S) != 0;
     if (pd->scratch_bytes
             && pd->attr.scratchpad_mode == dnnl_scratchpad_mode_user) {
         dnnl_dims_t dims = {(int64_t)pd->scratch_bytes};
@@ -1506,7 +1509,7 @@ dnnl_status_t dnnl_primitive_create(
     if (p->pd->kind == kind_sdpa && p->pd->scratch_bytes
             && p->pd->attr.scratchpad_mode == dnnl_scratchpad_mode_library) {
         const int dev = p->pd->engine->device;
-        const bool needed = qmm_sdpa_needs_scratch(&p->pd->sd) != 0;
+        const bool needed = p->pd->scratch_needed;
         // one that only makes the launch faster is asked for, and done without where
         // there is none to have; the attempt leaves a capture under way on this thread
         // and the runtime's last error as they are
@@ -1660,6 +1663,11 @@ dnnl_status_t dnnl_primitive_execute(const_dnnl_primitive_t primitive,
         A.v_zp = handle(DNNL_ARG_ATTR_ZERO_POINTS | DNNL_ARG_VALUES);
         A.scratch = pd.scratchpad.ndims ? handle(DNNL_ARG_SCRATCHPAD)
                                         : lib_scratch;
+        // graphs of one primitive may run side by side, and after it is gone: they only
+        // hold the library's scratchpad where the launch cannot do without
+        if (A.scratch && A.scratch == lib_scratch && !pd.scratch_needed
+                && is_capturing(stream->hip_stream))
+            A.scratch = nullptr;
         scratch_order_t order(
                 A.scratch && A.scratch == lib_scratch ? guard : nullptr,
                 stream->hip_stream);

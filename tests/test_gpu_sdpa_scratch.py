@@ -61,3 +61,35 @@ def test_a_user_scratchpad_or_none(ctx, given):  # noqa: F811
     dnnl.sdpa(p.pd).execute(ctx[1], p.args)
     ctx[1].wait()
     p.check("given" if given else "none")
+
+
+def test_graphs_of_one_primitive_side_by_side(ctx):  # noqa: F811
+    """Two graphs recorded from one primitive in library mode, with operands of their own, replayed at the same time on two
+    streams after the primitive is gone: neither holds the library's scratchpad."""
+    import gc
+    import torch
+    say("sdpa graphs side by side")
+    probs = [Problem(ctx, seed, dnnl.scratchpad_mode.library) for seed in (5, 6)]
+    prim = dnnl.sdpa(probs[0].pd)
+    prim.execute(ctx[1], probs[0].args)
+    ctx[1].wait()
+    probs[0].check("eager")
+    streams, graphs = [torch.cuda.Stream() for _ in probs], []
+    for p, s in zip(probs, streams):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            prim.execute(dnnl.stream(p.eng, hip_stream=s.cuda_stream), p.args)
+        graphs.append(g)
+    del prim
+    gc.collect()
+    for turn in range(4):
+        for p in probs:
+            p.out.write(np.full((1, H, Qn, D), 0x7E00, np.uint16))
+        torch.cuda.synchronize()
+        for g, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                for _ in range(20):
+                    g.replay()
+        torch.cuda.synchronize()
+        for i, p in enumerate(probs):
+            p.check("turn %d graph %d" % (turn, i))
