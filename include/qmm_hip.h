@@ -247,7 +247,7 @@ QMM_API const char *qmm_sdpa_impl_name(const qmm_sdpa_desc_t *desc);
 /* Bytes of scratch for a launch. At most 16 queries with enough keys to be cut into
  * several ranges: the ranges' partial results, without which the launch fails
  * (qmm_sdpa_needs_scratch() is 1). Many queries and keys of an 8-bit cache: the cache in
- * 16 bits; without it the launch
+ * 16 bits; without it (or where it does not start on a 16-byte boundary) the launch
  * dequantizes while it stages the keys, which takes longer. */
 QMM_API size_t qmm_sdpa_scratch_size(const qmm_sdpa_desc_t *desc);
 QMM_API int qmm_sdpa_needs_scratch(const qmm_sdpa_desc_t *desc);

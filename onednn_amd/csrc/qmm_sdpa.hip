@@ -1138,8 +1138,10 @@ int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc, const qmm_sdpa_args_t *args,
                     dim3(128), 0, (hipStream_t)hip_stream, p, D);
         return hipGetLastError() == hipSuccess ? QMM_OK : QMM_RUNTIME_ERROR;
     }
-    // (an 8-bit cache without the scratchpad it asks for: dequantized while staging)
-    if (sdpa_prefill_takes(p, D) && (args->scratch || !sdpa_prefill_scratch(p, D))) {
+    // (an 8-bit cache without the scratchpad it asks for, or with one that the kernels'
+    // 16-byte loads and stores cannot address: dequantized while staging)
+    const bool room = args->scratch && ((uintptr_t)args->scratch & 15) == 0;
+    if (sdpa_prefill_takes(p, D) && (room || !sdpa_prefill_scratch(p, D))) {
         if (!sdpa_prefill_launch(p, D, args->scratch, hip_stream)) return QMM_UNIMPLEMENTED;
         return hipGetLastError() == hipSuccess ? QMM_OK : QMM_RUNTIME_ERROR;
     }

@@ -47,7 +47,7 @@ class Problem:
         assert bad <= total * 0.0006
 
 
-@pytest.mark.parametrize("given", [False, True], ids=["none", "nan_filled"])
+@pytest.mark.parametrize("given", [False, True, "off"], ids=["none", "nan_filled", "off_the_boundary"])
 def test_a_user_scratchpad_or_none(ctx, given):  # noqa: F811
     import torch
     say("sdpa scratchpad %s" % given)
@@ -55,12 +55,14 @@ def test_a_user_scratchpad_or_none(ctx, given):  # noqa: F811
     md = p.pd.scratchpad_desc()
     assert md.get_size() == 2 * KV * S * D * 2
     if given:
-        buf = torch.full((md.get_size() // 2,), float("nan"), dtype=torch.float16, device="cuda")
+        buf = torch.full((md.get_size() // 2 + 8,), float("nan"), dtype=torch.float16, device="cuda")
         torch.cuda.synchronize()
-        p.args[dnnl.DNNL_ARG_SCRATCHPAD] = memory(md, p.eng, buf.data_ptr())
+        p.args[dnnl.DNNL_ARG_SCRATCHPAD] = memory(md, p.eng, buf.data_ptr() + (2 if given == "off" else 0))
     dnnl.sdpa(p.pd).execute(ctx[1], p.args)
     ctx[1].wait()
-    p.check("given" if given else "none")
+    p.check(str(given))
+    if given:
+        assert torch.isnan(buf).all() if given == "off" else not torch.isnan(buf[:-8]).any()
 
 
 def test_graphs_of_one_primitive_side_by_side(ctx):  # noqa: F811
