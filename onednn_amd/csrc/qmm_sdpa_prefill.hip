@@ -38,6 +38,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "qmm_plan.hpp"
 #include "qmm_sdpa.hpp"
 
 namespace qmm {
@@ -583,6 +584,7 @@ bool sdpa_prefill_launch(
     }
     const int lds = 8 / QW * 4 * KT * D * 2 + 2048;
     auto go = [&](auto kern) {
+        ensure_dynamic_lds((const void *)kern, lds);
         hipLaunchKernelGGL(kern, grid, dim3(512), lds, (hipStream_t)hip_stream, p);
     };
     if (D == 128)
