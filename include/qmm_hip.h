@@ -254,6 +254,11 @@ QMM_API int qmm_sdpa_needs_scratch(const qmm_sdpa_desc_t *desc);
 QMM_API int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc,
         const qmm_sdpa_args_t *args, void *hip_stream);
 
+/* The first row (upper 32 bits) and the block of 32 columns (lower) that a workgroup of the
+ * streaming int8 / fp8 kernel works on, more than 32 rows; -1: it has none. Workgroup w
+ * runs on XCD w % 8. */
+QMM_API int64_t qmm_gemv_b8_block(int64_t M, int64_t N, int64_t workgroup);
+
 /* Whether attention over more than 16 queries without an explicit mask takes the
  * kernel of many queries (1), with dense rows of head_size, or its sizes leave it to
  * the other one (0). Both carry the same implementation name; this tells them apart. */

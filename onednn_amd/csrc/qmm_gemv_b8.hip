@@ -55,6 +55,33 @@ QMM_D int bits(T v) {
     return __builtin_bit_cast(int, v);
 }
 
+// Column block and first row of a workgroup, more than 32 rows. Workgroup w runs on XCD
+// w % 8. Whole groups of 8 column blocks: one to an XCD, its row blocks one after
+// another, close in time and on one L2. The last 0 ... 7: every XCD takes an eighth of
+// their blocks in order (s8, us, a column to an XCD there too / so: 43008 x 4096 x 32 191
+// / 46.3, 16384 x 4096 x 64 68.2 / 25.4, 2000 x 4096 x 288 22.5 / 18.0; all columns in
+// order, an eighth to an XCD, reads them from places far apart: fp8 33 x 4096 x 32768 39.9
+// / 47.3). False: nothing left for it.
+__host__ __device__ inline int gb8_grid(int M, int nb32) {
+    const int nrb = (M + 31) / 32;
+    return nrb * (nb32 / 8 * 8) + (nrb * (nb32 % 8) + 7) / 8 * 8;
+}
+__host__ __device__ inline bool gb8_block(int M, int nb32, int w, int &nb, int &m0) {
+    const int nrb = (M + 31) / 32, whole = nb32 / 8 * 8;
+    int rb;
+    if (w < nrb * whole) {
+        nb = w / (8 * nrb) * 8 + w % 8;
+        rb = w / 8 % nrb;
+    } else {
+        w -= nrb * whole;
+        const int item = w % 8 * ((nrb * (nb32 - whole) + 7) / 8) + w / 8;
+        nb = whole + item / nrb;
+        rb = item % nrb;
+    }
+    m0 = rb * 32;
+    return nb < nb32;
+}
+
 // What a thread adds up and stores: four neighbouring columns of one row, so that a
 // block of 32 columns is one pass of the workgroup and everything the epilogue reads
 // per row and column is requested before the waves meet. red: the waves' results,
@@ -132,15 +159,8 @@ gemv_b8_kernel(const gemm_params_t p) {
     auto red_rs = [&](int w, int r) -> int & {
         return ((int *)(lds_raw + w * WAVE_LDS))[MR * 32 + r];
     };
-    // column block and first row. A column block's row blocks are 8 workgroups apart:
-    // on one XCD, close in time, so that its weights come from memory once
-    const int nrb = QUADS ? (p.M + 31) / 32 : 1;
     int nb = blockIdx.x, m0 = 0;
-    if (nrb > 1) {
-        nb = blockIdx.x / (8 * nrb) * 8 + blockIdx.x % 8;
-        m0 = blockIdx.x / 8 % nrb * 32;
-        if (nb >= p.nb32) return;
-    }
+    if (QUADS && p.M > 32 && !gb8_block(p.M, p.nb32, blockIdx.x, nb, m0)) return;
     const int rows = p.M - m0;
     const uint8_t *const A = p.A + (int64_t)m0 * p.lda;
     // the wave's fragments (32 k each): an even cut of the K / 32 that hold data
@@ -447,8 +467,7 @@ void launch_gemv_b8(const gemm_params_t &p, bool f8, hipStream_t stream) {
                 kern, dim3((unsigned)blocks), dim3(GB8_WAVES * 64), lds, stream, p);
     };
     constexpr int lds4 = GB8_WAVES * gb8_wave_lds(4), lds32 = GB8_WAVES * gb8_wave_lds(32);
-    const int64_t nrb = (p.M + 31) / 32;
-    const int64_t grid32 = nrb > 1 ? (p.nb32 + 7) / 8 * 8 * nrb : p.nb32;
+    const int64_t grid32 = p.M > 32 ? gb8_grid((int)p.M, p.nb32) : p.nb32;
     if (p.M <= 4)
         f8 ? go(gemv_b8_kernel<4, true, false>, p.nb32, lds4)
            : go(gemv_b8_kernel<4, false, false>, p.nb32, lds4);
@@ -466,3 +485,12 @@ void launch_gemv_b8(const gemm_params_t &p, bool f8, hipStream_t stream) {
 }
 
 } // namespace qmm
+
+extern "C" int64_t qmm_gemv_b8_block(int64_t M, int64_t N, int64_t workgroup) {
+    int nb = 0, m0 = 0;
+    if (M <= 32 || M > 1 << 20 || N < 1 || N > 1 << 20 || workgroup < 0
+            || workgroup >= qmm::gb8_grid((int)M, (int)((N + 31) / 32))
+            || !qmm::gb8_block((int)M, (int)((N + 31) / 32), (int)workgroup, nb, m0))
+        return -1;
+    return (int64_t)m0 << 32 | nb;
+}
