@@ -56,29 +56,33 @@ QMM_D int bits(T v) {
 }
 
 // Column block and first row of a workgroup, more than 32 rows. Workgroup w runs on XCD
-// w % 8. Whole groups of 8 column blocks: one to an XCD, its row blocks one after
-// another, close in time and on one L2. The last 0 ... 7: every XCD takes an eighth of
-// their blocks in order (s8, us, a column to an XCD there too / so: 43008 x 4096 x 32 191
-// / 46.3, 16384 x 4096 x 64 68.2 / 25.4, 2000 x 4096 x 288 22.5 / 18.0; all columns in
-// order, an eighth to an XCD, reads them from places far apart: fp8 33 x 4096 x 32768 39.9
-// / 47.3). False: nothing left for it.
-__host__ __device__ inline int gb8_grid(int M, int nb32) {
+// w % 8. A column block's row blocks go to one XCD, one after another: close in time and
+// on one L2. With many of them (an XCD has 32 CUs) the columns past the last whole group
+// of 8 would leave XCDs idle: there every XCD takes an eighth of their blocks (s8, us, one
+// XCD a column / so: 43008 x 4096 x 32 191 / 46.3, 16384 x 4096 x 64 68.2 / 25.4, 2000 x
+// 4096 x 288 22.5 / 18.0; with few row blocks the other way, 226 x 8192 x 2055 25.0 / 29.4).
+// False: nothing left for it.
+struct gb8_map_t {
+    int nrb, whole, share; // row blocks; columns of whole groups; rest of an XCD, or 0
+};
+__host__ __device__ inline gb8_map_t gb8_map(int M, int nb32) {
     const int nrb = (M + 31) / 32;
-    return nrb * (nb32 / 8 * 8) + (nrb * (nb32 % 8) + 7) / 8 * 8;
+    return {nrb, nb32 / 8 * 8, nrb >= 32 ? (nrb * (nb32 % 8) + 7) / 8 : 0};
+}
+__host__ __device__ inline int gb8_grid(int M, int nb32) {
+    const gb8_map_t g = gb8_map(M, nb32);
+    return g.share ? g.nrb * g.whole + 8 * g.share : g.nrb * ((nb32 + 7) / 8 * 8);
 }
 __host__ __device__ inline bool gb8_block(int M, int nb32, int w, int &nb, int &m0) {
-    const int nrb = (M + 31) / 32, whole = nb32 / 8 * 8;
-    int rb;
-    if (w < nrb * whole) {
-        nb = w / (8 * nrb) * 8 + w % 8;
-        rb = w / 8 % nrb;
-    } else {
-        w -= nrb * whole;
-        const int item = w % 8 * ((nrb * (nb32 - whole) + 7) / 8) + w / 8;
-        nb = whole + item / nrb;
-        rb = item % nrb;
+    const gb8_map_t g = gb8_map(M, nb32);
+    nb = w / (8 * g.nrb) * 8 + w % 8;
+    m0 = w / 8 % g.nrb * 32;
+    if (g.share && nb >= g.whole) {
+        w -= g.nrb * g.whole;
+        const int item = w % 8 * g.share + w / 8;
+        nb = g.whole + item / g.nrb;
+        m0 = item % g.nrb * 32;
     }
-    m0 = rb * 32;
     return nb < nb32;
 }
 

@@ -6,19 +6,23 @@ import pytest
 from onednn_amd import _capi
 
 
-@pytest.mark.parametrize("M,N", [(33, 1), (64, 32), (1024, 33), (16384, 64), (43008, 32), (97, 257), (300, 4096), (200, 1000), (1000, 225)])
-def test_every_xcd_takes_an_eighth_of_the_blocks(M, N):
+def blocks(M, N):
     lib = _capi.lib()
     rows, cols = (M + 31) // 32, (N + 31) // 32
-    per_xcd, seen = collections.Counter(), set()
-    for w in range(8 * ((rows * cols + 7) // 8)):
-        b = lib.qmm_gemv_b8_block(M, N, w)
-        if b >= 0:
-            seen.add((b >> 32, b & 0xffffffff))
-            per_xcd[w % 8] += 1
-    assert seen == {(32 * r, c) for r in range(rows) for c in range(cols)} and sum(per_xcd.values()) == rows * cols
-    assert max(per_xcd.values()) == (rows * cols + 7) // 8
-    assert lib.qmm_gemv_b8_block(M, N, 8 * ((rows * cols + 7) // 8)) == -1
+    end = rows * (cols // 8 * 8 + 8)
+    found = [(w, lib.qmm_gemv_b8_block(M, N, w)) for w in range(end)]
+    assert lib.qmm_gemv_b8_block(M, N, end) == -1
+    return [(w, b >> 32, b & 0xffffffff) for w, b in found if b >= 0]
+
+
+@pytest.mark.parametrize("M,N", [(33, 1), (64, 32), (1024, 33), (16384, 64), (43008, 32), (97, 257), (300, 4096), (200, 1000),
+                                 (992, 225), (993, 225), (2000, 288)])
+def test_every_block_once(M, N):
+    found = blocks(M, N)
+    assert sorted((r, c) for _, r, c in found) == [(r, c) for r in range(0, M, 32) for c in range((N + 31) // 32)]
+    per_xcd = collections.Counter(w % 8 for w, _, _ in found)
+    if M > 992:  # 32 row blocks and more: every XCD an eighth
+        assert max(per_xcd.values()) == (len(found) + 7) // 8
 
 
 def test_blocks_of_a_column_share_an_xcd():
