@@ -254,6 +254,12 @@ QMM_API int qmm_sdpa_needs_scratch(const qmm_sdpa_desc_t *desc);
 QMM_API int qmm_sdpa_launch(const qmm_sdpa_desc_t *desc,
         const qmm_sdpa_args_t *args, void *hip_stream);
 
+/* Rows of the tiles in which hip:gfx950:mfma_b8 works on `batch` M x N x K problems of s8
+ * or f8_e4m3 operands with packed weights, without overrides: 32 the streaming kernel, 64,
+ * 128 or 256 the tiled ones; 0: not one of theirs. */
+QMM_API int qmm_gemm_b8_tile(int src_dt, int64_t batch, int64_t M, int64_t N, int64_t K,
+        int post_ops);
+
 /* The first row (upper 32 bits) and the block of 32 columns (lower) that a workgroup of the
  * streaming int8 / fp8 kernel works on, more than 32 rows; -1: it has none. Workgroup w
  * runs on XCD w % 8. */

@@ -30,7 +30,7 @@ void launch_quantize_rows(const quant_rows_params_t &p, hipStream_t stream);
 void launch_quantize_transpose(const quant_tr_params_t &p, hipStream_t stream);
 void launch_w4a8_prep(const w4a8_prep_t &p, hipStream_t stream);
 void launch_gemv_b8(const gemm_params_t &p, bool f8, hipStream_t stream);
-bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256);
+bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256, bool post_ops);
 void launch_gemm_f16(const gemm16_params_t &p, hipStream_t stream);
 void launch_rowsum_b8(const void *src, int32_t *dst, int64_t batch, int64_t M,
         int64_t K, int64_t lda, int64_t a_sb, bool a_is_u8, const void *src_zp,
@@ -1129,7 +1129,7 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
                 && ((!f8 && P.M <= 64)
                         || (plan->b8x_variant == 1 && !plan->measure
                                 && gemv_b8_takes(P.M, P.N, P.K, f8,
-                                        gemm_b8_uses_tile256(g, f8, 0))))) {
+                                        gemm_b8_uses_tile256(g, f8, 0), D.npo > 0)))) {
             if (b8_needs_rowsum(D)) {
                 const qmm_quant_t &wz = D.zps[QMM_WEI];
                 g.wei_zp = wz.set ? args->zps[QMM_WEI] : nullptr;

@@ -513,6 +513,14 @@ bool gemm_b8_uses_tile256(const gemm_params_t &p, bool f8, int variant) {
     return tiles128 >= 32 && (rows_full || tiles128 >= 96);
 }
 
+// by size: small problems: more, smaller tiles keep more CUs busy
+// (fp8 on 256 x 128: 88.5 instead of 58.4 us, 2048 x 4096 x 4096)
+static int tile_variant(const gemm_params_t &p, bool f8) {
+    const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 127) / 128) * p.batch;
+    const int64_t mid = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+    return big >= 256 && !f8 ? 1 : (mid >= 64 ? 2 : 3);
+}
+
 void launch_gemm_b8(const gemm_params_t &p, bool f8, int variant,
         hipStream_t stream) {
     if (p.M <= 0 || p.N <= 0 || p.batch <= 0) return;
@@ -521,21 +529,39 @@ void launch_gemm_b8(const gemm_params_t &p, bool f8, int variant,
         return;
     }
     if (variant == 6) variant = 0;
-    if (variant == 0) {
-        const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 127) / 128)
-                * p.batch;
-        const int64_t mid = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128)
-                * p.batch;
-        // small problems: more, smaller tiles keep more CUs busy
-        // (fp8 on 256 x 128: 88.5 instead of 58.4 us, 2048 x 4096 x 4096)
-        variant = big >= 256 && !f8 ? 1 : (mid >= 64 ? 2 : 3);
-    }
+    if (variant == 0) variant = tile_variant(p, f8);
     switch (variant) {
         case 1: launch_gemm_b8_v1(p, f8, stream); break;
         case 3: launch_gemm_b8_v3(p, f8, stream); break;
         default: launch_gemm_b8_v2(p, f8, stream); break;
     }
 }
+
+bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256, bool post_ops);
 #endif
 
 } // namespace qmm
+
+#if !defined(QMM_GEMM_VARIANT)
+extern "C" int qmm_gemm_b8_tile(
+        int src_dt, int64_t batch, int64_t M, int64_t N, int64_t K, int post_ops) {
+    using namespace qmm;
+    const int64_t top = 1 << 24;
+    const bool f8 = src_dt == dt_f8_e4m3;
+    if ((!f8 && src_dt != dt_s8) || batch < 1 || M < 1 || N < 1 || K < 16 || K % 16
+            || batch > top || M > top || N > top || K > top)
+        return 0;
+    gemm_params_t p = {};
+    p.M = (int32_t)M;
+    p.N = (int32_t)N;
+    p.K = (int32_t)K;
+    p.lda = K;
+    p.batch = (int32_t)batch;
+    p.kb32 = (int32_t)((K + 31) / 32);
+    const bool tile256 = gemm_b8_uses_tile256(p, f8, 0);
+    if (batch == 1 && (!f8 || K % 64 == 0) && gemv_b8_takes(M, N, K, f8, tile256, post_ops))
+        return 32;
+    if (tile256) return 256;
+    return 256 >> (tile_variant(p, f8) - 1);
+}
+#endif

@@ -454,11 +454,28 @@ gemv_b8_rows64_kernel(const gemm_params_t p) {
 // 12.4 / 11.7 (1024), 70 x 1024 x 16384 17.5 / 18.1 (1536), 300 x 1024 x 3072 23.5 / 11.6 (960).
 // f8_e4m3 (tiled / here): 256 x 1024 x 1024 12.8 / 7.1, 512 x 4096 x 4096 43.5 / 35.5
 // (2048), 1024 x 2048 x 2048 31.9 / 27.7 (2048), 919 x 1152 x 1664 22.8 / 23.9 (1508),
-// 2048 x 1024 x 1024 23.0 / 26.7 (2048), 700 x 14336 x 2048 85.0 / 94.6 (1408).
-bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256) {
+// 2048 x 1024 x 1024 23.0 / 26.7 (2048), 700 x 14336 x 2048 85.0 / 94.6 (1408), 100 x 4096 x
+// 16384 37.7 / 36.8 (2048), 100 x 6144 x 16384 46.0 / 55.9, 200 x 6144 x 8192 45.5 / 46.3 (1792).
+//
+// Against 64 x 64 tiles (fewer than 64 tiles of 128 x 128 and not the 256-row kernels),
+// which keep every CU at one workgroup and take 10.4 / 11.8 / 13.0 / 19.7 / 32 us at K =
+// 1024 / 1536 / 2048 / 4096 / 8192: up to 512 workgroups here always (7.7 at 256 x 1024 x
+// 2048); up to 768 past K = 1024 (256 x 2816, with a swish 11.4 / 11.6 / 11.9 / 16.5 / 26.1);
+// above that with no post-op to walk and between (226 x 3552 11.6 / 12.1 / 12.8 / 18.3 / 31,
+// with a swish 12.9 / 13.5 / 14.3 / 19.1 / 31.8; 128 x 8000 36.6 at 8192).
+// f8_e4m3, 33 ... 64 rows (tiles / here): 33 x 4096 x 16384 31.1 / 22.9 (1024), 64 x 14336 x
+// 16384 97.8 / 73.7, 64 x 8192 x 24576 69.1 / 62.2 (1536), 33 x 14336 x 24576 97.8 / 114,
+// 33 x 4096 x 32768 34.6 / 41.5 (2048), 64 x 8192 x 65536 118.7 / 166.9.
+bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256, bool post_ops) {
     const int64_t wgs = (M + 31) / 32 * ((N + 31) / 32);
-    if (M <= 64) return true;
-    if (f8) return wgs <= (K >= 8192 ? 1024 : K >= 2048 ? 2048 : 1344);
+    if (M <= (f8 ? 32 : 64)) return true;
+    if (M <= 64) return wgs <= (K > 8192 ? 1024 : 1536);
+    if (!tile256 && (M + 127) / 128 * ((N + 127) / 128) < 64) {
+        if (wgs <= 512) return true;
+        if (wgs <= 768) return K > 1024;
+        return !f8 && !post_ops && K >= 2048 && K < 8192;
+    }
+    if (f8) return wgs <= (K >= 8192 ? 1024 : K > 4096 ? 1536 : K >= 2048 ? 2048 : 1344);
     return wgs <= (K >= 2048 ? 1344 : tile256 ? 960 : 1024);
 }
 
