@@ -489,17 +489,29 @@ bool gemm_b8_uses_tile256(const gemm_params_t &p, bool f8, int variant) {
     const int64_t tm = (p.M + 255) / 256;
     const int64_t tiles256 = tm * ((p.N + 255) / 256) * p.batch;
     if (tiles256 >= 192) return true;
-    // fp8 with fewer tiles: time against time. Measured (us, into a bf16 residual): one
-    // round of 256 x 256 tiles 23 / 32 / 46 / 75 / 120 at K = 1024 / 2048 / 4096 / 8192 /
-    // 14336, about 20 more where columns end inside a wave's 128; 128 x 128 tiles 26 / 35
-    // / 45 / 60 / 87 while every CU has one at most, 58 / 83 (4096 / 8192) with two
-    // (2048 x 4096 x 4096 58.4 / 49.6, 512 x 14336 x 4096 86.6 / 119.8, 1100 x 2048 x 4000
-    // 48.0 / 55.3)
+    // fp8 with fewer tiles: time against time (us, into a bf16 residual, K = 1024 / 2048 /
+    // 4096 / 8192). 256 x 256 tiles, one round: 23 / 31 / 46 / 75, about 20 more where
+    // columns end inside a wave's 128 (less with fewer rows: 1100 x 4000 47.6 / 56 / 70 /
+    // 100), up to 9 where rows end inside its 64 (1000 x 8192 30.3 / 38.0 / 52.7 / 82.2).
+    // 128 x 128 tiles: one to a CU 23.4 / 30 / 39 / 55 (512 x 8192), 1.1 ... 2 25.1 / 31.2 /
+    // 43.4 / 68.2 (1100 x 4096) ... 29.7 / 36.0 / 51.5 / 83.2 (2048 x 4096), three 33.4 / 43.8
+    // / 66.3 / 125 (700 x 14336); with one row of tiles no weights are found in L2 (100 x
+    // 43008 26.9 / 33.5 / 62 / 110, here 28.2 / 35.5 / 56.8 / 98). Fewer than 64 of them are
+    // worse than 64 x 64 tiles, which beat both (2 x 128 x 1024 9.5 / 12.8 / 18.8, here 21.6 /
+    // 28.6 / 43). Batches were measured up to 16 with whole rows (8 x 64 x 1024, K 512: 19.1 /
+    // 14.6, 16 x 64 x 4096 25.1 / 19.3); more of them run a second round of workgroups (40 x
+    // 256 x 512 25.8 / 40.8, 64 x 200 x 256 24.6 / 44.0).
     if (f8) {
+        const int64_t mid = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
+        if (mid < 64 || (p.batch > 1 && (p.batch > 16 || p.M % 64))) return false;
         const double k = p.K / 1024.0;
-        const double mid = (double)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;
-        const double t128 = (mid <= 256 ? 22 + 5 * k : 33 + 6.2 * k) * (mid > 512 ? mid / 512 : 1);
-        return 16 + 7.3 * k + (p.N % 128 ? 20 : 0) < t128;
+        const double per_cu = mid <= 256 ? 1
+                : mid > 512              ? 3
+                : p.M <= 128             ? 2
+                                         : 1.35 + 0.65 * (double)(mid - 256) / 256;
+        const double t128 = 17 + 2 * per_cu + k * (1 + 3.3 * per_cu);
+        const double edge = p.N % 128 ? 0.08 * std::min(p.M, 256) : 0.15 * (p.M % 64);
+        return 15.5 + 7.4 * k + edge < t128;
     }
     // int8 with an s8 source also has the 256 x 128 kernel with two workgroups
     // per CU, which beats the tiles below from 32 such tiles on, unless the row
@@ -514,7 +526,9 @@ bool gemm_b8_uses_tile256(const gemm_params_t &p, bool f8, int variant) {
 }
 
 // by size: small problems: more, smaller tiles keep more CUs busy
-// (fp8 on 256 x 128: 88.5 instead of 58.4 us, 2048 x 4096 x 4096)
+// (fp8 never on 256 x 128, 128 x 128 tiles / these, us: 2048 x 4096 x 4096 58.4 / 88.5, and
+// where the 256 x 256 kernels do not take K: 4096 x 256 x 4096 42.9 / 54.3, 8192 x 1088 x 4096
+// 86 / 127, 4096 x 4160 x 14336 320 / 378; only QMM_GEMM_VARIANT reaches it)
 static int tile_variant(const gemm_params_t &p, bool f8) {
     const int64_t big = (int64_t)((p.M + 255) / 256) * ((p.N + 127) / 128) * p.batch;
     const int64_t mid = (int64_t)((p.M + 127) / 128) * ((p.N + 127) / 128) * p.batch;

@@ -50,6 +50,41 @@ def test_fp8_few_results(M, K, N, want):
     assert tile(dt.f8_e4m3, M, K, N) == want
 
 
+@pytest.mark.parametrize("batch,M,K,N,want", [
+    # tiles of 128 (below 64 of them: 64) / 256 x 256
+    (2, 128, 512, 1024, 64),  # 8.2 / 18.0
+    (2, 128, 2048, 1024, 64),  # 12.8 / 28.6
+    (32, 128, 1024, 128, 64),  # 9.2 / 19.7
+    (3, 500, 1024, 520, 64),  # 10.8 / 48.2
+    (8, 16, 512, 1024, 128),  # 9.6 / 14.6
+    (64, 200, 512, 256, 128),  # 24.6 / 44.0
+    (40, 256, 1024, 512, 128),  # 31.7 / 49.8
+    (4, 500, 2048, 2048, 128),  # 30.4 / 39.8
+    (8, 64, 512, 1024, 256),  # 19.1 / 14.6
+    (12, 384, 2048, 1024, 256),  # 43.5 / 33.3
+    (16, 64, 2048, 4096, 256),  # 41.6 / 37.8
+    (8, 128, 4096, 1024, 128),  # 37.8 / 44.4
+    # one matrix
+    (1, 1500, 4096, 3000, 128),  # 42.4 / 67.0
+    (1, 512, 8192, 8192, 128),  # 55.2 / 75.3
+    (1, 1024, 4096, 4096, 128),  # 38.9 / 45.9
+    (1, 2048, 4096, 4096, 256),  # 51.5 / 47.4
+    (1, 1152, 1024, 6144, 256),  # 26.9 / 24.0
+    (1, 1000, 2048, 6144, 128),  # 32.5 / 37.3
+    (1, 700, 8192, 14336, 256),  # 124.8 / 87.7
+    (1, 1746, 2048, 5856, 128),  # 44.0 / 52.7
+    (1, 1746, 8192, 5856, 256),  # 113.2 / 96.8
+    (1, 100, 8192, 43008, 256),  # 110.5 / 98.3
+    (1, 33, 2048, 32768, 128),  # 23.6 / 30.7
+    (1, 256, 1024, 2816, 64),  # 9.8, streaming 11.7
+    (1, 256, 2048, 2816, 32),  # 12.6, streaming 11.8
+    (1, 256, 2048, 3584, 64),  # 12.6, streaming 13.6
+    (1, 8192, 8192, 8192, 256),
+])
+def test_fp8_tiles(batch, M, K, N, want):
+    assert tile(dt.f8_e4m3, M, K, N, batch) == want
+
+
 def test_other_arguments_take_nothing():
     assert tile(dt.f32, 64, 64, 64) == 0 and tile(dt.s8, 0, 64, 64) == 0 and tile(dt.s8, 64, 40, 64) == 0
 

@@ -94,6 +94,27 @@ def test_fp8_into_a_residual(ctx, M, K, N, dst):
     fp8_sum(ctx, M, K, N, M + N, dst)
 
 
+@pytest.mark.parametrize("B,M,K,N", [(8, 64, 512, 1024), (2, 130, 384, 257), (3, 33, 512, 64), (20, 64, 512, 640)])
+def test_fp8_batches(ctx, B, M, K, N):
+    """The default choice on either side of its lines: 256 x 256 tiles, 64 x 64 ones, more batches than the former take."""
+    import torch
+    from onednn_amd import memory
+    eng, strm = ctx
+    print("[case] fp8 batches %d %d %d %d" % (B, M, K, N), flush=True)
+    g = torch.Generator().manual_seed(B + M)
+    a, b = (torch.randint(-3, 4, s, generator=g).float() for s in ((B, M, K), (B, K, N)))  # (sums below 2^24: exact)
+    T = lambda name: 2 + memory.format_tag._plain.index(name)  # noqa: E731
+    f8 = lambda x: x.to(torch.float8_e4m3fn).view(torch.uint8).numpy()  # noqa: E731
+    mds = [memory.desc(d, t, T("abc")) for d, t in (([B, M, K], dt.f8_e4m3), ([B, K, N], dt.f8_e4m3), ([B, M, N], dt.f32))]
+    pd = dnnl.matmul.primitive_desc(eng, *mds)
+    out = memory(mds[2], eng)
+    dnnl.matmul(pd).execute(strm, {dnnl.DNNL_ARG_SRC: memory(mds[0], eng).write(f8(a)),
+                                   dnnl.DNNL_ARG_WEIGHTS: memory(mds[1], eng).write(f8(b)), dnnl.DNNL_ARG_DST: out})
+    strm.wait()
+    got = torch.from_numpy(out.read(np.float32, (B, M, N)).copy())
+    assert (got == torch.bmm(a, b)).all()
+
+
 @pytest.mark.parametrize("variant", [2, 3, 6])
 @pytest.mark.parametrize("M,K,N,dst", [(300, 512, 520, dt.bf16), (255, 384, 257, dt.bf16), (190, 640, 390, dt.f32),
                                        (64, 384, 130, dt.f32), (449, 512, 513, dt.f32)], ids=str)
