@@ -265,6 +265,11 @@ QMM_API int qmm_gemm_b8_tile(int src_dt, int64_t batch, int64_t M, int64_t N, in
  * runs on XCD w % 8. */
 QMM_API int64_t qmm_gemv_b8_block(int64_t M, int64_t N, int64_t workgroup);
 
+/* Whether more than 16 rows of f16 / bf16 activations under 4- or 8-bit weights run on the
+ * tiled kernel (1) or on the decode kernel once per 16 rows (0), where one of these takes
+ * them (hip:gfx950:decode_w4). */
+QMM_API int qmm_gemm_w4f_tiled(int src_dt, int weights_bits, int64_t M, int64_t N, int64_t K);
+
 /* Whether attention over more than 16 queries without an explicit mask takes the
  * kernel of many queries (1), with dense rows of head_size, or its sizes leave it to
  * the other one (0). Both carry the same implementation name; this tells them apart. */

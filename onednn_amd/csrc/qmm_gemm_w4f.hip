@@ -382,24 +382,39 @@ void launch_gemm_w4f_part2(const gemv_params_t &, int, int, hipStream_t);
 void launch_gemm_w4f_part3(const gemv_params_t &, int, int, hipStream_t);
 
 // Whether the tiled kernel is the better way to run p.M > 16 rows, against the
-// decode kernel once per block of 16 rows. Measured (us, f16 x u4): a round of
-// 128-column workgroups of 32 rows 10.5 / 15.7 / 26 / 47 at K = 1024 / 2048 / 4096 /
-// 8192, of 64 rows 15.4 / 21.9 / 36 / 64; a pass of the decode kernel over 4096 columns
-// 4.3 up to K = 4096 (what is left of a short K is its start and end), 7.8 at 8192. Decode
-// kernel / tiled: 100 x 1024 x 4096 30.0 / 15.4, 20 x 1024 x 10576 22.6 / 10.6, 232 x 1024
-// x 1280 23.2 / 15.1, 100 x 1024 x 1280 13.5 / 15.4, 100 x 8192 x 4096 54.4 / 64.1; u8
-// weights alike (100 x 1024 x 4096 34.3 / 18.3).
+// decode kernel once per block of 16 rows: rounds of 256 workgroups, priced by what one
+// takes. Measured (us, f16 x u4, K = 1024 / 4096 / 8192 / 14336). Tiled, 128 columns: 32
+// rows 10.2 / 26 / 48 / 82, 64 rows 15.3 / 36 / 64 / 106; bf16 11.1 / 27.5 / 50 / 84 and
+// 17.5 / 42.5 / 76 / 127; u8 weights 12.9 / 36 / 66 / 112 and 18.2 / 48 / 88 / 148; a
+// begun round costs a whole one (32 x 8192 x 43008 96.5). Decode kernel: K counts in
+// steps of 4096, 512 for each of its 8 waves (100 x 4096 x K, seven rounds: 29.7
+// at 1024, 29.4 at 3584, 53.8 at 4608, 53.5 at 8192, 79.3 at 10240, 105 at 14336; of two column
+// blocks 27.4 / 29.3 / 49.3 / 86.2 at 50 x K x 8192, of four 58.2 / 61.4 / 87 / 146 for 64 x K x
+// 16384; u8 33.5 / 36.5 / 68.5 / 129); a few workgroups past a round run beside the
+// others (17 x 8192 x 12304 40.6). Decode / tiled where the choice is close: 20 x 12288, K
+// = 4096 30.3 / 26.3, 7168 42.1 / 43.5, 8192 41.8 / 48.6; 50 x 8192, K = 2048 27.3 / 22.3, 4096
+// 29.3 / 36.3, 5120 48.8 / 43.3, 8192 49.3 / 64.5; 100 x 4096, K = 2048 29.5 / 22.1, 4096 29.1 /
+// 35.9, 4608 53.8 / 39.5, 8192 53.5 / 63.9; u8 20 x 4096 x 12288 29.0 / 35.9, 100 x 4096 x 4096
+// 36.5 / 47.9. Over 470 shapes of 512 ... 20480 k the choice is the faster kernel or within 8 %
+// of it.
 bool gemm_w4f_wins(const gemv_params_t &p) {
     if (p.M <= 16) return false;
     const int64_t wide = (int64_t)((p.M + 63) / 64) * ((p.N + 255) / 256);
     if (p.M > 64 && wide >= 128) return true;
     const int bm = p.M <= 32 ? 32 : 64;
     const double k = p.K / 1024.0;
-    const double wgs = (double)((p.M + bm - 1) / bm) * ((p.N + 127) / 128);
-    const double rounds = wgs <= 256 ? 1.0 : wgs / 256;
-    const double tiled = (bm == 32 ? 5.3 + 5.1 * k : 8.6 + 6.9 * k) * rounds;
-    const double passes = (double)((p.M + 15) / 16) * 4.3 * p.N / 4096.0 * (k > 4 ? k / 4 : 1);
-    return tiled < passes;
+    const int64_t wgs = (int64_t)((p.M + bm - 1) / bm) * ((p.N + 127) / 128);
+    const double round = p.w8 ? (bm == 32 ? 5.4 + 7.6 * k : 8.2 + 10 * k)
+            : p.act_f16       ? (bm == 32 ? 4.8 + 5.4 * k : 8.6 + 6.9 * k)
+                              : (bm == 32 ? 5.6 + 5.6 * k : 9.2 + 8.4 * k);
+    const int blocks = gemv_w4_column_blocks(p);
+    const int64_t dec_wgs = (int64_t)((p.M + 15) / 16) * (p.nb16 / blocks);
+    const int more = (p.K - 1) / 4096; // steps of K past the first
+    const double dec_round = p.w8 ? 5 + 4.3 * more
+            : blocks == 4         ? 15 + 7.5 * more
+            : blocks == 2         ? 7.3 + 4.9 * more
+                                  : 4.2 + 3.6 * more;
+    return (double)((wgs + 255) / 256) * round < (double)((dec_wgs + 240) / 256) * dec_round;
 }
 
 // more than 16 rows (the caller decides with gemm_w4f_wins), fast-variant
@@ -418,3 +433,21 @@ void launch_gemm_w4f(const gemv_params_t &p, int shifts, int flags_m,
 #endif
 
 } // namespace qmm
+
+#if !defined(QMM_W4F_PART)
+extern "C" int qmm_gemm_w4f_tiled(int src_dt, int weights_bits, int64_t M, int64_t N, int64_t K) {
+    using namespace qmm;
+    const int64_t top = 1 << 24;
+    if ((src_dt != dt_f16 && src_dt != dt_bf16) || (weights_bits != 4 && weights_bits != 8) || M < 1
+            || N < 1 || K < 1 || M > top || N > top || K > top)
+        return 0;
+    gemv_params_t p = {};
+    p.M = (int32_t)M;
+    p.N = (int32_t)N;
+    p.K = (int32_t)K;
+    p.nb16 = (int32_t)((N + 15) / 16);
+    p.act_f16 = src_dt == dt_f16;
+    p.w8 = weights_bits == 8;
+    return gemm_w4f_wins(p);
+}
+#endif

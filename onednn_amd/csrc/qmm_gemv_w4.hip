@@ -980,20 +980,11 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
         // stages its activations in LDS
         const bool staged = p.M > 8 && (int64_t)grid.x * grid.y <= 256;
         const int lds = staged ? GEMV_STAGE_BYTES : 0;
-        // two column blocks per workgroup where one block each would be more
-        // workgroups than the chip holds at once (two per CU)
-        // (5 .. 8 rows keep one block: with two, the 8-row form spills registers)
-        const bool two = !p.w8 && !staged && (p.nb16 & 1) == 0 && p.nb16 >= 512
-                && !(p.M > 4 && p.M <= 8);
-        // more than 8 rows: four blocks, for a quarter of the activation traffic
-        const bool four = two && p.M > 8 && (p.nb16 & 3) == 0 && p.nb16 >= 768;
+        const int blocks = staged ? 1 : gemv_w4_column_blocks(p);
         auto go = [&](auto kern) {
             if (lds) ensure_dynamic_lds((const void *)kern, lds);
             hipLaunchKernelGGL(kern,
-                    four       ? dim3(grid.x / 4, grid.y)
-                            : two ? dim3(grid.x / 2, grid.y)
-                                  : grid,
-                    dim3(GEMV_WAVES * 64), lds, stream, p.B,
+                    dim3(grid.x / blocks, grid.y), dim3(GEMV_WAVES * 64), lds, stream, p.B,
                     p.A, (const uint16_t *)p.scales, zp, p.kg128, p.N, p.K,
                     (int)p.lda, shifts, flags_m, q);
         };
@@ -1011,14 +1002,14 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
                 }
             }
             if constexpr (R == 16) {
-                if (four) {
+                if (blocks == 4) {
                     go(gemv_w4_fast_cb_kernel<F, R, S, 4>);
                     return;
                 }
             }
             if (p.w8)
                 go(gemv_w4_fast_kernel<F, R, S, true>);
-            else if (two)
+            else if (blocks == 2)
                 go(gemv_w4_fast_cb_kernel<F, R, S, 2>);
             else
                 go(gemv_w4_fast_kernel<F, R, S, false>);

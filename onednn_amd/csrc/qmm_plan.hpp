@@ -217,6 +217,14 @@ struct gemv_params_t {
     int32_t w8; // 8-bit weights, QMM_LAYOUT_MFMA_W8 (fast variant only)
     epilogue_t ep;
 };
+// blocks of 16 columns in a workgroup of the decode kernel (activations not staged):
+// several where one each would be more workgroups than the chip holds at once (two per
+// CU); 5 .. 8 rows keep one block, with two that form spills registers; more than 8 rows:
+// four, for a quarter of the activation traffic
+inline int gemv_w4_column_blocks(const gemv_params_t &p) {
+    if (p.w8 || p.nb16 % 2 || p.nb16 < 512 || (p.M > 4 && p.M <= 8)) return 1;
+    return p.M > 8 && p.nb16 % 4 == 0 && p.nb16 >= 768 ? 4 : 2;
+}
 
 // ---- s8 activations x 4-bit weights, K-grouped scales on both sides ---------
 // The scale / zero-point buffers are rewritten per launch into the scratchpad,
