@@ -21,9 +21,10 @@ def ctx():
 
 
 # M, K, N: one row past a block of 32 and of 64; columns that end inside a quad; fewer fragments than waves, a last
-# chunk of one; one past 8 column blocks (the XCD order's last, partial group)
+# chunk of one; one past 8 column blocks (the XCD order's last, partial group). The last: the kernel of 33 ... 64 rows over
+# more than 4096 columns where waves have no fragment
 SHAPES = [(33, 32, 33), (64, 224, 72), (65, 288, 64), (63, 2080, 4130), (96, 512, 257), (97, 1056, 290), (130, 256, 1001),
-          (256, 1024, 96), (40, 4096, 4128), (5, 224, 70)]
+          (256, 1024, 96), (40, 4096, 4128), (5, 224, 70), (63, 96, 4200)]
 
 
 @pytest.mark.parametrize("src", [dt.s8, dt.u8], ids=["s8", "u8"])
@@ -40,8 +41,10 @@ def test_blocks_of_rows_and_columns(ctx, monkeypatch, shape, src):
     assert_bit_exact(p.run_gpu(eng, strm, weights_any=True), want, "tiles")
 
 
-@pytest.mark.parametrize("M,K,N", [(70, 256, 98), (40, 512, 4200), (33, 96, 64), (40, 208, 72)])
+@pytest.mark.parametrize("M,K,N", [(70, 256, 98), (40, 512, 4200), (33, 96, 64), (40, 208, 72), (64, 208, 4130),
+                                   (33, 1040, 4130)])
 def test_post_ops_row_by_row(ctx, M, K, N):
+    """... and, with u8 sources, K that ends inside a fragment of 32."""
     eng, strm = ctx
     print("[case] stream post-ops %d %d %d" % (M, K, N), flush=True)
     p = cases.int8_linear(M, K, N, 3, post_ops=[{"kind": "eltwise", "alg": A.eltwise_relu, "alpha": 0.5},

@@ -23,11 +23,13 @@ def check(got, q, k, v, qdt, scale, causal, rep):
 
 CASES = [
     # heads, kv heads, queries, keys, D, causal: one tile and less; one row past the 32 queries of a wave and the 128
-    # of a workgroup; 32 / 64 / 128 keys and one more or less; fewer keys than queries and more
+    # of a workgroup; 32 / 64 / 128 keys and one more or less; fewer keys than queries and more. (The fewest keys are the
+    # other kernel's, see below.)
     (2, 2, 17, 1, 64, False), (2, 1, 31, 31, 128, True), (3, 3, 33, 64, 64, True), (2, 2, 32, 65, 128, False),
     (1, 1, 128, 127, 128, True), (4, 2, 129, 129, 64, True), (2, 2, 129, 400, 128, False), (2, 2, 300, 63, 128, True),
     (2, 2, 65, 192, 64, False), (2, 2, 257, 513, 64, True), (1, 1, 1100, 1100, 128, True), (2, 2, 600, 2305, 64, False),
-    # more query tiles than workgroups: two rounds, the second one backwards; a third, partial one
+    (2, 1, 17, 97, 64, False), (2, 2, 31, 128, 128, False), (2, 2, 32, 129, 64, False), (1, 1, 65, 65, 128, True),
+    # more workgroups than CUs: a second round, a partial third one
     (40, 8, 1000, 1000, 64, True), (40, 40, 1000, 130, 128, False), (100, 4, 700, 70, 64, True),
 ]
 
