@@ -36,8 +36,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int GB8_WAVES = 8;
 constexpr int GB8_CH = 16; // fragments in flight per wave
 
-// MR = 32 / 64 (one or two blocks of 32 rows against the same weights
-// fragments): the source bytes of a chunk go through a wave-private piece of LDS --
+// MR = 32: the source bytes of a chunk go through a wave-private piece of LDS --
 // requested as whole 256-byte row pieces (16 lanes a row, 4 rows an
 // instruction) instead of one 16-byte piece per lane out of 32 different rows
 // -- and come back in operand order. The same bytes hold the wave's results
@@ -45,9 +44,9 @@ constexpr int GB8_CH = 16; // fragments in flight per wave
 constexpr int GB8_CH32 = 8; // fragments per chunk with 32 rows
 constexpr int GB8_APITCH = GB8_CH32 * 32 + 16; // bytes of a staged row
 constexpr int gb8_wave_lds(int mr) { // >= mr x 32 s32 of results + row sums
-    return mr >= 32 ? mr * GB8_APITCH : (4 * 32 + 4) * 4;
+    return mr == 32 ? 32 * GB8_APITCH : (4 * 32 + 4) * 4;
 }
-static_assert(gb8_wave_lds(64) >= 64 * 32 * 4 + 64 * 4, "");
+static_assert(gb8_wave_lds(32) >= 32 * 32 * 4 + 32 * 4, "");
 
 // (by value: of a vector's element in place the builtin takes the first one's bits)
 template <typename T>
@@ -57,7 +56,8 @@ QMM_D int bits(T v) {
 
 // Column block and first row of a workgroup, more than 32 rows. Workgroup w runs on XCD
 // w % 8. A column block's row blocks go to one XCD, one after another: close in time and
-// on one L2. With many of them (an XCD has 32 CUs) the columns past the last whole group
+// on one L2 (counted there: 256 x 4096 x 4096 fetches 27.9 MB, 8.4 of them the rows once per
+// XCD, so its 16.8 MB of weights 1.1 times; 32 rows 18.3 MB in all). With many of them (an XCD has 32 CUs) the columns past the last whole group
 // of 8 would leave XCDs idle: there every XCD takes an eighth of their blocks (s8, us, one
 // XCD a column / so: 43008 x 4096 x 32 191 / 46.3, 16384 x 4096 x 64 68.2 / 25.4, 2000 x
 // 4096 x 288 22.5 / 18.0; with few row blocks the other way, 226 x 8192 x 2055 25.0 / 29.4).
@@ -150,8 +150,8 @@ template <int MR, bool F8, bool QUADS>
 __global__ void __launch_bounds__(GB8_WAVES * 64)
 gemv_b8_kernel(const gemm_params_t p) {
     typedef typename std::conditional<F8, v16f, v16i>::type acc_t;
-    constexpr int CH = MR >= 32 ? GB8_CH32 : GB8_CH;
-    constexpr int RB = MR >= 32 ? MR / 32 : 1; // blocks of 32 rows
+    static_assert(MR == 4 || MR == 32, "");
+    constexpr int CH = MR == 32 ? GB8_CH32 : GB8_CH;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds_raw[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -180,50 +180,37 @@ gemv_b8_kernel(const gemm_params_t p) {
     const bool need_rs = p.wei_zp != nullptr || p.w_off != 0;
     uint8_t *const stage = lds_raw + wave * WAVE_LDS;
 
-    acc_t acc[RB];
-    int rsum[RB];
+    acc_t acc;
+    int rsum = 0;
 #pragma unroll
-    for (int rb = 0; rb < RB; rb++) {
-        rsum[rb] = 0;
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[rb][r] = 0;
-    }
+    for (int r = 0; r < 16; r++) acc[r] = 0;
     for (int fb = f0; fb < f1; fb += CH) {
         v4u bq[CH];
-        uint4 av[RB][CH];
+        uint4 av[CH];
         // every request of the chunk before the first use; fragments past the
         // wave's end repeat its last one and are skipped below
-        if constexpr (MR >= 32) {
+        if constexpr (MR == 32) {
             // piece l % 16 of rows l / 16 + 4 i (K is a multiple of 16: a piece
             // is inside the row or past it)
             static_assert(CH == 8, "a block of 32 rows is 8 row quadruples");
             const int k = fb * 32 + (lane & 15) * 16;
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-                for (int i = 0; i < CH; i++) {
-                    const int r = min(32 * rb + 4 * i + (lane >> 4), rows - 1);
-                    av[rb][i] = *(const uint4 *)(A + (int64_t)r * p.lda
-                            + min(k, p.K - 16));
-                }
+            for (int i = 0; i < CH; i++) {
+                const int r = min(4 * i + (lane >> 4), rows - 1);
+                av[i] = *(const uint4 *)(A + (int64_t)r * p.lda + min(k, p.K - 16));
+            }
 #pragma unroll
             for (int j = 0; j < CH; j++)
                 bq[j] = __builtin_nontemporal_load(bsrc + (int64_t)min(fb + j, f1 - 1) * 64);
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++)
+            for (int i = 0; i < CH; i++)
+                *(uint4 *)(stage + (4 * i + (lane >> 4)) * GB8_APITCH + (lane & 15) * 16)
+                        = k >= p.K ? make_uint4(flip, flip, flip, flip) // zero after the flip
+                                   : av[i];
 #pragma unroll
-                for (int i = 0; i < CH; i++)
-                    *(uint4 *)(stage + (32 * rb + 4 * i + (lane >> 4)) * GB8_APITCH
-                            + (lane & 15) * 16)
-                            = k >= p.K ? make_uint4(flip, flip, flip, flip) // zero after the flip
-                                       : av[rb][i];
-#pragma unroll
-            for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-                for (int j = 0; j < CH; j++)
-                    av[rb][j] = *(const uint4 *)(stage
-                            + (32 * rb + (lane & 31)) * GB8_APITCH + j * 32
-                            + (lane >> 5) * 16);
+            for (int j = 0; j < CH; j++)
+                av[j] = *(const uint4 *)(stage + (lane & 31) * GB8_APITCH + j * 32
+                        + (lane >> 5) * 16);
         } else {
 #pragma unroll
             for (int j = 0; j < CH; j++) {
@@ -231,43 +218,33 @@ gemv_b8_kernel(const gemm_params_t p) {
                 bq[j] = __builtin_nontemporal_load(bsrc + (int64_t)f * 64);
                 // K is a multiple of 16: a half fragment is inside the row or past it
                 const int k = f * 32 + (lane >> 5) * 16;
-                av[0][j] = *(const uint4 *)(arow + min(k, p.K - 16));
-                if (k >= p.K) av[0][j] = make_uint4(flip, flip, flip, flip); // zero after the flip
+                av[j] = *(const uint4 *)(arow + min(k, p.K - 16));
+                if (k >= p.K) av[j] = make_uint4(flip, flip, flip, flip); // zero after the flip
             }
         }
 #pragma unroll
         for (int j = 0; j < CH; j += F8 ? 2 : 1) {
             if (fb + j < f1) {
                 if constexpr (F8) {
-#pragma unroll
-                    for (int rb = 0; rb < RB; rb++) {
-                        const uint4 a0 = av[rb][j], a1 = av[rb][j + 1];
-                        const v8i a = {(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w,
-                                (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
-                        const v8i b = {(int)bq[j].x, (int)bq[j].y, (int)bq[j].z,
-                                (int)bq[j].w, (int)bq[j + 1].x, (int)bq[j + 1].y,
-                                (int)bq[j + 1].z, (int)bq[j + 1].w};
-                        acc[rb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-                                a, b, acc[rb], 0, 0, 0, 0, 0, 0);
-                    }
-                    continue;
+                    const uint4 a0 = av[j], a1 = av[j + 1];
+                    const v8i a = {(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w,
+                            (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
+                    const v8i b = {(int)bq[j].x, (int)bq[j].y, (int)bq[j].z,
+                            (int)bq[j].w, (int)bq[j + 1].x, (int)bq[j + 1].y,
+                            (int)bq[j + 1].z, (int)bq[j + 1].w};
+                    acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                            a, b, acc, 0, 0, 0, 0, 0, 0);
                 } else {
-                const v4i b = {(int)bq[j].x, (int)bq[j].y, (int)bq[j].z,
-                        (int)bq[j].w};
-#pragma unroll
-                for (int rb = 0; rb < RB; rb++) {
-                    const v4i a = {(int)(av[rb][j].x ^ flip), (int)(av[rb][j].y ^ flip),
-                            (int)(av[rb][j].z ^ flip), (int)(av[rb][j].w ^ flip)};
+                    const v4i b = {(int)bq[j].x, (int)bq[j].y, (int)bq[j].z,
+                            (int)bq[j].w};
+                    const v4i a = {(int)(av[j].x ^ flip), (int)(av[j].y ^ flip),
+                            (int)(av[j].z ^ flip), (int)(av[j].w ^ flip)};
                     if (need_rs) {
-                        int t = rsum[rb];
-                        t = __builtin_amdgcn_sdot4(a[0], 0x01010101, t, false);
-                        t = __builtin_amdgcn_sdot4(a[1], 0x01010101, t, false);
-                        t = __builtin_amdgcn_sdot4(a[2], 0x01010101, t, false);
-                        t = __builtin_amdgcn_sdot4(a[3], 0x01010101, t, false);
-                        rsum[rb] = t;
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            rsum = __builtin_amdgcn_sdot4(a[q], 0x01010101, rsum, false);
                     }
-                    acc[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc[rb], 0, 0, 0);
-                }
+                    acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc, 0, 0, 0);
                 }
             }
         }
@@ -277,21 +254,15 @@ gemv_b8_kernel(const gemm_params_t p) {
     if constexpr (MR == 4) {
         if (lane < 32) {
 #pragma unroll
-            for (int r = 0; r < 4; r++) red(wave, r, lane) = bits(acc[0][r]);
+            for (int r = 0; r < 4; r++) red(wave, r, lane) = bits(acc[r]);
         }
     } else {
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++)
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-                red(wave, 32 * rb + 8 * (r / 4) + 4 * (lane >> 5) + r % 4, lane & 31)
-                        = bits(acc[rb][r]);
+        for (int r = 0; r < 16; r++)
+            red(wave, 8 * (r / 4) + 4 * (lane >> 5) + r % 4, lane & 31) = bits(acc[r]);
     }
-#pragma unroll
-    for (int rb = 0; rb < RB; rb++) {
-        const int tot = rsum[rb] + __shfl_xor(rsum[rb], 32);
-        if (lane < (MR < 32 ? MR : 32)) red_rs(wave, 32 * rb + lane) = tot;
-    }
+    const int tot = rsum + __shfl_xor(rsum, 32);
+    if (lane < MR) red_rs(wave, lane) = tot;
     const int tid = threadIdx.x;
     if constexpr (!QUADS) {
         __syncthreads();
@@ -335,8 +306,7 @@ gemv_b8_kernel(const gemm_params_t p) {
     }
 }
 
-// 33 ... 64 rows: a workgroup owns CB blocks of 32 columns, so that the source rows,
-// more bytes than the weights with one block, are fetched half as often with two.
+// 33 ... 64 rows over many columns: both blocks of 32 rows against the same weights.
 // A chunk is CH fragments of k: its source bytes, 128-byte row pieces, go through the
 // wave's piece of LDS, and the next chunk is requested before the products.
 __global__ void __launch_bounds__(GB8_WAVES * 64, 4)

@@ -89,7 +89,9 @@ QMM_D void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-template <int DC, int QW, int KT, bool BF>
+constexpr int QW = 4, KT = 64; // waves of a group, 32 queries each; keys of a tile
+
+template <int DC, bool BF>
 __global__ void __launch_bounds__(512, 2)
 sdpa_prefill_kernel(const sdpa_params_t p) {
     constexpr int D = 32 * DC, ROW = D * 2; // bytes of a row
@@ -561,7 +563,6 @@ size_t sdpa_prefill_scratch(const sdpa_params_t &p, int D) {
 
 bool sdpa_prefill_launch(
         const sdpa_params_t &p0, int D, void *scratch, void *hip_stream) {
-    constexpr int QW = 4, KT = 64;
     sdpa_params_t p = p0;
     const dim3 grid((unsigned)(p.B0 * p.B1), (unsigned)((p.Qn + 32 * QW - 1) / (32 * QW)));
     if (grid.y > 65535) return false;
@@ -588,11 +589,11 @@ bool sdpa_prefill_launch(
         hipLaunchKernelGGL(kern, grid, dim3(512), lds, (hipStream_t)hip_stream, p);
     };
     if (D == 128)
-        p.bf ? go(sdpa_prefill_kernel<4, QW, KT, true>)
-             : go(sdpa_prefill_kernel<4, QW, KT, false>);
+        p.bf ? go(sdpa_prefill_kernel<4, true>)
+             : go(sdpa_prefill_kernel<4, false>);
     else
-        p.bf ? go(sdpa_prefill_kernel<2, QW, KT, true>)
-             : go(sdpa_prefill_kernel<2, QW, KT, false>);
+        p.bf ? go(sdpa_prefill_kernel<2, true>)
+             : go(sdpa_prefill_kernel<2, false>);
     return true;
 }
 
