@@ -390,13 +390,14 @@ void launch_gemm_w4f_part3(const gemv_params_t &, int, int, hipStream_t);
 // steps of 4096, 512 for each of its 8 waves (100 x 4096 x K, seven rounds: 29.7
 // at 1024, 29.4 at 3584, 53.8 at 4608, 53.5 at 8192, 79.3 at 10240, 105 at 14336; of two column
 // blocks 27.4 / 29.3 / 49.3 / 86.2 at 50 x K x 8192, of four 58.2 / 61.4 / 87 / 146 for 64 x K x
-// 16384; u8 33.5 / 36.5 / 68.5 / 129); a few workgroups past a round run beside the
-// others (17 x 8192 x 12304 40.6). Decode / tiled where the choice is close: 20 x 12288, K
-// = 4096 30.3 / 26.3, 7168 42.1 / 43.5, 8192 41.8 / 48.6; 50 x 8192, K = 2048 27.3 / 22.3, 4096
-// 29.3 / 36.3, 5120 48.8 / 43.3, 8192 49.3 / 64.5; 100 x 4096, K = 2048 29.5 / 22.1, 4096 29.1 /
-// 35.9, 4608 53.8 / 39.5, 8192 53.5 / 63.9; u8 20 x 4096 x 12288 29.0 / 35.9, 100 x 4096 x 4096
-// 36.5 / 47.9. Over 470 shapes of 512 ... 20480 k the choice is the faster kernel or within 8 %
-// of it.
+// 16384; u8 33.5 / 36.5 / 68.5 / 129). A begun round counts whole there too, but a last
+// block of one to four rows reads less (M x 1408 x 4480, 17 / 18 / 20 / 24 / 30 rows: 10.7 /
+// 10.7 / 11.7 / 12.6 / 14.3). Decode / tiled where the choice is close: 20 x 12288, K = 4096
+// 30.3 / 26.3, 7168 42.1 / 43.5, 8192 41.8 / 48.6; 50 x 8192, K = 2048 27.3 / 22.3, 4096 29.3 /
+// 36.3, 5120 48.8 / 43.3, 8192 49.3 / 64.5; 100 x 4096, K = 2048 29.5 / 22.1, 4096 29.1 / 35.9,
+// 4608 53.8 / 39.5, 8192 53.5 / 63.9; u8 20 x 4096 x 12288 29.0 / 35.9, 100 x 4096 x 4096 36.5 /
+// 47.9. Over 720 shapes of 512 ... 20480 k the choice is the faster kernel or within 9 % of it
+// (one: 13 %), 0.2 % in the mean.
 bool gemm_w4f_wins(const gemv_params_t &p) {
     if (p.M <= 16) return false;
     const int64_t wide = (int64_t)((p.M + 63) / 64) * ((p.N + 255) / 256);
@@ -408,13 +409,16 @@ bool gemm_w4f_wins(const gemv_params_t &p) {
             : p.act_f16       ? (bm == 32 ? 4.8 + 5.4 * k : 8.6 + 6.9 * k)
                               : (bm == 32 ? 5.6 + 5.6 * k : 9.2 + 8.4 * k);
     const int blocks = gemv_w4_column_blocks(p);
-    const int64_t dec_wgs = (int64_t)((p.M + 15) / 16) * (p.nb16 / blocks);
+    const int64_t row_wgs = p.nb16 / blocks, dec_wgs = (int64_t)((p.M + 15) / 16) * row_wgs;
+    const int last = p.M % 16;
+    const double light = last == 0 || last > 4 ? 0. : last > 2 ? 0.15 : 0.45;
     const int more = (p.K - 1) / 4096; // steps of K past the first
     const double dec_round = p.w8 ? 5 + 4.3 * more
             : blocks == 4         ? 15 + 7.5 * more
             : blocks == 2         ? 7.3 + 4.9 * more
                                   : 4.2 + 3.6 * more;
-    return (double)((wgs + 255) / 256) * round < (double)((dec_wgs + 240) / 256) * dec_round;
+    const double dec_rounds = (double)((dec_wgs + 255) / 256) - light * row_wgs / 256;
+    return (double)((wgs + 255) / 256) * round < dec_rounds * dec_round;
 }
 
 // more than 16 rows (the caller decides with gemm_w4f_wins), fast-variant

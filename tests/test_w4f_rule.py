@@ -33,8 +33,11 @@ def tiled(M, K, N, bits=4, src=dt.f16):
     (20, 14336, 16384, False),  # 72.9 / 82.8
     (20, 14336, 10240, False),  # 58.1 / 82.1
     (100, 14336, 5120, True),  # 135.5 / 106.0
-    # a few workgroups past a round; a second round of the tiled kernel
+    # a last block of few rows; a second round of the tiled kernel
     (17, 8192, 12304, False),  # 40.6 / 48.8
+    (18, 1408, 4480, False),  # 10.7 / 12.5
+    (24, 1408, 4480, True),  # 12.6 / 12.1
+    (33, 3840, 12336, True),  # 35.8 / 33.8
     (32, 8192, 43008, True),  # 132.7 / 96.5
     (24, 4096, 65536, True),  # 126.9 / 53.5
 ])
@@ -65,6 +68,8 @@ def test_4_bit_weights_under_bf16(M, K, N, want):
     (50, 8192, 8192, False),  # 74.2 / 88.6
     (100, 14336, 4096, False),  # 129 / 148
     (200, 11008, 3072, True),  # 144 / 116
+    (18, 3840, 12336, False),  # 31.2 / 34.5
+    (28, 3840, 12336, True),  # 36.1 / 34.1
 ])
 def test_8_bit_weights(M, K, N, want):
     assert tiled(M, K, N, 8) == want
