@@ -35,7 +35,7 @@ UNITS = [("qmm_generic.hip", "", []), ("qmm_gemv_w4.hip", "", PRELOAD),
          ("qmm_pack.hip", "", []), ("qmm_quantize.hip", "", []),
          ("qmm_dispatch.hip", "", []), ("qmm_measure.hip", "", PRELOAD), ("qmm_softmax.hip", "", []), ("qmm_sdpa.hip", "", []), ("qmm_sdpa_prefill.hip", "", []),
          ("qmm_gemm_b8.hip", "", []),
-         ("qmm_gemm_b8x.hip", "", []), ("qmm_gemm_w4a8.hip", "", []), ("qmm_gemv_b8.hip", "", []), ("qmm_gemm_w4f.hip", "", []), ("qmm_gemm_g128.hip", "", []), ("qmm_gemm_f16.hip", "", []),
+         ("qmm_gemm_b8x.hip", "", []), ("qmm_gemm_w4a8.hip", "", []), ("qmm_gemv_b8.hip", "", []), ("qmm_gemm_w4f.hip", "", []), ("qmm_gemm_w4k.hip", "", []), ("qmm_gemm_g128.hip", "", []), ("qmm_gemm_f16.hip", "", []),
          ("dnnl_core.cpp", "", []), ("dnnl_primitives.cpp", "", [])]
 # the tiled GEMM is instantiated once per tile configuration, each in its own
 # object so the instantiations compile in parallel
@@ -56,6 +56,9 @@ for v in (0, 1):
 # the tiled decompression kernel per activation type and weights width
 for v in (0, 1, 2, 3):
     UNITS.append(("qmm_gemm_w4f.hip", "_p%d" % v, ["-DQMM_W4F_PART=%d" % v]))
+# the kernel that cuts K over its waves, likewise
+for v in (0, 1, 2, 3):
+    UNITS.append(("qmm_gemm_w4k.hip", "_p%d" % v, ["-DQMM_W4K_PART=%d" % v]))
 # the tiled kernel for groups of 128 k: s8, f16 and bf16 activations
 for v in (0, 1, 2):
     UNITS.append(("qmm_gemm_g128.hip", "_p%d" % v, ["-DQMM_G128_PART=%d" % v]))

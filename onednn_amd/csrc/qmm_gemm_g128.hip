@@ -600,6 +600,16 @@ int gemm_g128_rows(int M, int N, int K, int kind) {
     }
     return c64 < ct ? 64 : tall;
 }
+// what that tile takes (5 us of start and end aside the groups)
+double gemm_g128_us(int M, int N, int K, int kind) {
+    const bool s8 = kind == G_S8;
+    const int64_t tn = ((int64_t)N + 255) / 256;
+    const int tall = s8 ? 128 : 96;
+    const int64_t t64 = ((int64_t)M + 63) / 64 * tn, tt = ((int64_t)M + tall - 1) / tall * tn;
+    const double us = s8 ? std::min(group_us(t64, 1.10, 1.45), group_us(tt, 1.75, 2.45))
+                         : std::min(group_us(t64, 1.75, 2.35), group_us(tt, 2.2, 2.7));
+    return 5.0 + K / 128 * us * (kind == G_BF16 ? 1.1 : 1.0);
+}
 #endif
 } // namespace qmm
 

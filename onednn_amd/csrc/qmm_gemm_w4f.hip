@@ -17,6 +17,7 @@
 //     the exponent of 16 * offset (P = sum a * (17 offset + w)).
 // One 16-bit scale and at most one byte-sized zero point per column and k tile
 // (group widths 128 << s or all of K), as in the decode kernel's fast variant.
+#include <algorithm>
 #include <type_traits>
 
 #include "qmm_device.hpp"
@@ -398,16 +399,16 @@ void launch_gemm_w4f_part3(const gemv_params_t &, int, int, hipStream_t);
 // 4608 53.8 / 39.5, 8192 53.5 / 63.9; u8 20 x 4096 x 12288 29.0 / 35.9, 100 x 4096 x 4096 36.5 /
 // 47.9. Over 720 shapes of 512 ... 20480 k the choice is the faster kernel or within 9 % of it
 // (one: 13 %), 0.2 % in the mean.
-bool gemm_w4f_wins(const gemv_params_t &p) {
-    if (p.M <= 16) return false;
-    const int64_t wide = (int64_t)((p.M + 63) / 64) * ((p.N + 255) / 256);
-    if (p.M > 64 && wide >= 128) return true;
+static double w4f_tiled_us(const gemv_params_t &p) {
     const int bm = p.M <= 32 ? 32 : 64;
     const double k = p.K / 1024.0;
     const int64_t wgs = (int64_t)((p.M + bm - 1) / bm) * ((p.N + 127) / 128);
     const double round = p.w8 ? (bm == 32 ? 5.4 + 7.6 * k : 8.2 + 10 * k)
             : p.act_f16       ? (bm == 32 ? 4.8 + 5.4 * k : 8.6 + 6.9 * k)
                               : (bm == 32 ? 5.6 + 5.6 * k : 9.2 + 8.4 * k);
+    return (double)((wgs + 255) / 256) * round;
+}
+static double w4f_decode_us(const gemv_params_t &p) {
     const int blocks = gemv_w4_column_blocks(p);
     const int64_t row_wgs = p.nb16 / blocks, dec_wgs = (int64_t)((p.M + 15) / 16) * row_wgs;
     const int last = p.M % 16;
@@ -418,7 +419,24 @@ bool gemm_w4f_wins(const gemv_params_t &p) {
             : blocks == 2         ? 7.3 + 4.9 * more
                                   : 4.2 + 3.6 * more;
     const double dec_rounds = (double)((dec_wgs + 255) / 256) - light * row_wgs / 256;
-    return (double)((wgs + 255) / 256) * round < dec_rounds * dec_round;
+    return dec_rounds * dec_round;
+}
+static int64_t w4f_wide(const gemv_params_t &p) { // 64 x 256 tiles
+    return (int64_t)((p.M + 63) / 64) * ((p.N + 255) / 256);
+}
+bool gemm_w4f_wins(const gemv_params_t &p) {
+    if (p.M <= 16) return false;
+    if (p.M > 64 && w4f_wide(p) >= 128) return true;
+    return w4f_tiled_us(p) < w4f_decode_us(p);
+}
+// What the kernel that gemm_w4f_wins picks takes. 64 x 256 tiles: 6 us and 1.75 (f16), 2.0
+// (bf16) or 2.6 (8-bit weights) per 128 k and round; over 230 shapes of 1024 ... 14336 k
+// within 16 % below and 25 % above, blocks of rows of the decode kernel up to 30 % below.
+double gemm_w4f_us(const gemv_params_t &p) {
+    if (p.M > 64 && w4f_wide(p) >= 128)
+        return (double)((w4f_wide(p) + 255) / 256)
+                * (6 + (p.w8 ? 2.6 : p.act_f16 ? 1.75 : 2.0) * p.kg128);
+    return std::min(w4f_tiled_us(p), 1.5 + w4f_decode_us(p));
 }
 
 // more than 16 rows (the caller decides with gemm_w4f_wins), fast-variant

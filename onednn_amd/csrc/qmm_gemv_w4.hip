@@ -874,6 +874,9 @@ gemv_w4_fast_cb_kernel(const uint8_t *__restrict__ pB,
 void launch_gemm_w4f(const gemv_params_t &p, int shifts, int flags_m,
         hipStream_t stream);
 bool gemm_w4f_wins(const gemv_params_t &p);
+int gemm_w4k_shape(const gemv_params_t &p);
+void launch_gemm_w4k(const gemv_params_t &p, int rb, int cb, int shifts, int flags_m,
+        hipStream_t stream);
 void launch_gemm_g128_f16(const g128_params_t &p, int rows, hipStream_t stream);
 void launch_gemm_g128_bf16(const g128_params_t &p, int rows, hipStream_t stream);
 int gemm_g128_rows(int M, int N, int K, int kind);
@@ -939,6 +942,11 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
         // an absent zero-point buffer is never dereferenced past its first
         // byte: the weights stand in for it
         const uint8_t *zp = p.zps ? (const uint8_t *)p.zps : p.B;
+        // 17 rows to some hundred: K cut over a workgroup's waves
+        if (const int shape = gemm_w4k_shape(q)) {
+            launch_gemm_w4k(q, shape / 16, shape % 16, shifts, flags_m, stream);
+            return true;
+        }
         // 4-bit weights at many rows (few: where it is the faster one, over very
         // wide weights): the kernel whose wave tile is up to 96 rows tall (direct 16-byte loads: rows on 16-byte boundaries, whole groups of
         // 128 k, 32-bit offsets inside a tile of rows)
