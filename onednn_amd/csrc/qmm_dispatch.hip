@@ -42,6 +42,8 @@ void launch_gemm_w4a8(const w4a8_params_t &p, int variant, hipStream_t stream);
 void launch_gemm_w4a8_small(const w4a8_small_t &p, bool has_zp,
         hipStream_t stream);
 bool gemm_w4a8_small_takes(const w4a8_prep_t &q);
+int gemm_w4a8k_shape(const g128_params_t &p);
+void launch_gemm_w4a8k(const g128_params_t &p, int shape, hipStream_t stream);
 void launch_gemm_g128_s8(const g128_params_t &p, int rows, hipStream_t stream);
 int gemm_g128_rows(int M, int N, int K, int kind);
 void launch_gemm_w4a8_tiny(const w4a8_small_t &p, bool has_zp, int nwv,
@@ -1243,6 +1245,45 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
             q.zsT = (int32_t *)(arrays + sc.zs_off);
             q.c2T = (int32_t *)(arrays + sc.c2_off);
         }
+        // s8 source x s4 weights without zero points, 16-bit scales per 128 k on both
+        // sides: kernels of their own, without a pre-pass
+        // (the sums of the one for many rows start from the bits of 1.5 * 2^23, which
+        // times a 16-bit scale is an f32 number; direct 16-byte loads, 32-bit offsets)
+        auto is16 = [](int dt) { return dt == dt_f16 || dt == dt_bf16; };
+        const bool g128 = w4a8_variant == 0 && !sc.has_zp
+                && q.gk == 128 && q.ss && q.sw && is16(q.ss_dt) && is16(q.sw_dt)
+                && q.ss_g == 128 && q.sw_g == 128 && q.lda % 16 == 0 && q.lda < (1 << 24)
+                && ((uintptr_t)q.A & 15) == 0;
+        const int g128_rows = gemm_g128_rows(q.M, q.N, q.K, G_S8);
+        g128_params_t t;
+        if (g128) {
+            std::memset(&t, 0, sizeof(t));
+            t.A = q.A;
+            t.lda = q.lda;
+            t.B = packed;
+            t.ss = q.ss;
+            t.ss_sm = q.ss_sm;
+            t.ss_sk = q.ss_sk;
+            t.ss_f16 = q.ss_dt == dt_f16;
+            t.scales = q.sw;
+            t.sw_sk = q.sw_sk;
+            t.sw_sn = q.sw_sn;
+            t.sw_f16 = q.sw_dt == dt_f16;
+            t.M = q.M;
+            t.N = q.N;
+            t.ng = q.ng;
+            t.nb = (int32_t)geom.nb32;
+            t.ep = g.ep;
+            const int shape = plan->w4a8_variant == 0 && geom.kt64 == 2 * (int64_t)q.ng
+                    ? gemm_w4a8k_shape(t)
+                    : 0;
+            if (shape) {
+                launch_gemm_w4a8k(t, shape, stream);
+                const hipError_t e = hipGetLastError();
+                if (e != hipSuccess) return hip_fail(e, "kernel launch");
+                return QMM_OK;
+            }
+        }
         const w4a8_small_plan_t sm = w4a8_small_plan(P, w4a8_variant);
         // the single-token kernel where the split-K kernel is not used
         const bool tiny_only = !sm.use && w4a8_variant == 0 && P.M <= 4
@@ -1316,34 +1357,8 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
                 return QMM_OK;
             }
         }
-        // s8 source x s4 weights without zero points, 16-bit scales per 128 k on both
-        // sides: the kernel with the tall wave tiles, which needs no pre-pass
-        // (its sums start from the bits of 1.5 * 2^23, which times a 16-bit scale
-        // is an f32 number; direct 16-byte loads, 32-bit offsets inside a tile)
-        const int g128_rows = gemm_g128_rows(q.M, q.N, q.K, G_S8);
-        auto is16 = [](int dt) { return dt == dt_f16 || dt == dt_bf16; };
-        if (g128_rows && w4a8_variant == 0 && !sc.has_zp && q.gk == 128 && q.ss && q.sw
-                && is16(q.ss_dt) && is16(q.sw_dt) && q.ss_g == 128 && q.sw_g == 128
-                && q.lda % 16 == 0 && q.lda < (1 << 24)
-                && ((uintptr_t)q.A & 15) == 0) {
-            g128_params_t t;
-            std::memset(&t, 0, sizeof(t));
-            t.A = q.A;
-            t.lda = q.lda;
-            t.B = packed;
-            t.ss = q.ss;
-            t.ss_sm = q.ss_sm;
-            t.ss_sk = q.ss_sk;
-            t.ss_f16 = q.ss_dt == dt_f16;
-            t.scales = q.sw;
-            t.sw_sk = q.sw_sk;
-            t.sw_sn = q.sw_sn;
-            t.sw_f16 = q.sw_dt == dt_f16;
-            t.M = q.M;
-            t.N = q.N;
-            t.ng = q.ng;
-            t.nb = (int32_t)geom.nb32;
-            t.ep = g.ep;
+        // many rows: the kernel with the tall wave tiles, which needs no pre-pass either
+        if (g128 && g128_rows) {
             launch_gemm_g128_s8(t, g128_rows, stream);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(e, "kernel launch");
