@@ -406,7 +406,7 @@ QMM_HD int part_pitch(int Qn, int D) {
 // flight. One workgroup per (group of heads, key range); its four waves take the
 // range's 32-key tiles in turn, each with its own running maximum, sum and
 // accumulators and its own piece of LDS (the V tile it transposes): no barrier
-// until the end, where wave 0 merges the four states. With more than one range
+// until the end, where all four merge their states. With more than one range
 // the merged state goes to the scratchpad (unnormalised accumulators, maximum,
 // sum per query) and sdpa_combine_kernel finishes.
 //   * p.pack heads that share a K / V head ride in the 16 query columns of one
@@ -420,6 +420,9 @@ QMM_HD int part_pitch(int Qn, int D) {
 //   * QUANT = 1: the lane that fetched a key's scale and zero point writes them to
 //     LDS as the packed f16 operands of the dequantization, one 8-byte read for
 //     each use; keys past the end are looked for in the last tile only.
+// The ranges could be added by the workgroup that ends last (a flag per range, release at
+// agent scope) instead of a second launch: 25.4 -> 37.8 us for 32 heads x 8191 keys, 7.5 ->
+// 8.5 for 8 heads x 511, since every workgroup then writes its XCD's L2 back.
 // 1 query, head size 128, launches back to back with the combining kernel, one head to
 // a workgroup and one tile ahead / this kernel (us): 32 heads x 8191 keys, s8 28.2 /
 // 23.4, f16 29.2 / 28.4; x 32768 keys, s8 79.8 / 55.0 (5.0 TB/s), f16 102.1 / 100.3;
@@ -432,9 +435,10 @@ sdpa_decode_kernel(const sdpa_params_t p) {
     constexpr int D = 32 * DC;
     constexpr int DVB = D / 16;
     constexpr int V_PITCH = D * 2 + 32;
-    constexpr int ST = D + 2; // floats of one query's state
+    constexpr int ST = D + 2; // floats of one query's state in the scratchpad
+    constexpr int SL = D + 4; // and in LDS
     constexpr int SLOTS = !QUANT && DC > 4 ? 1 : 2; // tiles requested ahead
-    constexpr int V_BYTES = SDPA_KT * V_PITCH, ST_BYTES = 16 * ST * 4;
+    constexpr int V_BYTES = SDPA_KT * V_PITCH, ST_BYTES = 16 * SL * 4;
     constexpr int W_BYTES = V_BYTES > ST_BYTES ? V_BYTES : ST_BYTES;
     // per wave: the V tile while it walks, its state at the end
     __shared__ __attribute__((aligned(16))) uint8_t lds_w[SDPA_WAVES][W_BYTES];
@@ -701,63 +705,57 @@ sdpa_decode_kernel(const sdpa_params_t p) {
     // ---- merge the four waves' states: query r, accumulator rows d = 16 dv + 4 c + i
     // (over the wave's own V tile, which it has read)
     const float l_wave = rows_sum(l_run);
-    float *mine = (float *)lds_w[wave] + r * ST;
+    float *mine = (float *)lds_w[wave] + r * SL;
 #pragma unroll
-    for (int d = 0; d < DVB; d++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) mine[d * 16 + 4 * c + i] = oacc[d][i];
+    for (int d = 0; d < DVB; d++) *(v4f *)(mine + d * 16 + 4 * c) = oacc[d];
     if (c == 0) {
         mine[D] = m_run;
         mine[D + 1] = l_wave;
     }
     __syncthreads();
-    if (wave != 0) return;
-    const float *state[SDPA_WAVES];
+    // four neighbouring values of a row per thread of all four waves (by wave 0 alone, 16
+    // lanes to a d, one query of 128 left 4 lanes 128 reads each: 32 heads over 8 K / V heads
+    // x 700 keys of 128, bf16 8.1 / 7.2 us, 32 heads x 8191 keys, s8 26.7 / 25.8)
+    constexpr int D4 = D / 4;
+    auto store = [&](int row, int d, const v4f &o, float l) {
+        uint16_t h[4];
 #pragma unroll
-    for (int w = 0; w < SDPA_WAVES; w++) state[w] = (const float *)lds_w[w] + r * ST;
-    float m_all = -INFINITY;
+        for (int i = 0; i < 4; i++) h[i] = __builtin_bit_cast(uint16_t, cvt16<BF>(o[i] / l));
+        uint16_t *Ob = p.dst + b0 * p.o.b0 + (b1_0 + row / p.Qn) * p.o.b1
+                + (int64_t)(row % p.Qn) * p.o.row;
+        *(uint2 *)(Ob + d) = make_uint2(
+                h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+    };
+    for (int idx = tid; idx < rows * D4; idx += SDPA_WAVES * 64) {
+        const int row = idx / D4, d = idx % D4 * 4;
+        const float *state[SDPA_WAVES];
+        float m_all = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < SDPA_WAVES; w++) m_all = fmaxf(m_all, state[w][D]);
-    const float m_use = m_all == -INFINITY ? 0.f : m_all;
-    float l_all = 0.f, wgt[SDPA_WAVES];
-#pragma unroll
-    for (int w = 0; w < SDPA_WAVES; w++) {
-        wgt[w] = __builtin_amdgcn_exp2f(state[w][D] - m_use);
-        l_all += wgt[w] * state[w][D + 1];
-    }
-    if (r >= rows) return;
-    if (p.nsplit == 1) {
-        uint16_t *Ob = p.dst + b0 * p.o.b0 + b1 * p.o.b1 + (int64_t)q * p.o.row;
-#pragma unroll
-        for (int d = 0; d < DVB; d++) {
-            uint16_t h[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float o = 0.f;
-#pragma unroll
-                for (int w = 0; w < SDPA_WAVES; w++)
-                    o += wgt[w] * state[w][d * 16 + 4 * c + i];
-                h[i] = __builtin_bit_cast(uint16_t, cvt16<BF>(o / l_all));
-            }
-            *(uint2 *)(Ob + d * 16 + 4 * c) = make_uint2(
-                    h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+        for (int w = 0; w < SDPA_WAVES; w++) {
+            state[w] = (const float *)lds_w[w] + row * SL;
+            m_all = fmaxf(m_all, state[w][D]);
         }
-    } else {
-        const int64_t head = (int64_t)b0 * p.B1 + b1;
-        float *out = p.part + (head * p.nsplit + split) * part_pitch(p.Qn, D) + q * ST;
+        const float m_use = m_all == -INFINITY ? 0.f : m_all;
+        float l_all = 0.f;
+        v4f o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int d = 0; d < DVB; d++)
+        for (int w = 0; w < SDPA_WAVES; w++) {
+            const float wgt = __builtin_amdgcn_exp2f(state[w][D] - m_use);
+            l_all += wgt * state[w][D + 1];
+            o += wgt * *(const v4f *)(state[w] + d);
+        }
+        if (p.nsplit == 1) {
+            store(row, d, o, l_all);
+        } else {
+            const int64_t head = (int64_t)b0 * p.B1 + b1_0 + row / p.Qn;
+            float *const out = p.part + (head * p.nsplit + split) * part_pitch(p.Qn, D)
+                    + row % p.Qn * ST;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float o = 0.f;
-#pragma unroll
-                for (int w = 0; w < SDPA_WAVES; w++)
-                    o += wgt[w] * state[w][d * 16 + 4 * c + i];
-                out[d * 16 + 4 * c + i] = o;
+            for (int i = 0; i < 4; i++) out[d + i] = o[i];
+            if (d == 0) {
+                out[D] = m_all;
+                out[D + 1] = l_all;
             }
-        if (c == 0) {
-            out[D] = m_all;
-            out[D + 1] = l_all;
         }
     }
 }
