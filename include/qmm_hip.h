@@ -275,6 +275,10 @@ QMM_API int qmm_gemm_w4k_shape(int src_dt, int weights_bits, int per_column, int
  * zero points (mfma_w4a8): the workgroup whose waves cut K, 0: another kernel. */
 QMM_API int qmm_gemm_w4a8k_shape(int64_t M, int64_t N, int64_t K);
 
+/* The same for s8 / u8 x s8 and f8_e4m3 without weights zero points (mfma_b8, one matrix);
+ * post_ops: there are some. */
+QMM_API int qmm_gemm_b8k_shape(int src_dt, int64_t M, int64_t N, int64_t K, int post_ops);
+
 /* Whether more than 16 rows of f16 / bf16 activations under 4- or 8-bit weights run on the
  * tiled kernel (1) or on the decode kernel once per 16 rows (0), where one of these takes
  * them (hip:gfx950:decode_w4). */

@@ -41,6 +41,8 @@ int gemm_f16w8_splits(int64_t M, int64_t N, int64_t K);
 void launch_gemm_w4a8(const w4a8_params_t &p, int variant, hipStream_t stream);
 void launch_gemm_w4a8_small(const w4a8_small_t &p, bool has_zp,
         hipStream_t stream);
+int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops);
+void launch_gemm_b8k(const gemm_params_t &p, bool f8, int shape, hipStream_t stream);
 bool gemm_w4a8_small_takes(const w4a8_prep_t &q);
 int gemm_w4a8k_shape(const g128_params_t &p);
 void launch_gemm_w4a8k(const g128_params_t &p, int shape, hipStream_t stream);
@@ -1125,6 +1127,17 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
         g.batch = (int32_t)P.batch;
         g.kb32 = (int32_t)geom.kb32;
         g.nb32 = (int32_t)geom.nb32;
+        // one matrix, where tiles that walk all of K leave CUs idle
+        const int b8k = P.batch == 1 && gemm_variant == 0 && plan->b8x_variant == 1
+                        && !plan->measure && !b8_needs_rowsum(D)
+                ? gemm_b8k_shape(g, f8, D.npo > 0)
+                : 0;
+        if (b8k) {
+            launch_gemm_b8k(g, f8, b8k, stream);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return hip_fail(e, "kernel launch");
+            return QMM_OK;
+        }
         // few rows of one matrix, or few results: the streaming kernel (it forms the
         // row sums a weights zero point needs itself)
         if (P.batch == 1 && gemm_variant == 0 && (!f8 || P.K % 64 == 0)

@@ -559,6 +559,15 @@ void launch_gemm_b8(const gemm_params_t &p, bool f8, int variant,
 }
 
 bool gemv_b8_takes(int64_t M, int64_t N, int64_t K, bool f8, bool tile256, bool post_ops);
+// rows of the results of a workgroup: 32 the streaming kernel, else tiles that walk all of K
+int gemm_b8_tile(const gemm_params_t &p, bool f8, bool post_ops) {
+    const bool tile256 = gemm_b8_uses_tile256(p, f8, 0);
+    if (p.batch == 1 && (!f8 || p.K % 64 == 0)
+            && gemv_b8_takes(p.M, p.N, p.K, f8, tile256, post_ops))
+        return 32;
+    if (tile256) return 256;
+    return 256 >> (tile_variant(p, f8) - 1);
+}
 #endif
 
 } // namespace qmm
@@ -579,10 +588,6 @@ extern "C" int qmm_gemm_b8_tile(
     p.lda = K;
     p.batch = (int32_t)batch;
     p.kb32 = (int32_t)((K + 31) / 32);
-    const bool tile256 = gemm_b8_uses_tile256(p, f8, 0);
-    if (batch == 1 && (!f8 || K % 64 == 0) && gemv_b8_takes(M, N, K, f8, tile256, post_ops))
-        return 32;
-    if (tile256) return 256;
-    return 256 >> (tile_variant(p, f8) - 1);
+    return gemm_b8_tile(p, f8, post_ops);
 }
 #endif

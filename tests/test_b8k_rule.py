@@ -1,0 +1,46 @@
+"""Which 8-bit products take the kernel whose waves cut K (qmm_gemm_b8k_shape): host work only. Times in us, the kernels
+before / this one, measured on an MI355X."""
+import pytest
+
+from onednn_amd import _capi, memory
+
+dt = memory.data_type
+
+
+def shape(M, K, N, src=dt.s8, post_ops=0):
+    return _capi.lib().qmm_gemm_b8k_shape(src, M, N, K, post_ops)
+
+
+@pytest.mark.parametrize("M,K,N,want", [
+    (64, 4096, 14336, 0x44),  # 23.3 / 18.0
+    (16, 12288, 2048, 0x12),  # 15.2 / 10.7
+    (195, 6912, 3296, 0x44),  # 29.5 / 16.0
+    (256, 4096, 4096, 0x44),  # 21.9 / 12.9
+    (1, 12032, 9248, 0x14),  # 27.6 / 24.5
+    (1, 4096, 14336, 0),  # 13.3 / 14.0
+    (894, 2944, 12624, 0),  # 61 / 108
+    (16384, 1024, 128, 0),  # 13.7 / 16.9
+    (4096, 4096, 14336, 0),
+])
+def test_integers(M, K, N, want):
+    assert shape(M, K, N) == want
+
+
+@pytest.mark.parametrize("M,K,N,want", [
+    (413, 12672, 3584, 0x44),  # 84 / 49
+    (350, 8704, 1472, 0x24),  # 32 / 15
+    (967, 8576, 4064, 0),  # 66 / 83
+    (1, 4096, 14336, 0),  # 13.2 / 14.5
+    (8192, 8192, 8192, 0),
+])
+def test_fp8(M, K, N, want):
+    assert shape(M, K, N, dt.f8_e4m3, 1) == want
+
+
+def test_u8_sources():
+    assert shape(256, 1024, 1024, dt.u8) == 0x22  # 5.8 / 4.9
+
+
+def test_other_arguments_take_nothing():
+    assert not shape(64, 4160, 4096) and not shape(0, 4096, 4096) and not shape(64, 1 << 40, 4096)
+    assert not shape(64, 4096, 4096, dt.f16)
