@@ -42,6 +42,8 @@ void launch_gemm_w4a8(const w4a8_params_t &p, int variant, hipStream_t stream);
 void launch_gemm_w4a8_small(const w4a8_small_t &p, bool has_zp,
         hipStream_t stream);
 int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops);
+bool gemm_b8s_takes(const gemm_params_t &p);
+void launch_gemm_b8s(const gemm_params_t &p, hipStream_t stream);
 void launch_gemm_b8k(const gemm_params_t &p, bool f8, int shape, hipStream_t stream);
 bool gemm_w4a8_small_takes(const w4a8_prep_t &q);
 int gemm_w4a8k_shape(const g128_params_t &p);
@@ -1134,6 +1136,14 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
                 : 0;
         if (b8k) {
             launch_gemm_b8k(g, f8, b8k, stream);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return hip_fail(e, "kernel launch");
+            return QMM_OK;
+        }
+        // many matrices of a short K
+        if (gemm_variant == 0 && plan->b8x_variant == 1 && !plan->measure && D.src.dt == dt_s8
+                && !g.src_zp && !b8_needs_rowsum(D) && gemm_b8s_takes(g)) {
+            launch_gemm_b8s(g, stream);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return hip_fail(e, "kernel launch");
             return QMM_OK;
