@@ -43,6 +43,8 @@ void launch_gemm_w4a8_small(const w4a8_small_t &p, bool has_zp,
         hipStream_t stream);
 int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops);
 bool gemm_b8s_takes(const gemm_params_t &p);
+int gemm_f16w8k_shape(const gemm_params_t &p);
+void launch_gemm_f16w8k(const gemm_params_t &p, int shape, hipStream_t stream);
 void launch_gemm_b8s(const gemm_params_t &p, hipStream_t stream);
 void launch_gemm_b8k(const gemm_params_t &p, bool f8, int shape, hipStream_t stream);
 bool gemm_w4a8_small_takes(const w4a8_prep_t &q);
@@ -1470,6 +1472,14 @@ int qmm_matmul_launch(const qmm_plan_t *plan, const qmm_matmul_args_t *args,
         g.batch = 1;
         g.kb32 = (int32_t)geom.kb32;
         g.nb32 = (int32_t)geom.nb32;
+        // few block tiles: the kernel whose waves cut K
+        const int w8k = gemm_variant == 0 && plan->b8x_variant == 1 ? gemm_f16w8k_shape(g) : 0;
+        if (w8k) {
+            launch_gemm_f16w8k(g, w8k, stream);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return hip_fail(e, "kernel launch");
+            return QMM_OK;
+        }
         // gemm_variant 1: never cut K into slices
         const int splits
                 = gemm_variant == 1 ? 1 : gemm_f16w8_splits(P.M, P.N, P.K);
