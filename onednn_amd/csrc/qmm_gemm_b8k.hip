@@ -291,8 +291,8 @@ static double b8_other_us(const gemm_params_t &p, bool f8, bool post_ops) {
 // 4832 7.3 / 8.1, 1 x 4096 x 14336 13.3 / 14.0; 1 x 12032 x 9248 27.6 / 24.5). Over 640 problems
 // of 1 ... 2500 rows 1.25 times as fast in the mean, the choice 0.6 % behind the faster kernel,
 // 20 % at most. A round of workgroups costs a start, an end and the waves' K; a CU holds one,
-// or (up to 64 products of 16 x 16) two.
-// one matrix; p.wei_zp, p.w_off: none (the caller checks)
+// or (up to 16 x 64 or 32 x 32 results) two. The caller checks that there is one matrix and no
+// weights zero point.
 int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops) {
     if (p.K % 128 != 0 || (int64_t)p.M * p.lda >= (int64_t)1 << 32) return 0;
     if (p.M <= 4 && p.K > 3072 && p.K <= 4096 && p.N > 4096) return 0;
