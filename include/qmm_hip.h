@@ -266,7 +266,7 @@ QMM_API int qmm_gemm_b8_tile(int src_dt, int64_t batch, int64_t M, int64_t N, in
 QMM_API int64_t qmm_gemv_b8_block(int64_t M, int64_t N, int64_t workgroup);
 
 /* The blocks of 16 rows (times 16) and of 16 columns that a workgroup works on where more
- * than 16 rows of f16 / bf16 activations under 4- or 8-bit weights (decode_w4; one scale
+ * than 8 rows of f16 / bf16 activations under 4- or 8-bit weights (decode_w4; one scale
  * per column, or one per K group) run with K cut over its waves; 0: another kernel. */
 QMM_API int qmm_gemm_w4k_shape(int src_dt, int weights_bits, int per_column, int64_t M,
         int64_t N, int64_t K);

@@ -942,7 +942,7 @@ bool launch_gemv_w4(const gemv_params_t &p, hipStream_t stream) {
         // an absent zero-point buffer is never dereferenced past its first
         // byte: the weights stand in for it
         const uint8_t *zp = p.zps ? (const uint8_t *)p.zps : p.B;
-        // 17 rows to some hundred: K cut over a workgroup's waves
+        // 9 rows to some hundred: K cut over a workgroup's waves
         if (const int shape = gemm_w4k_shape(q)) {
             launch_gemm_w4k(q, shape / 16, shape % 16, shifts, flags_m, stream);
             return true;

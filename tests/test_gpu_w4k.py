@@ -53,6 +53,10 @@ CASES = {
     "f16_u8_groups": (S22, dict(M=60, K=1024, N=1500, G=256, **U8, **F)),
     "f16_s8_groups_no_zero_points": (S22, dict(M=36, K=1024, N=1500, wei_dt=dt.s8, with_zp=False, **F)),
     "bf16_u8_per_column": (S22, dict(M=65, K=1024, N=1500, per_column=True, **U8, **B)),
+    # 9 ... 16 rows: half of a block of 32 repeats the last row
+    "f16_u4_9_rows": (S22, dict(M=9, K=1152, N=4100, **F)),
+    "bf16_u4_16_rows": (S24, dict(M=16, K=1152, N=9220, **B)),
+    "f16_u8_15_rows": (S22, dict(M=15, K=1280, N=4166, per_column=True, **U8, **F)),
     "bf16_s8_groups": (S22, dict(M=39, K=1024, N=2000, wei_dt=dt.s8, zp_dt=dt.s8, **B)),
 }
 

@@ -56,3 +56,15 @@ def test_groups_of_8_bit_weights_take_no_tall_tile():
 def test_other_arguments_take_nothing():
     assert shape(0, 1024, 1024) == 0 and shape(100, 1024, 4096, 2) == 0 and shape(100, 1024, 4096, src=dt.s8) == 0
     assert shape(100, 1 << 40, 4096) == 0
+
+
+@pytest.mark.parametrize("M,K,N,bits,src,want", [
+    (16, 1280, 4160, 8, dt.f16, 0x22),  # 13.1 / 6.1
+    (14, 8704, 11712, 8, dt.f16, 0x24),  # 45.5 / 27.9
+    (15, 3456, 5408, 4, dt.f16, 0x22),  # 11.7 / 7.8
+    (12, 2432, 12432, 4, dt.bf16, 0x24),  # 17.5 / 9.3
+    (14, 7808, 3440, 4, dt.f16, 0),  # 9.9 / 11.5
+    (8, 4096, 14336, 4, dt.f16, 0), (9, 4096, 4096, 8, dt.f16, 0),
+])
+def test_9_to_16_rows(M, K, N, bits, src, want):
+    assert shape(M, K, N, bits, src, per_column=bits == 8) == want
