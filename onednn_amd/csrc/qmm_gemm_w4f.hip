@@ -101,7 +101,8 @@ gemm_w4f_kernel(const gemv_params_t p, const int shifts, const int flags_m) {
     const uint8_t *Bt[CBW];
     const uint16_t *scn[CBW];
     int zcol[CBW];
-    const int64_t sN = scale_per_n ? N : 0, zN = zp_per_n ? N : 0;
+    // from one group's scales / zero points to the next: a row of N, or one for all columns
+    const int64_t sN = scale_per_n ? N : 1, zN = zp_per_n ? N : 1;
     const uint8_t *pZP = p.zps ? (const uint8_t *)p.zps : p.B;
 #pragma unroll
     for (int cb = 0; cb < CBW; cb++) {

@@ -145,7 +145,8 @@ gemm_w4k_kernel(const gemv_params_t p, const int shifts, const int flags_m) {
     const uint32_t rd_at = r * 256 + (((r & 3) << 6) | ((r >> 2) ^ c) << 4);
     // (no branch on any of these in the loop: one would wait for every load before it)
     const int gs_sh = gs_shift < 0 ? 31 : gs_shift, gz_sh = gz_shift < 0 ? 31 : gz_shift;
-    const uint32_t sN = scale_per_n ? N : 0, zN = has_zp && zp_per_n ? N : 0;
+    // from one group's scales / zero points to the next: a row of N, or one for all columns
+    const uint32_t sN = scale_per_n ? N : 1, zN = !has_zp ? 0 : zp_per_n ? N : 1;
     const uint8_t *const pZP = has_zp ? (const uint8_t *)p.zps : p.B;
     const uint32_t zhalf = zp4 ? 1 : 0;
     const uint32_t zmask = !has_zp ? 0u : zp4 ? 15u : 255u;

@@ -158,7 +158,6 @@ gemv_w4_kernel(const gemv_params_t p, const int MR, const int KC) {
     // Loading and decoding are split: the raw bits are fetched without any
     // dependent instruction, so the compiler can leave the loads in flight
     // next to the weights stream and convert when the value is needed.
-    const int64_t sN = p.scale_per_n ? p.N : 0, zN = p.zp_per_n ? p.N : 0;
     const bool lane_ok = n < p.N;
     auto scale_raw = [&](int kq) -> uint32_t {
         if (!p.scales || !lane_ok) return 0u;
@@ -413,7 +412,8 @@ gemv_w4_fast_kernel(const uint8_t *__restrict__ pB,
     constexpr int TILE_BYTES = 1024 * NP;
     const uint8_t *__restrict__ Bt
             = pB + ((int64_t)nb * kg128) * TILE_BYTES + lane * 16;
-    const int64_t sN = scale_per_n ? N : 0, zN = zp_per_n ? N : 0;
+    // from one group's scales / zero points to the next: a row of N, or one for all columns
+    const int64_t sN = scale_per_n ? N : 1, zN = zp_per_n ? N : 1;
 
     // Waves are independent until the final reduction: each one fetches its
     // weight tiles, their scales / zero points AND its activation fragments
@@ -662,7 +662,8 @@ gemv_w4_fast_cb_kernel(const uint8_t *__restrict__ pB,
     const uint8_t *__restrict__ Bt
             = pB + ((int64_t)nb * kg128) * TILE_BYTES + lane * 16;
     const int64_t BSTEP = (int64_t)kg128 * TILE_BYTES; // to the next column block
-    const int64_t sN = scale_per_n ? N : 0, zN = zp_per_n ? N : 0;
+    // from one group's scales / zero points to the next: a row of N, or one for all columns
+    const int64_t sN = scale_per_n ? N : 1, zN = zp_per_n ? N : 1;
 
     // Waves are independent until the final reduction: each one fetches its
     // weight tiles, their scales / zero points AND its activation fragments
