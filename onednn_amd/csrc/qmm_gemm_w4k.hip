@@ -433,20 +433,22 @@ int gemm_g128_rows(int M, int N, int K, int kind);
 // of workgroups (one on a CU, 32 on an XCD) costs a start, an end and the waves' K; a begun
 // round costs most of a whole one. us at K = 1024 (f16 x u4, one round 32 x 32 / 32 x 64 /
 // 48 x 64 results): 4.6 / 5.8 / 7.5, and 1.1 / 1.5 / 2.2 per further 1024 k.
-// 9 ... 16 rows: from 256 blocks of 16 columns on the decode kernel has more than one
+// 9 ... 16 rows: past 256 blocks of 16 columns the decode kernel has more than one
 // workgroup on a CU and stages no rows; 29 problems there 1.15 ... 2.2 times as fast here
 // (u8 16 x 1280 x 4160 13.1 / 6.1, 14 x 8704 x 11712 45 / 28; u4 f16 15 x 3456 x 5408 11.7 / 7.8,
 // bf16 12 x 2432 x 12432 17.5 / 9.3); with fewer it may be ahead (u4 14 x 7808 x 3440 9.9 / 11.5).
+// Over 65536 columns and more, few k under 4-bit weights are the tall tiles' (qmm_gemm_g128.hip:
+// bf16 10 x 128 x 95648 10.3 / 21.6, 15 x 512 x 78560 18.0 / 21.9, f16 12 x 512 x 69472 16.7 / 19.9).
 int gemm_w4k_shape(const gemv_params_t &p) {
     if (p.M <= 8 || (p.M <= 16 && p.N <= 4096) || p.K % 128 != 0
             || (int64_t)p.M * p.lda * 2 >= (int64_t)1 << 32
             || (int64_t)p.kg128 * p.N >= (int64_t)1 << 31)
         return 0;
     const int kind = p.act_f16 ? G_F16 : G_BF16;
-    const double other = p.M <= 16 ? 1e30
-            : !p.w8 && gemm_g128_rows(p.M, p.N, p.K, kind)
+    const double other = !p.w8 && gemm_g128_rows(p.M, p.N, p.K, kind)
             ? gemm_g128_us(p.M, p.N, p.K, kind)
-            : gemm_w4f_us(p);
+            : p.M <= 16 ? 1e30
+                        : gemm_w4f_us(p);
     const bool tall = w4k_tall(p.act_f16, p.w8, w4k_fold(p));
     // {once, per round, per round and 1024 k}
     static const double f16[3][3] = {{1.1, 2.4, 1.09}, {0.4, 3.9, 1.54}, {-0.6, 5.9, 2.19}};

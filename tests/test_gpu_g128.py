@@ -31,6 +31,8 @@ def run(ctx, p, tile, impl):
     eng, strm = ctx
     (M, K), N = p.src.dims, p.wei.dims[1]
     assert _capi.lib().qmm_gemm_g128_rows(p.src.dt, M, N, K) == tile
+    if impl == parity.DECODE:  # (the launch asks for this one first)
+        assert not _capi.lib().qmm_gemm_w4k_shape(p.src.dt, 4, int(p.scales["wei"][2] is None), M, N, K)
     got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
     assert pd.impl_info_str() == impl
     return got

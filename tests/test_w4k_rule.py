@@ -65,6 +65,12 @@ def test_other_arguments_take_nothing():
     (12, 2432, 12432, 4, dt.bf16, 0x24),  # 17.5 / 9.3
     (14, 7808, 3440, 4, dt.f16, 0),  # 9.9 / 11.5
     (8, 4096, 14336, 4, dt.f16, 0), (9, 4096, 4096, 8, dt.f16, 0),
+    # very wide 4-bit weights with few k: the tall tiles
+    (10, 128, 95648, 4, dt.bf16, 0),  # 10.3 / 21.6
+    (10, 256, 76352, 4, dt.bf16, 0),  # 12.2 / 19.2
+    (15, 512, 78560, 4, dt.bf16, 0),  # 18.0 / 21.9
+    (12, 512, 69472, 4, dt.f16, 0),  # 16.7 / 19.9
+    (16, 256, 65590, 4, dt.bf16, 0),
 ])
 def test_9_to_16_rows(M, K, N, bits, src, want):
     assert shape(M, K, N, bits, src, per_column=bits == 8) == want
