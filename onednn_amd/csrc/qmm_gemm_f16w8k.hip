@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "qmm_device.hpp"
+#include "qmm_kcut.hpp"
 #include "qmm_hip.h"
 #include "qmm_plan.hpp"
 
@@ -236,7 +237,8 @@ static double f16w8_tiled_us(const gemm_params_t &p) {
 // Row and column blocks of a workgroup as 16 * rb + cb, 0: 256 x 256 tiles are faster. Before /
 // now (us): 263 x 1280 x 3040 43.4 / 12.6, 350 x 2688 x 2384 44.6 / 14, 424 x 2816 x 5344 63 / 40,
 // 468 x 10496 x 1792 51 / 31, 872 x 8192 x 2208 79 / 55, 303 x 5632 x 12304 102 / 90; there from
-// some 500 rows and 20 million weights on (614 x 1664 x 10400 56 / 70, 1922 x 2304 x 2864 63 / 82, 4096 x 1024 x 1024 36 / 42).
+// some 500 rows and 20 million weights on (614 x 1664 x 10400 56 / 70, 1922 x 2304 x 2864 63 / 82, 4096 x 1024 x 1024 36 / 42)
+// and with long rows (1473 x 14464 x 1344 107 / 124, 2102 x 9216 x 816 75 / 81; but 885 x 12160 x 1472 91 / 70).
 // Over 150 problems 1.9 times as fast in the mean, the choice 2 % behind the faster kernel. One
 // workgroup on a CU (32 on an XCD); a begun round costs most of a whole one.
 int gemm_f16w8k_shape(const gemm_params_t &p) {
@@ -248,10 +250,11 @@ int gemm_f16w8k_shape(const gemm_params_t &p) {
             {4, 4, 0.72, 7.07, 2.69, 0.68}};
     double best = f16w8_tiled_us(p) / (p.M > 2500 ? 1.5 : 1.15); // (clearly, or not)
     int pick = 0;
+    const double rows = many_rows(p.M, p.K, 0.25);
     for (const auto &s : shapes) {
         const double wgs = f16w8k_map(p.M, (p.N + 15) / 16, s.rb, s.cb).share / 32.0;
         const double rounds = std::max(1.0, s.begun * std::ceil(wgs) + (1 - s.begun) * wgs);
-        const double us = s.once + rounds * (s.start + s.k1024 * p.K / 1024);
+        const double us = s.once + rounds * (s.start + s.k1024 * p.K / 1024) * rows;
         if (us < best) {
             best = us;
             pick = 16 * s.rb + s.cb;

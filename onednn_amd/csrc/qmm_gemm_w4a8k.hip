@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "qmm_device.hpp"
+#include "qmm_kcut.hpp"
 #include "qmm_hip.h"
 #include "qmm_plan.hpp"
 
@@ -264,10 +265,11 @@ static double w4a8_tiled_us(int M, int N, int K) {
 // now (us): 64 x 4096 x 14336 24 / 17, 8 x 4096 x 4096 16.5 / 5.9, 1 x 13312 x 1312 10.3 /
 // 9.0, 128 x 12288 x 2048 85 / 12.9, 435 x 5376 x 3888 43 / 31, 1941 x 1024 x 1072 18.8 /
 // 18.0; the tall tiles of qmm_gemm_g128.hip stay ahead from some 200 rows and 15 million
-// weights on (256 x 4096 x 14336 37 / 50, 1000 x 4096 x 4096 37 / 58). Up to 64 rows no
+// weights on (256 x 4096 x 14336 37 / 50, 1000 x 4096 x 4096 37 / 58, 1267 x 14336 x 2768 109 / 129). Up to 64 rows no
 // problem but the one below was faster without. Over 365 problems of 1 ... 4096 rows the choice is 0.2 %
 // behind the faster kernel in the mean and 15 % at most, 2.2 times as fast as before in the
-// mean. A round of workgroups costs a start, an end and the waves' K; a CU holds one, or (16
+// mean; over 1700 further ones up to 5 % slower than the kernels before (17 ... 32 rows of few k
+// over some 20000 columns up to 12 %: 17 x 640 x 22400 7.8 / 8.7). A round of workgroups costs a start, an end and the waves' K; a CU holds one, or (16
 // rows) two, which take about twice as long as one.
 int gemm_w4a8k_shape(const g128_params_t &p) {
     // 32-bit offsets of rows, row scales and column scales
@@ -290,6 +292,7 @@ int gemm_w4a8k_shape(const g128_params_t &p) {
     } shapes[] = {{1, 2, 2.79, 0.98, 0.44, 0.79}, {1, 4, 3.17, 1.17, 0.68, 0.95},
             {2, 4, 1.49, 3.14, 1.03, 0.99}, {3, 4, 1.03, 4.14, 1.33, 0.94}};
     int pick = 0;
+    const double rows = many_rows(p.M, K, 0.25);
     for (const auto &s : shapes) {
         // workgroups on a CU (32 on an XCD)
         const double wgs = w4a8k_map(p.M, (p.N + 15) / 16, s.rb, s.cb).share / 32.0;
@@ -304,7 +307,8 @@ int gemm_w4a8k_shape(const g128_params_t &p) {
         } else {
             rounds = s.begun * std::ceil(wgs) + (1 - s.begun) * wgs;
         }
-        const double us = s.once + std::max(1.0, rounds) * (s.start + s.k1024 * K / 1024);
+        const double us
+                = s.once + std::max(1.0, rounds) * (s.start + s.k1024 * K / 1024) * rows;
         if (us < best) {
             best = us;
             pick = 16 * s.rb + s.cb;

@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "qmm_device.hpp"
+#include "qmm_kcut.hpp"
 #include "qmm_plan.hpp"
 
 // Instantiated per activation type and weights width (QMM_W4K_PART = 0..3: bit 0 f16
@@ -428,8 +429,9 @@ int gemm_g128_rows(int M, int N, int K, int kind);
 // 1248 22.7 / 11.5, 269 x 9856 x 5168 82 / 53; bf16 x u4 204 x 12928 x 2176 111 / 25, 711 x
 // 9088 x 3520 131 / 102; f16 x u8 148 x 12800 x 1424 83 / 19, 64 x 4096 x 14336 51 / 28; the
 // other kernels stay ahead from 450 rows and 8 million weights on (727 x 4480 x 4064 64 / 65,
-// bf16 684 x 9472 x 14016 252 / 381). Over 260 shapes of 17 ... 2048 rows 1.75 times as fast in
-// the mean, the choice within 0.5 % of the faster kernel in the mean and 20 % at most. A round
+// bf16 684 x 9472 x 14016 252 / 381, 1324 x 13824 x 2544 192 / 220). Over 260 shapes of 17 ... 2048 rows 1.75 times as fast in
+// the mean, the choice within 0.5 % of the faster kernel in the mean and 20 % at most; over 1900 further ones 8 % at
+// most slower than the others (bf16 948 x 6912 x 3328 104 / 113). A round
 // of workgroups (one on a CU, 32 on an XCD) costs a start, an end and the waves' K; a begun
 // round costs most of a whole one. us at K = 1024 (f16 x u4, one round 32 x 32 / 32 x 64 /
 // 48 x 64 results): 4.6 / 5.8 / 7.5, and 1.1 / 1.5 / 2.2 per further 1024 k.
@@ -458,12 +460,13 @@ int gemm_w4k_shape(const gemv_params_t &p) {
     static const int shapes[3][2] = {{2, 2}, {2, 4}, {3, 4}};
     double best = other / 1.1; // (clearly, or not)
     int pick = 0;
+    const double rows = many_rows(p.M, p.K, 0.25);
     for (int i = 0; i < (tall ? 3 : 2); i++) {
         const double rounds = w4k_map(p.M, p.nb16, shapes[i][0], shapes[i][1]).share / 32.0;
         const double us = (p.w8 && !p.act_f16 ? 1.2 : 1.0)
                 * (c[i][0]
                         + std::max(1.0, 0.8 * std::ceil(rounds) + 0.2 * rounds)
-                                * (c[i][1] + c[i][2] * p.K / 1024));
+                                * (c[i][1] + c[i][2] * p.K / 1024) * rows);
         if (us < best) {
             best = us;
             pick = 16 * shapes[i][0] + shapes[i][1];

@@ -13,6 +13,10 @@ from onednn_amd import _capi
     (1922, 2304, 2864, 0),  # 62.9 / 82.2
     (4096, 1024, 1024, 0),  # 36.3 / 42.4
     (3000, 1024, 1024, 0x44),  # 42.8 / 32.1
+    # long rows that no L2 holds
+    (1473, 14464, 1344, 0),  # 106.3 / 124.2
+    (2102, 9216, 816, 0),  # 74.9 / 80.9
+    (885, 12160, 1472, 0x34),  # 90.3 / 69.3
     (2176, 4096, 14336, 0), (300, 1056, 1168, 0), (0, 1024, 1168, 0), (300, 1 << 40, 1168, 0),
 ])
 def test_shape(M, K, N, want):

@@ -17,6 +17,7 @@ from onednn_amd import _capi, memory
     (200, 4096, 14336, 0),  # 37.6 / 42.3
     (1000, 4096, 4096, 0),  # 37.5 / 57.9
     (1941, 4096, 14336, 0),  # 161.8 / 341.2
+    (1267, 14336, 2768, 0),  # 106.0 / 128.1
 ])
 def test_shape(M, K, N, want):
     assert _capi.lib().qmm_gemm_w4a8k_shape(M, N, K) == want

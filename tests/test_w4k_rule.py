@@ -34,6 +34,8 @@ def test_4_bit_weights_under_f16(M, K, N, want):
     (711, 9088, 3520, 0x24),  # 131.1 / 102.4
     (1310, 3968, 1488, 0),  # 45.3 / 51.8
     (361, 10112, 16288, 0),  # 188.8 / 240.4
+    (1324, 13824, 2544, 0),  # 191.4 / 219.1
+    (400, 6784, 9872, 0x24),  # 134.7 / 114.2
 ])
 def test_4_bit_weights_under_bf16(M, K, N, want):
     assert shape(M, K, N, src=dt.bf16) == want
