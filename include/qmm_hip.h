@@ -279,7 +279,7 @@ QMM_API int qmm_gemm_w4a8k_shape(int64_t M, int64_t N, int64_t K);
  * post_ops: there are some. */
 QMM_API int qmm_gemm_b8k_shape(int src_dt, int64_t M, int64_t N, int64_t K, int post_ops);
 
-/* The same for f16 x 8-bit weights at many rows (mfma_f16w8). */
+/* The same for f16 x 8-bit weights at many rows (mfma_f16w8), without post-ops. */
 QMM_API int qmm_gemm_f16w8k_shape(int64_t M, int64_t N, int64_t K);
 
 /* Whether more than 16 rows of f16 / bf16 activations under 4- or 8-bit weights run on the

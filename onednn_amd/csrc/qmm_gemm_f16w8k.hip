@@ -1,7 +1,7 @@
 // hip:gfx950:mfma_f16w8 where 256 x 256 tiles are few: f16 activations x 8-bit weights of
 // QMM_LAYOUT_MFMA_B8, one scale and zero point per column or in all, K a multiple of 128
 // (arithmetic of qmm_gemm_f16w8.hip). A workgroup owns 16 RB x 64 results; its eight waves cut K
-// between them, 128 k each in turn, and each holds all the results, as in qmm_gemm_f16w8k.hip.
+// between them, 128 k each in turn, and each holds all the results, as in qmm_gemm_b8k.hip.
 //   * A lane's 16 weight bytes (column r, k 64 h + 16 c ...) are two operands of 16 x 16 x 32: k
 //     8 e ... + 7 of them, e = 0, 1; the rows' operand is the 16 bytes of the same k.
 //   * Rows are requested four lanes to 64 bytes and change to operand order in a piece of LDS
@@ -225,22 +225,30 @@ gemm_f16w8k_kernel(const gemm_params_t p) {
 
 int gemm_f16w8_splits(int64_t M, int64_t N, int64_t K);
 
-// us of the 256 x 256 kernel with as many K slices as it would take (150 problems of 256 ...
-// 3000 rows, 22 % rms: rows of a length off 16 bytes cost it up to twice that)
+// us of the 256 x 256 kernel with as many K slices as it would take (1500 problems of 256 ...
+// 3000 rows). What it takes besides its K is the store of its results: whole quads of 128
+// columns 15 us, 4 more with a post-op, and up to 0.4 per row past a multiple of 64; columns that end inside 128 26 us
+// more, with a post-op 67 (786 x 256 x 896 31 us, 778 x 752 x 640 52, with a swish 832 x 256 x
+// 512 28, 875 x 656 x 896 108). Slices store f32 sums and leave the post-ops to a second kernel.
 static double f16w8_tiled_us(const gemm_params_t &p) {
     const int splits = gemm_f16w8_splits(p.M, p.N, p.K);
     const int64_t tiles = (int64_t)((p.M + 255) / 256) * ((p.N + 255) / 256) * splits;
-    const double us = 5.8 + (double)((tiles + 255) / 256) * (33.0 + 17.45 * p.K / 1024 / splits);
-    return splits == 1 ? us : us - 12.45 + 0.54e-6 * splits * p.M * p.N * 4.0;
+    const double rounds = (double)((tiles + 255) / 256), k = p.K / 1024.0 / splits;
+    const bool ends = p.N % 128 != 0, post = p.ep.npo > 0;
+    if (splits > 1)
+        return 22.4 + rounds * (19.7 * k - 4 + (ends ? 10.3 : 0)) + 1.8e-6 * splits * p.M * p.N;
+    const double tail = ends ? (post ? 67 : 26) : (post ? 0.4 : 0.15) * (p.M % 64);
+    return 1 + rounds * (14.5 + (post ? 4 : 0) + 18 * k) + tail;
 }
 
 // Row and column blocks of a workgroup as 16 * rb + cb, 0: 256 x 256 tiles are faster. Before /
 // now (us): 263 x 1280 x 3040 43.4 / 12.6, 350 x 2688 x 2384 44.6 / 14, 424 x 2816 x 5344 63 / 40,
 // 468 x 10496 x 1792 51 / 31, 872 x 8192 x 2208 79 / 55, 303 x 5632 x 12304 102 / 90; there from
-// some 500 rows and 20 million weights on (614 x 1664 x 10400 56 / 70, 1922 x 2304 x 2864 63 / 82, 4096 x 1024 x 1024 36 / 42)
-// and with long rows (1473 x 14464 x 1344 107 / 124, 2102 x 9216 x 816 75 / 81; but 885 x 12160 x 1472 91 / 70).
-// Over 150 problems 1.9 times as fast in the mean, the choice 2 % behind the faster kernel. One
-// workgroup on a CU (32 on an XCD); a begun round costs most of a whole one.
+// some 500 rows and 20 million weights on (614 x 1664 x 10400 56 / 70, 1922 x 2304 x 2864 63 / 82, 4096 x 1024 x 1024 36 / 42),
+// earlier where columns come in whole multiples of 128 (331 x 256 x 8960 22 / 24, 1103 x 5504 x 2560 65 / 73), and
+// with long rows (1473 x 14464 x 1344 106 / 124, 2102 x 9216 x 816 75 / 81; but 885 x 12160 x 1472 90 / 69).
+// Over 1750 problems of 256 ... 3000 rows 1.7 times as fast in the mean and up to 6 % slower than before
+// (2141 x 3456 x 1152 57 / 61). One workgroup on a CU (32 on an XCD); a begun round costs most of a whole one.
 int gemm_f16w8k_shape(const gemm_params_t &p) {
     if (p.K % 128 != 0 || (int64_t)p.M * p.lda >= (int64_t)1 << 32) return 0;
     static const struct {
@@ -248,7 +256,7 @@ int gemm_f16w8k_shape(const gemm_params_t &p) {
         double once, start, k1024, begun;
     } shapes[] = {{2, 4, 2.48, 4.28, 1.9, 0.69}, {3, 4, 1.45, 5.95, 2.29, 0.76},
             {4, 4, 0.72, 7.07, 2.69, 0.68}};
-    double best = f16w8_tiled_us(p) / (p.M > 2500 ? 1.5 : 1.15); // (clearly, or not)
+    double best = f16w8_tiled_us(p) / 1.1; // (clearly, or not)
     int pick = 0;
     const double rows = many_rows(p.M, p.K, 0.25);
     for (const auto &s : shapes) {

@@ -17,6 +17,11 @@ from onednn_amd import _capi
     (1473, 14464, 1344, 0),  # 106.3 / 124.2
     (2102, 9216, 816, 0),  # 74.9 / 80.9
     (885, 12160, 1472, 0x34),  # 90.3 / 69.3
+    # columns in multiples of 128, which the tiles store faster
+    (331, 256, 8960, 0),  # 21.8 / 23.8
+    (1283, 512, 2816, 0),  # 25.7 / 27.5
+    (1031, 640, 3840, 0),
+    (344, 256, 12528, 0x44),  # with a swish 87 / 38
     (2176, 4096, 14336, 0), (300, 1056, 1168, 0), (0, 1024, 1168, 0), (300, 1 << 40, 1168, 0),
 ])
 def test_shape(M, K, N, want):
