@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "qmm_device.hpp"
+#include "qmm_kcut.hpp"
 #include "qmm_hip.h"
 #include "qmm_plan.hpp"
 
@@ -256,41 +257,65 @@ gemm_b8k_kernel(const gemm_params_t p) {
 } // namespace
 
 int gemm_b8_tile(const gemm_params_t &p, bool f8, bool post_ops);
+bool gemm_b8x_two_per_cu(const gemm_params_t &p, bool f8);
 
-// us of the kernels that gemm_b8_tile chooses between, from 65 rows on (400 problems of 1024
-// ... 14336 k and up to 2500 rows, 6 ... 14 % rms): {once, per round, per round and 1024 k,
-// per 1024 k while no CU has two, a begun round's share}
+// us of the kernels that gemm_b8_tile chooses between (4900 problems of 128 ... 16384 k, 33 ...
+// 2500 rows and 16 ... 131072 columns, weights in and out of the caches, 5 ... 12 % rms): {rows,
+// columns and workgroups of a round, once, per round, per round and 1024 k, a begun round's share;
+// what workgroups alone on their CUs save once and per 1024 k; columns off a multiple of
+// `align`, per round; per MB of results}. The last three are the kernels of 256 rows, which take half as
+// long over few k where columns are aligned (s8 2398 x 128 x 1152 9.8 us, 2423 x 128 x 1264 16.3).
 static double b8_other_us(const gemm_params_t &p, bool f8, bool post_ops) {
     static const struct {
         int rows, cols, slots;
-        double once, start, k1024, single, begun;
+        double once, start, k1024, begun, alone, alone_k1024;
+        int align;
+        double tail, mb;
     } kernels[] = {
-            {32, 32, 512, 2.12, 3.84, 2.12, -1.02, 0.31},
-            {32, 32, 512, 1.86, 3.48, 2.18, -1.17, 0.29},
-            {64, 64, 256, 3.7, 4.0, 3.1, 0, 0.5},
-            {64, 64, 256, 2.8, 3.5, 3.5, 0, 0.5},
-            {128, 128, 256, 16.1, 1.46, 4.72, 0.77, 0.62},
-            {128, 128, 256, 13.6, 2.0, 5.1, 0, 0.5},
-            {256, 256, 256, 20.7, 23.4, 0.65, 4.75, 0.3},
-            {256, 128, 512, 51.7, -38.2, 16.6, -10.3, 0.5},
+            {32, 32, 512, 2.12, 3.84, 2.12, 0.31, 0, 1.02, 1, 0, 0},
+            {32, 32, 512, 1.86, 3.48, 2.18, 0.29, 0, 1.17, 1, 0, 0},
+            {64, 64, 256, 3.7, 4.0, 3.1, 0.5, 0, 0, 1, 0, 0},
+            {64, 64, 256, 2.8, 3.5, 3.5, 0.5, 0, 0, 1, 0, 0},
+            {128, 128, 256, 16.1, 1.46, 4.72, 0.62, 0, -0.77, 1, 0, 0},
+            {128, 128, 256, 13.6, 2.0, 5.1, 0.5, 0, 0, 1, 0, 0},
+            {256, 256, 256, 31.0, -8.6, 12.3, 0.3, 11.6, 2.5, 128, 6.7, 0.89},
+            {256, 128, 512, -3.8, 12.4, 12.6, 0.31, 0, 5.4, 64, 5.2, 0.13},
+            {256, 256, 256, 10.8, 11.9, 12.1, 0.6, 4.3, 0, 64, 0, 0.13},
     };
-    const int tile = gemm_b8_tile(p, f8, post_ops);
-    const auto &t = kernels[(tile == 32 ? 0 : tile == 64 ? 2 : tile == 128 ? 4 : 6) + !f8];
+    gemm_params_t q = p;
+    const int64_t tiles256 = (((int64_t)p.M + 255) / 256) * (((int64_t)p.N + 255) / 256);
+    double flip = 0;
+    if (p.a_is_u8 && p.K > 256 && p.K % 64 == 0 && tiles256 >= 192
+            && !gemm_b8x_two_per_cu(p, f8)) { // (rewritten as s8 by a pre-pass)
+        q.a_preflipped = 1;
+        flip = 3 + (double)p.M * p.K / 2e6;
+    }
+    const int tile = gemm_b8_tile(q, f8, post_ops);
+    const auto &t = kernels[tile == 32 ? !f8 : tile == 64 ? 2 + !f8 : tile == 128 ? 4 + !f8
+                    : f8                                                          ? 6
+                    : gemm_b8x_two_per_cu(q, f8)                                  ? 7
+                                                                                  : 8];
     const int64_t wgs = (((int64_t)p.M + t.rows - 1) / t.rows) * ((p.N + t.cols - 1) / t.cols);
     const double k = p.K / 1024.0, x = (double)wgs / t.slots;
     const double rounds = std::max(1.0, t.begun * std::ceil(x) + (1 - t.begun) * x);
-    return t.once + rounds * (t.start + t.k1024 * k) + (wgs <= 256 ? t.single * k : 0.0);
+    const double mb = (double)p.M * p.N * (p.ep.dst.dt == dt_f32 || p.ep.dst.dt == dt_s32 ? 4e-6 : 2e-6);
+    return t.once + flip + t.mb * mb
+            + rounds * (t.start + t.k1024 * k + (p.N % t.align ? t.tail : 0.0))
+            - (wgs <= 256 ? t.alone + t.alone_k1024 * k : 0.0);
 }
 
 // Row and column blocks of a workgroup as 16 * rb + cb, 0: another kernel is faster. Before /
 // now (us): s8 64 x 4096 x 14336 23.3 / 18.0, 16 x 12288 x 2048 15.2 / 10.7, 195 x 6912 x
 // 3296 29.5 / 16.0, 256 x 4096 x 4096 21.9 / 12.9, u8 256 x 1024 x 1024 5.8 / 4.9; fp8 413 x
 // 12672 x 3584 84 / 49, 350 x 8704 x 1472 32 / 15. The tiles that walk all of K stay ahead
-// from some hundred rows on (fp8 967 x 8576 x 4064 66 / 83, s8 894 x 2944 x 12624 61 / 108), and
+// from some hundred rows on (fp8 967 x 8576 x 4064 66 / 83, s8 894 x 2944 x 12624 61 / 108), over few k
+// and many aligned columns from 33 rows on (fp8 65 x 640 x 62464 21 / 50, 1102 x 640 x 4608 20.6 / 45,
+// 40 x 384 x 56928 21 / 27; s8 74 x 6016 x 49408 84 / 121) and for u8 rows where these are rewritten once
+// for many tiles (1934 x 14336 x 4112 184 / 284); and
 // up to 4 rows of 4096 k the streaming kernel, which requests all of them at once (1 x 4096 x
 // 4832 7.3 / 8.1, 1 x 4096 x 14336 13.3 / 14.0; 1 x 12032 x 9248 27.6 / 24.5). Over 640 problems
-// of 1 ... 2500 rows 1.25 times as fast in the mean, the choice 0.6 % behind the faster kernel,
-// 20 % at most. A round of workgroups costs a start, an end and the waves' K; a CU holds one,
+// of 1 ... 2500 rows 1.25 times as fast in the mean; over 5300 further ones 1.17 times, and up to 17 %
+// slower than the kernels before (fp8 82 x 15232 x 35968 164 / 191; u8 165 x 128 x 10208 12.0 / 13.4). A round of workgroups costs a start, an end and the waves' K; a CU holds one,
 // or (up to 16 x 64 or 32 x 32 results) two. The caller checks that there is one matrix and no
 // weights zero point.
 int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops) {
@@ -302,12 +327,15 @@ int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops) {
         double once, start, k1024, begun, second;
     } shapes[] = {{1, 2, 3.83, 0.95, 0.54, 1.0, 0.85}, {1, 4, 3.13, 1.86, 0.97, 1.0, 0.65},
             {2, 2, 3.44, 1.45, 0.71, 0.97, 1.0}, {2, 4, 1.35, 3.94, 1.16, 0.91, 0},
-            {4, 2, 0.97, 3.75, 1.13, 0.92, 0}, {4, 4, -0.27, 6.84, 1.57, 0.92, 0}};
-    // (clearly, or not; very tall problems are off what was measured: s8 16384 x 1024 x 128
-    // 13.7 / 16.9, 16384 x 4096 x 64 28.7 / 22.5)
-    double best = p.M > 64 ? b8_other_us(p, f8, post_ops) / (p.M > 2500 ? 1.3 : 1.05) : 1e30;
+            {4, 2, 0.97, 3.75, 1.13, 0.92, 0}, {4, 4, -0.27, 6.84, 1.57, 0.92, 0},
+            // (one row of workgroups, few k: the rounds overlap; 56 x 384 x 126800 in 32 x 32 73 us, so 60)
+            {4, 4, 2.2, 4.6, 1.57, 0.92, 0}};
+    double best = 1e30;
     int pick = 0;
+    const bool short_k = p.M <= 64 && p.K <= 1024 && !f8;
+    const double rows = many_rows(p.M, p.K, f8 ? 0.25 : 0.1);
     for (const auto &s : shapes) {
+        if (s.rb * s.cb == 16 && (s.once > 0) != short_k) continue;
         // workgroups on a CU (32 on an XCD)
         const double wgs = b8k_map(p.M, (p.N + 15) / 16, s.rb, s.cb).share / 32.0;
         double rounds = s.begun * std::ceil(wgs) + (1 - s.begun) * wgs;
@@ -318,13 +346,19 @@ int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops) {
                                     : rest <= 1 ? 1.0
                                                 : 1 + s.second * (s.begun + (1 - s.begun) * (rest - 1)));
         }
-        const double us = s.once + std::max(1.0, rounds) * (s.start + s.k1024 * p.K / 1024);
+        const double us = s.once + std::max(1.0, rounds) * (s.start + s.k1024 * p.K / 1024) * rows;
         if (us < best) {
             best = us;
             pick = 16 * s.rb + s.cb;
         }
     }
-    return pick;
+    if (p.M <= 32 || (p.M <= 64 && (!f8 || gemm_b8_tile(p, f8, post_ops) == 32))) return pick;
+    // (64 x 64 fp8 results of few k take longer than priced: 104 x 6352 x 128 8.4 / 9.0)
+    if (f8 && p.K <= 512 && pick == 0x44) best += 1.6;
+    // (clearly, or not; very tall problems are off what was measured: s8 16384 x 1024 x 128
+    // 13.7 / 16.9, 16384 x 4096 x 64 28.7 / 22.5; fp8 up to 64 rows in tiles is priced too high)
+    const double margin = p.M > 2500 ? 1.3 : p.M > 64 ? 1.05 : 1.25;
+    return best < b8_other_us(p, f8, post_ops) / margin ? pick : 0;
 }
 
 void launch_gemm_b8k(const gemm_params_t &p, bool f8, int shape, hipStream_t stream) {

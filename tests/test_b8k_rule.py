@@ -21,6 +21,13 @@ def shape(M, K, N, src=dt.s8, post_ops=0):
     (894, 2944, 12624, 0),  # 61 / 108
     (16384, 1024, 128, 0),  # 13.7 / 16.9
     (4096, 4096, 14336, 0),
+    # few k or many columns: the kernels of 256 rows
+    (2059, 256, 768, 0),  # 10.8 / 14.2
+    (74, 6016, 49408, 0),  # 84.0 / 121.0
+    (86, 2688, 39168, 0),  # 42.8 / 55.2
+    (403, 512, 3776, 0),  # 12.4 / 15.5
+    # one row of workgroups
+    (56, 384, 126800, 0x44),  # in 32 x 32 results 69.4, so 60.0
 ])
 def test_integers(M, K, N, want):
     assert shape(M, K, N) == want
@@ -32,6 +39,15 @@ def test_integers(M, K, N, want):
     (967, 8576, 4064, 0),  # 66 / 83
     (1, 4096, 14336, 0),  # 13.2 / 14.5
     (8192, 8192, 8192, 0),
+    # few k: 256 x 256 tiles
+    (65, 640, 62464, 0),  # 21.2 / 50.1
+    (129, 768, 35584, 0),  # 24.8 / 51.5
+    (1102, 640, 4608, 0),  # 20.6 / 45.3
+    (204, 640, 18944, 0),  # 21.0 / 39.7
+    (279, 1280, 16640, 0),  # 28.0 / 52.1
+    (40, 384, 56928, 0),  # 21.4 / 27.1
+    # rows that no L2 holds
+    (1921, 7168, 1040, 0),  # 53.7 / 72.5
 ])
 def test_fp8(M, K, N, want):
     assert shape(M, K, N, dt.f8_e4m3, 1) == want
@@ -39,6 +55,9 @@ def test_fp8(M, K, N, want):
 
 def test_u8_sources():
     assert shape(256, 1024, 1024, dt.u8) == 0x22  # 5.8 / 4.9
+    # the others' pre-pass pays over many tiles
+    assert shape(1934, 14336, 4112, dt.u8, 1) == 0  # 184 / 284
+    assert shape(404, 128, 3808, dt.u8) == 0x44  # 15.9 / 11.6
 
 
 def test_other_arguments_take_nothing():
