@@ -312,15 +312,19 @@ static double b8_other_us(const gemm_params_t &p, bool f8, bool post_ops) {
 // and many aligned columns from 33 rows on (fp8 65 x 640 x 62464 21 / 50, 1102 x 640 x 4608 20.6 / 45,
 // 40 x 384 x 56928 21 / 27; s8 74 x 6016 x 49408 84 / 121) and for u8 rows where these are rewritten once
 // for many tiles (1934 x 14336 x 4112 184 / 284); and
-// up to 4 rows of 4096 k the streaming kernel, which requests all of them at once (1 x 4096 x
-// 4832 7.3 / 8.1, 1 x 4096 x 14336 13.3 / 14.0; 1 x 12032 x 9248 27.6 / 24.5). Over 640 problems
+// where the streaming kernel requests all of its K at once: up to 4 rows of 4096 k (1 x 4096 x
+// 4832 7.3 / 8.1, 1 x 4096 x 14336 13.3 / 14.0; 3072 k and less, or very wide weights, are the same or
+// faster here: 2 x 2944 x 4192 7.6 / 7.6, 2 x 3200 x 65072 42 / 36, 1 x 12032 x 9248 27.6 / 24.5) and up to 32
+// of 2048 (25 x 1536 x 21808 12.6 / 13.6, 20 x 1664 x 85952 40 / 44). Over 640 problems
 // of 1 ... 2500 rows 1.25 times as fast in the mean; over 5300 further ones 1.17 times, and up to 17 %
 // slower than the kernels before (fp8 82 x 15232 x 35968 164 / 191; u8 165 x 128 x 10208 12.0 / 13.4). A round of workgroups costs a start, an end and the waves' K; a CU holds one,
 // or (up to 16 x 64 or 32 x 32 results) two. The caller checks that there is one matrix and no
 // weights zero point.
 int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops) {
     if (p.K % 128 != 0 || (int64_t)p.M * p.lda >= (int64_t)1 << 32) return 0;
-    if (p.M <= 4 && p.K > 3072 && p.K <= 4096 && p.N > 4096) return 0;
+    // K that the streaming kernel requests all at once: up to 4096 with 4 rows, 2048 with 32
+    if (p.M <= 4 && p.K > 3072 && p.K <= 4096 && p.N > 4096 && p.N <= 16384) return 0;
+    if (p.M > 16 && p.M <= 32 && p.K > 1408 && p.K <= 2048 && p.N > 16384) return 0;
     // {.., once, per round, per round and 1024 k, a begun round's share, the second on a CU}
     static const struct {
         int rb, cb;
@@ -338,6 +342,8 @@ int gemm_b8k_shape(const gemm_params_t &p, bool f8, bool post_ops) {
         if (s.rb * s.cb == 16 && (s.once > 0) != short_k) continue;
         // workgroups on a CU (32 on an XCD)
         const double wgs = b8k_map(p.M, (p.N + 15) / 16, s.rb, s.cb).share / 32.0;
+        // (17 ... 32 rows bound by HBM: 32 x 32 results twice on a CU, 23 x 3584 x 124496 99.5 / 86)
+        if (s.rb == 2 && s.cb == 4 && p.M <= 32 && wgs > 2) continue;
         double rounds = s.begun * std::ceil(wgs) + (1 - s.begun) * wgs;
         if (s.second > 0) { // pairs
             const double full = std::floor(wgs / 2), rest = wgs - 2 * full;

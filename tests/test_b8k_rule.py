@@ -26,7 +26,12 @@ def shape(M, K, N, src=dt.s8, post_ops=0):
     (74, 6016, 49408, 0),  # 84.0 / 121.0
     (86, 2688, 39168, 0),  # 42.8 / 55.2
     (403, 512, 3776, 0),  # 12.4 / 15.5
+    # what the streaming kernel requests at once, and where that is no gain
+    (25, 1536, 21808, 0),  # 12.6 / 13.6
+    (28, 1664, 117056, 0),  # 51 / 59
+    (2, 3200, 65072, 0x14),  # 42 / 36
     # one row of workgroups
+    (23, 3584, 124496, 0x22),  # in 32 x 64 results 99.5, so 86.1
     (56, 384, 126800, 0x44),  # in 32 x 32 results 69.4, so 60.0
 ])
 def test_integers(M, K, N, want):
