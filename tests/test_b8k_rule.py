@@ -26,6 +26,12 @@ def shape(M, K, N, src=dt.s8, post_ops=0):
     (74, 6016, 49408, 0),  # 84.0 / 121.0
     (86, 2688, 39168, 0),  # 42.8 / 55.2
     (403, 512, 3776, 0),  # 12.4 / 15.5
+    (202, 3584, 8448, 0),  # 32.5 / 34.2
+    (714, 1024, 2368, 0),  # 15.3 / 17.2
+    # three rows of tiles that find their weights in L2
+    (1851, 6656, 1216, 0),  # 48.2 / 56.3
+    (1582, 6400, 1792, 0),  # 45.9 / 51.5
+    (1169, 12544, 2560, 0x44),  # 84.9 / 75.6
     # what the streaming kernel requests at once, and where that is no gain
     (25, 1536, 21808, 0),  # 12.6 / 13.6
     (28, 1664, 117056, 0),  # 51 / 59
