@@ -48,7 +48,7 @@ constexpr int w4a8k_wave_lds(int rb, int cb) {
 constexpr int W4A8K_DW = 2;
 constexpr int w4a8k_da(int rb) { return rb <= 2 ? 2 : 1; }
 
-template <int RB, int CB, bool NT>
+template <int RB, int CB>
 __global__ void __launch_bounds__(WK_WAVES * 64, RB * CB <= 4 ? 4 : 2)
 gemm_w4a8k_kernel(const g128_params_t p) {
     constexpr int DW = W4A8K_DW, DA = w4a8k_da(RB);
@@ -105,9 +105,7 @@ gemm_w4a8k_kernel(const g128_params_t p) {
         const int t = group_of(i);
 #pragma unroll
         for (int cb = 0; cb < CB; cb++) {
-            const v4u *const q = (const v4u *)at(Bt[cb] + (int64_t)t * 2048, boff);
-            if constexpr (NT) wt[sl][cb] = __builtin_nontemporal_load(q);
-            else wt[sl][cb] = *q;
+            wt[sl][cb] = *(const v4u *)at(Bt[cb] + (int64_t)t * 2048, boff);
             swr[sl][cb] = *(const uint16_t *)at(
                     (const uint8_t *)p.scales + (int64_t)t * p.sw_sk * 2, scol[cb]);
         }
@@ -326,21 +324,15 @@ void launch_gemm_w4a8k(const g128_params_t &p, int shape, hipStream_t stream) {
         hipLaunchKernelGGL(kern, dim3((unsigned)(8 * map.share)), dim3(WK_WAVES * 64), lds,
                 stream, p);
     };
-    // Weights that are read once and of which few layers fit the 256 MB memory-side cache go
-    // past the caches: 1 x 4096 x 28672 16.7 / 14.8 us, 4 x 6400 x 16384 14.2 / 12.7, 16 x 2048 x
-    // 128256 39.5 / 34.4; smaller ones may stay there.
-    const bool nt = map.nrb == 1 && (int64_t)p.ng * 64 * p.N >= (int64_t)40 << 20;
-    auto by_shape = [&](auto n) {
-        constexpr bool NT = decltype(n)::value;
-        switch (shape) {
-            case 0x12: go(gemm_w4a8k_kernel<1, 2, NT>); break;
-            case 0x14: go(gemm_w4a8k_kernel<1, 4, NT>); break;
-            case 0x24: go(gemm_w4a8k_kernel<2, 4, NT>); break;
-            default: go(gemm_w4a8k_kernel<3, 4, NT>); break;
-        }
-    };
-    if (nt) by_shape(std::true_type {});
-    else by_shape(std::false_type {});
+    // (loads past the caches gain nothing from HBM and lose where weights are in the memory-side
+    // cache, us, so / past them: 1 x 4096 x 28672 15.6 / 15.9 and 12.6 / 13.9, 16 x 2048 x 128256
+    // 39.0 / 43.8 and 27.2 / 39.4)
+    switch (shape) {
+        case 0x12: go(gemm_w4a8k_kernel<1, 2>); break;
+        case 0x14: go(gemm_w4a8k_kernel<1, 4>); break;
+        case 0x24: go(gemm_w4a8k_kernel<2, 4>); break;
+        default: go(gemm_w4a8k_kernel<3, 4>); break;
+    }
 }
 
 } // namespace qmm
