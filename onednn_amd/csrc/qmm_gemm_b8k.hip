@@ -10,7 +10,7 @@
 //   * Rows are requested eight lanes to 128 bytes and change to operand order in a piece of
 //     LDS of the wave's own: no barrier. Weights are requested two tiles ahead.
 // Bound: HBM and a start and an end of 4 us where the weights are read once (64 x 4096 x 14336
-// 18.0 us, 4.0 TB/s with 224 of 256 CUs), else the requests through L1: 64 x 64 results need 16
+// 20.0 us, 2.9 TB/s, with 224 of 256 CUs; 16.4 with the weights in the memory-side cache), else the requests through L1: 64 x 64 results need 16
 // KB per 128 k of a wave, 32 x 64 12, which is why the largest tile wins as soon as it fills
 // the chip (413 x 12672 x 3584, fp8, in 16 x 64 / 32 x 64 / 64 x 64: 76 / 55 / 49 us).
 #include <algorithm>
@@ -307,15 +307,16 @@ static double b8_other_us(const gemm_params_t &p, bool f8, bool post_ops) {
 }
 
 // Row and column blocks of a workgroup as 16 * rb + cb, 0: another kernel is faster. Before /
-// now (us): s8 64 x 4096 x 14336 23.3 / 18.0, 16 x 12288 x 2048 15.2 / 10.7, 195 x 6912 x
-// 3296 29.5 / 16.0, 256 x 4096 x 4096 21.9 / 12.9, u8 256 x 1024 x 1024 5.8 / 4.9; fp8 413 x
-// 12672 x 3584 84 / 49, 350 x 8704 x 1472 32 / 15. The tiles that walk all of K stay ahead
+// now (us, weights in the memory-side cache): s8 64 x 4096 x 14336 21.3 / 16.4, 16 x 12288 x 2048 14.8 /
+// 10.3, 195 x 6912 x 3296 27.6 / 16.0, 256 x 4096 x 4096 19.0 / 12.5, u8 256 x 1024 x 1024 5.5 / 4.7; fp8
+// 413 x 12672 x 3584 73 / 46, 350 x 8704 x 1472 30 / 14.7; weights from HBM 24.1 / 20.0, 15.7 / 15.3, 28.7 /
+// 18.4, 19.7 / 14.9, 6.4 / 5.9; 84 / 54, 30 / 17.5. The tiles that walk all of K stay ahead
 // from some hundred rows on (fp8 967 x 8576 x 4064 66 / 83, s8 894 x 2944 x 12624 61 / 108), over few k
 // and many aligned columns from 33 rows on (fp8 65 x 640 x 62464 21 / 50, 1102 x 640 x 4608 20.6 / 45,
 // 40 x 384 x 56928 21 / 27; s8 74 x 6016 x 49408 84 / 121) and for u8 rows where these are rewritten once
 // for many tiles (1934 x 14336 x 4112 184 / 284); and
-// where the streaming kernel requests all of its K at once: up to 4 rows of 4096 k (1 x 4096 x
-// 4832 7.3 / 8.1, 1 x 4096 x 14336 13.3 / 14.0; 3072 k and less, or very wide weights, are the same or
+// where the streaming kernel requests all of its K at once: up to 4 rows of 4096 k (from HBM, 1 x
+// 4096 x 4832 8.2 / 8.5, 1 x 4096 x 14336 14.2 / 15.1; 3072 k and less, or very wide weights, are the same or
 // faster here: 2 x 2944 x 4192 7.6 / 7.6, 2 x 3200 x 65072 42 / 36, 1 x 12032 x 9248 27.6 / 24.5) and up to 32
 // of 2048 (25 x 1536 x 21808 12.6 / 13.6, 20 x 1664 x 85952 40 / 44). Over 640 problems
 // of 1 ... 2500 rows 1.25 times as fast in the mean; over 5300 further ones 1.17 times, and up to 17 %
@@ -389,10 +390,12 @@ void launch_gemm_b8k(const gemm_params_t &p, bool f8, int shape, hipStream_t str
             default: go(gemm_b8k_kernel<F, 4, 4, NT>); break;
         }
     };
-    // Weights that are read once and of which few layers fit the 256 MB memory-side cache go
-    // past the caches: 64 x 4096 x 14336 19.8 / 18.0 us; of those that stay there 8 x 4096 x
-    // 4096 lose (7.0 / 8.0), 4 x 2048 x 13000 8.8 / 9.5.
-    const bool nt = map.nrb == 1 && (int64_t)p.K * p.N >= (int64_t)40 << 20;
+    // Weights that are read once go past the caches from 128 MB on, where not even two of them fit
+    // the 256 MB memory-side cache. us, through / past the caches, weights from HBM: 64 x 8192 x 28672
+    // 59.5 / 57.2, 64 x 4096 x 14336 20.0 / 19.5, 4 x 2048 x 13000 9.8 / 9.8; weights in that cache: 44.6 /
+    // 54.4, 16.4 / 17.6, 8.1 / 9.1. Over 640 problems from HBM 0 % are won below 30 MB, 2 to 3 % from 40 to
+    // 100, 4 from 100 to 200 and 7 from there; what is in the cache loses 8 ... 14 %.
+    const bool nt = map.nrb == 1 && (int64_t)p.K * p.N >= (int64_t)128 << 20;
     auto by_nt = [&](auto f) {
         if (nt) by_shape(f, std::true_type {});
         else by_shape(f, std::false_type {});

@@ -40,7 +40,7 @@ CASES = {
     "rows32_64_17_tiles": (0x24, dict(M=65, K=2176, N=4203)),
     "rows64_32": (0x42, dict(M=127, K=1152, N=3590)),
     "rows64_64": (0x44, dict(M=190, K=1280, N=2795)),
-    "past_the_caches": (0x44, dict(M=63, K=4096, N=10250)),
+    "40_mb_of_weights": (0x44, dict(M=63, K=4096, N=10250)),
 }
 
 
@@ -71,3 +71,36 @@ def test_fp8_into_a_residual(ctx, M, K, N, shape):
     print("[case] b8k fp8 %d %d %d" % (M, K, N), flush=True)
     assert _capi.lib().qmm_gemm_b8k_shape(dt.f8_e4m3, M, N, K, 1) == shape
     fp8_sum(ctx, M, K, N, M + N, dt.f32)
+
+
+@pytest.mark.parametrize("M,K,N,shape", [(2, 8192, 16418, 0x12), (33, 3072, 43700, 0x44)])
+@pytest.mark.parametrize("kind", ["s8", "u8", "fp8"])
+def test_weights_past_the_caches(ctx, kind, M, K, N, shape):
+    """128 MB of weights and more, read once: the loads are others. Exact in f32, whatever the order of the sums."""
+    import torch
+    from onednn_amd import memory
+    print("[case] b8k past the caches %s %d %d %d" % (kind, M, K, N), flush=True)
+    assert K * N >= 128 << 20
+    code = {"s8": dt.s8, "u8": dt.u8, "fp8": dt.f8_e4m3}[kind]
+    assert _capi.lib().qmm_gemm_b8k_shape(code, M, N, K, kind == "fp8") == shape
+    if kind == "fp8":
+        fp8_sum(ctx, M, K, N, M, dt.f32)
+        return
+    eng, strm = ctx
+    g = torch.Generator().manual_seed(M)
+    lo, hi, kind_t = (0, 256, torch.uint8) if kind == "u8" else (-127, 128, torch.int8)
+    a = torch.randint(lo, hi, (M, K), generator=g, dtype=kind_t)
+    b = torch.randint(-127, 128, (K, N), generator=g, dtype=torch.int8)
+    T = lambda name: 2 + memory.format_tag._plain.index(name)  # noqa: E731
+    pd = dnnl.matmul.primitive_desc(eng, memory.desc([M, K], code, T("ab")), memory.desc([K, N], dt.s8, memory.format_tag.any),
+                                    memory.desc([M, N], dt.s32, T("ab")))
+    packed = memory(pd.weights_desc(), eng)
+    plain = memory(memory.desc([K, N], dt.s8, T("ab")), eng).write(b.numpy())
+    dnnl.reorder(plain, packed).execute(strm, plain, packed)
+    out = memory(pd.dst_desc(), eng)
+    dnnl.matmul(pd).execute(strm, {dnnl.DNNL_ARG_SRC: memory(pd.src_desc(), eng).write(a.numpy()),
+                                   dnnl.DNNL_ARG_WEIGHTS: packed, dnnl.DNNL_ARG_DST: out})
+    strm.wait()
+    want = a.double() @ b.double()
+    got = out.read(np.int32, (M, N))
+    assert (torch.from_numpy(got.copy()).double() == want).all()
