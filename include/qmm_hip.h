@@ -282,6 +282,15 @@ QMM_API int qmm_gemm_b8k_shape(int src_dt, int64_t M, int64_t N, int64_t K, int 
 /* The same for f16 x 8-bit weights at many rows (mfma_f16w8), without post-ops. */
 QMM_API int qmm_gemm_f16w8k_shape(int64_t M, int64_t N, int64_t K);
 
+/* The slices into which the 256 x 256 tiles beside it cut K (1: one pass). */
+QMM_API int qmm_gemm_f16w8_slices(int64_t M, int64_t N, int64_t K);
+
+/* Whether batches of s8 x s8 without zero points with an f32 destination take the kernel for
+ * many matrices of a short K; dst_pitch: elements from one row to the next, add: an f32
+ * operand is added per result and nothing else. */
+QMM_API int qmm_gemm_b8s_takes(int64_t batch, int64_t M, int64_t N, int64_t K,
+        int64_t dst_pitch, int add);
+
 /* Whether more than 16 rows of f16 / bf16 activations under 4- or 8-bit weights run on the
  * tiled kernel (1) or on the decode kernel once per 16 rows (0), where one of these takes
  * them (hip:gfx950:decode_w4). */

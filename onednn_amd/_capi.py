@@ -148,6 +148,8 @@ _SIGNATURES = {
     "qmm_gemm_w4a8k_shape": (_I, [C.c_int64] * 3),
     "qmm_gemm_b8k_shape": (_I, [_I] + [C.c_int64] * 3 + [_I]),
     "qmm_gemm_f16w8k_shape": (_I, [C.c_int64] * 3),
+    "qmm_gemm_f16w8_slices": (_I, [C.c_int64] * 3),
+    "qmm_gemm_b8s_takes": (_I, [C.c_int64] * 5 + [_I]),
     "qmm_gemm_w4f_tiled": (_I, [_I, _I] + [C.c_int64] * 3),
     "qmm_gemv_b8_block": (C.c_int64, [C.c_int64] * 3),
     "qmm_sdpa_pipelined": (_I, [_I, _I] + [C.c_int64] * 4 + [_I]),

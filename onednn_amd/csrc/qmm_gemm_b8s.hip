@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "qmm_device.hpp"
+#include "qmm_hip.h"
 #include "qmm_plan.hpp"
 
 namespace qmm {
@@ -161,3 +162,24 @@ void launch_gemm_b8s(const gemm_params_t &p, hipStream_t stream) {
 }
 
 } // namespace qmm
+
+extern "C" int qmm_gemm_b8s_takes(
+        int64_t batch, int64_t M, int64_t N, int64_t K, int64_t dst_pitch, int add) {
+    using namespace qmm;
+    const int64_t top = 1 << 24;
+    if (batch < 1 || M < 1 || N < 1 || K < 16 || K % 16 || dst_pitch < N || batch > top || M > top || N > top || K > top)
+        return 0;
+    gemm_params_t p = {};
+    p.M = (int32_t)M;
+    p.N = (int32_t)N;
+    p.K = (int32_t)K;
+    p.lda = K;
+    p.batch = (int32_t)batch;
+    p.kb32 = (int32_t)((K + 31) / 32);
+    p.ep.dst.dt = dt_f32;
+    p.ep.dst.sm = dst_pitch;
+    p.ep.dst.sn = 1;
+    p.ep.npo = add ? 1 : 0;
+    p.ep.fast = add ? EP_FAST_ADD : EP_FAST_PLAIN;
+    return gemm_b8s_takes(p);
+}

@@ -429,3 +429,11 @@ void launch_gemm_f16w8(const gemm_params_t &p, int splits, float *part,
 #endif
 
 } // namespace qmm
+
+#if QMM_F16W8_PART == 0
+extern "C" int qmm_gemm_f16w8_slices(int64_t M, int64_t N, int64_t K) {
+    const int64_t top = 1 << 24;
+    if (M < 1 || N < 1 || K < 32 || K % 32 != 0 || M > top || N > top || K > top) return 0;
+    return qmm::gemm_f16w8_splits(M, N, K);
+}
+#endif

@@ -1,12 +1,15 @@
 """The streaming kernel of few rows or few results (32 x 32 results a workgroup, K cut over its waves) and the rows that
 the tiled kernels store one vector at a time: where blocks of 32 rows, 32 columns and K's fragments end, s8 / u8 / f8
 operands, every kind of column and row operand. Integer problems bit for bit against the oracle and against the tiled
-kernels (QMM_GEMM_VARIANT), fp8 within the rounding of its sums."""
+kernels (QMM_GEMM_VARIANT), fp8 within the rounding of its sums. Where K is a multiple of 128 and there are no weights
+zero points, the default choice of most small problems is the kernel of qmm_gemm_b8k.hip (the same implementation name): the
+streaming kernel without row sums runs in test_the_streaming_kernel_itself and test_fp8_streams."""
 import numpy as np
 import pytest
 
 import onednn_amd as dnnl
 import test_gpu_parity as cases
+from onednn_amd import _capi
 from qmm_harness import assert_bit_exact, dt
 from test_gpu_int8_wei_zp import w8a8
 
@@ -39,6 +42,29 @@ def test_blocks_of_rows_and_columns(ctx, monkeypatch, shape, src):
     assert_bit_exact(p.run_gpu(eng, strm, weights_any=True), want, "stream")
     monkeypatch.setenv("QMM_GEMM_VARIANT", "3")  # 64 x 64 tiles
     assert_bit_exact(p.run_gpu(eng, strm, weights_any=True), want, "tiles")
+
+
+def streams(monkeypatch, src, M, K, N, post_ops=0):
+    """Plans made from here on take the streaming kernel: by default, or up to 64 rows of integers in a variant of the tiles,
+    which the kernel that cuts K over its waves is not for."""
+    lib = _capi.lib()
+    assert lib.qmm_gemm_b8_tile(dt.f8_e4m3 if src == dt.f8_e4m3 else dt.s8, 1, M, N, K, post_ops) == 32
+    if lib.qmm_gemm_b8k_shape(src, M, N, K, post_ops):
+        assert M <= 64 and src != dt.f8_e4m3
+        monkeypatch.setenv("QMM_B8X_VARIANT", "2")
+
+
+@pytest.mark.parametrize("src", [dt.s8, dt.u8], ids=["s8", "u8"])
+@pytest.mark.parametrize("M,K,N", [(33, 32, 33), (63, 2080, 4130), (40, 4096, 4128), (5, 256, 70), (1, 4224, 34), (4, 128, 40),
+                                   (17, 1024, 130), (64, 1152, 200), (96, 544, 257), (130, 288, 1001), (256, 1056, 96)], ids=str)
+def test_the_streaming_kernel_itself(ctx, monkeypatch, M, K, N, src):
+    """... without weights zero points, which by themselves keep a problem off the other kernel."""
+    print("[case] stream itself %s %d %d %d" % (src, M, K, N), flush=True)
+    kw = dict(src_zp=119) if src == dt.u8 else dict(src_zp=None, per_token=True, dst_dt=dt.bf16)
+    p = cases.int8_linear(M, K, N, M + K + N, src_dt=src, **kw)
+    streams(monkeypatch, src, M, K, N, bool(p.post_ops))
+    eng, strm = ctx
+    assert_bit_exact(p.run_gpu(eng, strm, weights_any=True), p.run_oracle(), "stream")
 
 
 @pytest.mark.parametrize("M,K,N", [(70, 256, 98), (40, 512, 4200), (33, 96, 64), (40, 208, 72), (64, 208, 4130),
@@ -95,6 +121,13 @@ def test_fp8_into_a_residual(ctx, M, K, N, dst):
     """The streaming kernel: pairs of fragments, one pair in all and an odd number of them per wave."""
     print("[case] fp8 stream %d %d %d" % (M, K, N), flush=True)
     fp8_sum(ctx, M, K, N, M + N, dst)
+
+
+@pytest.mark.parametrize("M,K,N", [(3, 64, 40), (33, 192, 33), (257, 1856, 130), (100, 448, 999), (16, 2112, 2050)])
+def test_fp8_streams(ctx, monkeypatch, M, K, N):
+    print("[case] fp8 streams %d %d %d" % (M, K, N), flush=True)
+    streams(monkeypatch, dt.f8_e4m3, M, K, N, 1)
+    fp8_sum(ctx, M, K, N, M + N, dt.f32)
 
 
 @pytest.mark.parametrize("B,M,K,N", [(8, 64, 512, 1024), (2, 130, 384, 257), (3, 33, 512, 64), (20, 64, 512, 640)])

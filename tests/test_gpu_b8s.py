@@ -1,7 +1,7 @@
 """GPU parity of the kernel for many matrices of a short K (qmm_gemm_b8s.hip, hip:gfx950:mfma_b8): rows and columns that end
 inside a wave's 32 x 64, more than 256 rows (the order of the row tiles), scales per column, a bias, a mask for all
-matrices or one each. Integer sums, so every result is bit for bit; widths off a multiple of 4 take this kernel
-from 64 tiles of 128 x 128 on."""
+matrices or one each, source scales per row. Integer sums, so every result is bit for bit; widths off a multiple of 4 take
+this kernel from 64 tiles of 128 x 128 on, which each case asserts: the kernels with tiles carry the same name."""
 import numpy as np
 import pytest
 
@@ -19,10 +19,10 @@ def ctx():
     return eng, dnnl.stream(eng)
 
 
-def scores(B, M, N, K, seed, mask=None, columns=False, bias=False):
+def scores(B, M, N, K, seed, mask=None, columns=False, bias=False, rows=False):
     r = np.random.default_rng(seed)
     q, k = r.integers(-127, 128, (B, M, K)), r.integers(-127, 128, (B, K, N))
-    scales = {"src": (0, dt.f32, None, [0.01]),
+    scales = {"src": (6, dt.f32, (1, K), r.uniform(0.005, 0.02, M)) if rows else (0, dt.f32, None, [0.01]),
               "wei": (4, dt.f32, None, r.uniform(0.001, 0.01, N)) if columns else (0, dt.f32, None, [0.012])}
     po = []
     if mask:
@@ -42,11 +42,14 @@ def scores(B, M, N, K, seed, mask=None, columns=False, bias=False):
     (4, 600, 385, 64, dict(mask="all", columns=True)),
     (16, 193, 191, 128, dict(columns=True)),
     (8, 130, 447, 64, dict(bias=True, columns=True)),
+    (16, 150, 129, 64, dict(rows=True, mask="all")),
+    (11, 290, 255, 128, dict(rows=True, columns=True)),
 ], ids=str)
 def test_scores(ctx, B, M, N, K, kw):
     print("[case] b8s %d %d %d %d %r" % (B, M, N, K, kw), flush=True)
     eng, strm = ctx
-    assert N % 4 and _capi.lib().qmm_gemm_b8_tile(dt.s8, B, M, N, K, "mask" in kw) > 64
+    # (a bias is not in the query; it does not enter the rule)
+    assert _capi.lib().qmm_gemm_b8s_takes(B, M, N, K, N, "mask" in kw)
     p = scores(B, M, N, K, B + M + N, **kw)
     got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
     assert pd.impl_info_str() == "hip:gfx950:mfma_b8"

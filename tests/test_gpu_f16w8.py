@@ -5,6 +5,10 @@ The shapes are those of the 8-bit weights-only prefill entries of the reference'
 (tests/benchdnn/inputs/matmul/option_set_fwks_llm_gpu: --dt=f16:u8:f16|f32 --wtag=ba --attr-scales=wei:per_oc:f16
 --attr-zero-points=wei:per_oc:u8 --attr-fpmath=f16:true, with swish / binary_add post-ops) at a reduced K and N.
 
+Two kernels carry the name: 256 x 256 tiles (qmm_gemm_f16w8.hip), their K whole or cut into slices, and one that cuts K
+over a workgroup's waves (qmm_gemm_f16w8k.hip), which by default takes most problems as small as these. `tiles` below makes a
+plan's problems take the former; test_gpu_f16w8k.py has the latter's own sizes.
+
 Bars: the kernel converts the weights exactly and sums f16 x f16 products in f32 (MFMA order) where the reference sums
 a x ((w - z) x scale) in f32 in k order: an f32 dst within 2e-5 of the summed magnitudes, an f16 dst within one f16
 step (2^-10 relative) plus that."""
@@ -15,6 +19,7 @@ import pytest
 
 import onednn_amd as dnnl
 import oracle as O
+from onednn_amd import _capi
 from qmm_harness import Problem, TensorSpec, dt
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +37,12 @@ def say(msg):
 def ctx():
     eng = dnnl.engine(dnnl.engine.kind.gpu, 0)
     return eng, dnnl.stream(eng)
+
+
+def tiles(monkeypatch):
+    """Plans made from here on take the 256 x 256 tiles: the kernel that cuts K over its waves is for the default variant only,
+    and 2 means nothing else to this implementation."""
+    monkeypatch.setenv("QMM_B8X_VARIANT", "2")
 
 
 def problem(M, K, N, seed, wei_dt=dt.u8, zp="per_column", zp_dt=dt.u8, scale="per_column", scale_dt=dt.f16,
@@ -138,10 +149,47 @@ def test_f16_activations_8bit_weights(ctx, name, weights_any):
     check(p, got, p.run_oracle(), name)
 
 
-def test_extreme_weights_and_zero_points_convert_exactly(ctx):
+# K slices that each case's sizes take in 256 x 256 tiles
+SLICES = {"u8_k4096_f32": 8, "u8_k1536_three_slices_swish": 3, "s8_k1088_two_odd_slices": 2, "u8_k2048_four_slices_add": 4,
+          "u8_k1024_slices_gelu_odd_columns": 2}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_256_x_256_tiles(ctx, monkeypatch, name):
+    eng, strm = ctx
+    say("mfma_f16w8 tiles %s" % name)
+    kw = CASES[name]
+    assert _capi.lib().qmm_gemm_f16w8_slices(kw["M"], kw["N"], kw["K"]) == SLICES.get(name, 1)
+    tiles(monkeypatch)
+    p = problem(seed=len(name) * 7 + 1, **kw)
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == F16W8
+    check(p, got, p.run_oracle(), name)
+
+
+@pytest.mark.parametrize("M,K,N,slices,kw", [
+    # what the default choice leaves to the tiles: K that is no multiple of 128, among it three, two and six slices
+    (300, 1632, 520, 3, dict(post="swish")), (257, 2112, 384, 3, dict(dst_dt=dt.f32, post="add")),
+    (256, 1088, 256, 2, dict(wei_dt=dt.s8, zp_dt=dt.s8)), (259, 3264, 260, 6, dict()), (513, 160, 515, 1, dict(post="gelu")),
+], ids=str)
+def test_tiles_by_default(ctx, M, K, N, slices, kw):
+    eng, strm = ctx
+    say("mfma_f16w8 default tiles %d %d %d" % (M, K, N))
+    assert _capi.lib().qmm_gemm_f16w8k_shape(M, N, K) == 0 and _capi.lib().qmm_gemm_f16w8_slices(M, N, K) == slices
+    p = problem(M, K, N, M + K, **kw)
+    got, pd = p.run_gpu(eng, strm, weights_any=True, return_pd=True)
+    assert pd.impl_info_str() == F16W8
+    check(p, got, p.run_oracle(), "default tiles")
+
+
+@pytest.mark.parametrize("kernel", ["waves", "tiles"])
+def test_extreme_weights_and_zero_points_convert_exactly(ctx, monkeypatch, kernel):
     """Weights and zero points at the ends of their ranges (differences of +-255) against a one-hot source: every
     output is a single product a x (w - z) x scale, so any error in the byte -> f16 conversion shows undiluted."""
     eng, strm = ctx
+    assert _capi.lib().qmm_gemm_f16w8k_shape(256, 256, 256)
+    if kernel == "tiles":
+        tiles(monkeypatch)
     for wei_dt, zp_dt in ((dt.u8, dt.u8), (dt.s8, dt.s8), (dt.u8, dt.s8), (dt.s8, dt.u8)):
         say("mfma_f16w8 one-hot %s / %s" % (wei_dt, zp_dt))
         M, K, N = 256, 256, 256
@@ -164,6 +212,8 @@ def test_extreme_weights_and_zero_points_convert_exactly(ctx):
 def test_slices_of_k_and_one_pass_agree(ctx, monkeypatch):
     """QMM_GEMM_VARIANT=1 keeps K in one pass: same problem both ways, each against the oracle's bar."""
     eng, strm = ctx
+    assert _capi.lib().qmm_gemm_f16w8_slices(256, 512, 2048) == 4
+    tiles(monkeypatch)
     p = problem(256, 2048, 512, 11, dst_dt=dt.f32)
     got_slices = p.run_gpu(eng, strm, weights_any=True)
     monkeypatch.setenv("QMM_GEMM_VARIANT", "1")

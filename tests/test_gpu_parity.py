@@ -11,7 +11,7 @@ import pytest
 
 import onednn_amd as dnnl
 import oracle as O
-from onednn_amd import memory
+from onednn_amd import _capi, memory
 from qmm_harness import (Problem, T, TensorSpec, assert_bf16_within_1ulp, assert_bit_exact,
                          assert_f32_close, dt, tag)
 
@@ -814,6 +814,10 @@ def test_decode_8bit_weights(ctx, name, weights_any):
         assert_bf16_within_1ulp(got, want, "decode 8-bit bf16", abs_slack=2e-5 * decode_term_scale(p))
 
 
+# Those of the tables below that the kernel with K cut over its waves takes (qmm_gemm_w4k.hip; it has tests of its own):
+# they pin its results at these sizes, no longer the tiles'.
+CUT_OVER_WAVES = {"f16_u4_24_rows_wide", "bf16_u4_50_rows_wide", "f16_u8_130_rows_per_column"}
+
 TILED_CASES = {
     "bf16_u4_g128_zp_u4": dict(M=1100, K=256, N=2048),
     "f16_u8_per_column_row_and_column_tails": dict(M=1030, K=384, N=2040, act_dt=dt.f16, wei_dt=dt.u8, zp_dt=dt.u8,
@@ -828,6 +832,16 @@ TILED_CASES = {
                                        per_column=True),
     "f16_s4_32_rows_k_tail": dict(M=32, K=200, N=12800, act_dt=dt.f16, wei_dt=dt.s4, with_zp=False, G=200,
                                   per_column=True),
+    # ... at sizes that stay with them: groups of 128 k over many columns, K that is no multiple of 128
+    "bf16_u4_17_rows": dict(M=17, K=384, N=16664),
+    "f16_u4_20_rows_zp_u8": dict(M=20, K=256, N=16400, act_dt=dt.f16, zp_dt=dt.u8),
+    "bf16_s4_33_rows": dict(M=33, K=256, N=16776, wei_dt=dt.s4, zp_dt=dt.s4),
+    "f16_u4_61_rows_k_tail": dict(M=61, K=328, N=4200, act_dt=dt.f16, per_column=True),
+    "bf16_u4_50_rows_k_tail": dict(M=50, K=328, N=8200, per_column=True),
+    "f16_u8_130_rows_k_tail": dict(M=130, K=264, N=4616, act_dt=dt.f16, wei_dt=dt.u8, zp_dt=dt.u8, per_column=True),
+    "bf16_u8_40_rows_k_tail": dict(M=40, K=392, N=8200, wei_dt=dt.u8, zp_dt=dt.u8, per_column=True),
+    "bf16_s8_33_rows": dict(M=33, K=384, N=8488, wei_dt=dt.s8, zp_dt=dt.s8, per_column=True),
+    "f16_u8_17_rows_groups": dict(M=17, K=384, N=16664, act_dt=dt.f16, wei_dt=dt.u8, zp_dt=dt.u8),
 }
 
 
@@ -839,6 +853,10 @@ def test_decompression_at_many_rows(ctx, name):
     eng, strm = ctx
     say("decode_w4 tiled %s" % name)
     kw = TILED_CASES[name]
+    query = (kw.get("act_dt", dt.bf16), 8 if kw.get("wei_dt") in (dt.u8, dt.s8) else 4)
+    size = (kw["M"], kw["N"], kw["K"])
+    assert bool(_capi.lib().qmm_gemm_w4k_shape(*query, int(kw.get("per_column", False)), *size)) == (name in CUT_OVER_WAVES)
+    assert name in CUT_OVER_WAVES or _capi.lib().qmm_gemm_w4f_tiled(*query, *size)
     p = decode_w4(seed=70 + len(name), **kw)
     # (asked for by name: f16 x 8-bit weights at 256 rows and more go to mfma_f16w8 first)
     got, pd = p.run_gpu(eng, strm, weights_any=True, impl=DECODE, return_pd=True)
