@@ -259,15 +259,15 @@ static double w4a8_tiled_us(int M, int N, int K) {
     return 3.9 - 0.34 * K / 1024 + one * (tiles <= 256 ? 1.0 : 1.24 * (double)((tiles + 511) / 512));
 }
 
-// Row and column blocks of a workgroup as 16 * rb + cb, 0: another kernel is faster. Before /
-// now (us): 64 x 4096 x 14336 24 / 17, 8 x 4096 x 4096 16.5 / 5.9, 1 x 13312 x 1312 10.3 /
-// 9.0, 128 x 12288 x 2048 85 / 12.9, 435 x 5376 x 3888 43 / 31, 1941 x 1024 x 1072 18.8 /
-// 18.0; the tall tiles of qmm_gemm_g128.hip stay ahead from some 200 rows and 15 million
+// Row and column blocks of a workgroup as 16 * rb + cb, 0: another kernel is faster. The other
+// kernels / this one (us), weights from HBM: 1 x 4096 x 14336 10.5 / 10.3, 64 x 4096 x 14336
+// 23.6 / 19.7, 8 x 4096 x 4096 17.2 / 6.7, 1 x 13312 x 1312 11.5 / 10.3; in the caches: 9.3 /
+// 8.5, 22.8 / 16.3, 16.1 / 5.7, 10.4 / 8.7, 128 x 12288 x 2048 85 / 12.9, 435 x 5376 x 3888
+// 43 / 31, 1941 x 1024 x 1072 18.8 / 18.0; the tall tiles of qmm_gemm_g128.hip stay ahead from some 200 rows and 15 million
 // weights on (256 x 4096 x 14336 37 / 50, 1000 x 4096 x 4096 37 / 58, 1267 x 14336 x 2768 109 / 129). Up to 64 rows no
-// problem but the one below was faster without. Over 365 problems of 1 ... 4096 rows the choice is 0.2 %
-// behind the faster kernel in the mean and 15 % at most, 2.2 times as fast as before in the
-// mean; over 1700 further ones up to 5 % slower than the kernels before (17 ... 32 rows of few k
-// over some 20000 columns up to 12 %: 17 x 640 x 22400 7.8 / 8.7). A round of workgroups costs a start, an end and the waves' K; a CU holds one, or (16
+// problem but the one below was faster without. Over 1785 problems of 1 ... 4096 rows, HBM and
+// caches, the choice is 1.74 times as fast as the other kernels in the mean and up to 5 % slower
+// (17 ... 32 rows of few k over some 20000 columns up to 12 %: 17 x 640 x 22400 7.8 / 8.7). A round of workgroups costs a start, an end and the waves' K; a CU holds one, or (16
 // rows) two, which take about twice as long as one.
 int gemm_w4a8k_shape(const g128_params_t &p) {
     // 32-bit offsets of rows, row scales and column scales

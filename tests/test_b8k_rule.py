@@ -1,5 +1,6 @@
 """Which 8-bit products take the kernel whose waves cut K (qmm_gemm_b8k_shape): host work only. Times in us, the kernels
-before / this one, measured on an MI355X with weights that come from HBM."""
+before / this one, measured on an MI355X: weights from HBM, in the entries below the first comment the geometric mean of
+weights from HBM and in the caches."""
 import pytest
 
 from onednn_amd import _capi, memory
